@@ -2,10 +2,11 @@
 
     python -m bgy3d_amd.build
 
-hipcc compiles the HIP translation unit for gfx950 only (cross-compiles
+hipcc compiles the HIP translation units for gfx950 only (cross-compiles
 without a GPU); the host C++ of the 1D chi producer is built by hipcc as
 plain C++.  Packed-FP32 instruction selection is disabled for device code.
 """
+import concurrent.futures
 import os
 import subprocess
 import sys
@@ -22,19 +23,31 @@ HIP_FLAGS = [
 ]
 
 
+# (object, source, flags): the residual chain's kernels are templates with
+# many instantiations, split by pass and working type to build in parallel.
+UNITS = [("solver", "solver.hip", HIP_FLAGS), ("rism1d", "rism1d.cpp", None)] + [
+    (f"{src}_{t[0]}", f"{src}.hip", HIP_FLAGS + [f"-DRISM_T={t}"])
+    for src, types in (("chain_rows", ("double", "float")), ("chain_zpass", ("double", "float")),
+                       ("chain_planes", ("float",)))
+    for t in types]
+
+
 def build(verbose=False):
-    objs = []
-    srcs = [("solver.hip", True), ("rism1d.cpp", False)]
-    for src, is_hip in srcs:
-        out = os.path.join(CSRC, os.path.splitext(src)[0] + ".o")
-        cmd = [HIPCC] + (HIP_FLAGS if is_hip else ["-O3", "-std=c++17", "-fPIC", "-Wall"])
+    def compile_unit(unit):
+        name, src, flags = unit
+        out = os.path.join(CSRC, name + ".o")
+        if flags is None:
+            cmd = [HIPCC, "-x", "c++", "-O3", "-std=c++17", "-fPIC", "-Wall"]
+        else:
+            cmd = [HIPCC] + flags
         cmd += ["-c", os.path.join(CSRC, src), "-o", out]
-        if not is_hip:
-            cmd = [HIPCC, "-x", "c++"] + cmd[1:]
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.run(cmd, check=True)
-        objs.append(out)
+        return out
+
+    with concurrent.futures.ThreadPoolExecutor(max_workers=8) as pool:
+        objs = list(pool.map(compile_unit, UNITS))
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB + ".tmp"] + objs
     if verbose:
         print(" ".join(cmd), flush=True)

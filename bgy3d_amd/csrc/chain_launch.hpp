@@ -1,0 +1,72 @@
+// Launchers of the residual chain's kernels (chain.hpp).  Each is compiled
+// for one working type in a translation unit of its own (chain_rows.hip,
+// chain_zpass.hip, chain_planes.hip, once with RISM_T double and once with
+// float), so that the instantiations build in parallel.
+#pragma once
+#include <cstdlib>
+
+#include "chain.hpp"
+
+namespace rism {
+
+struct HipFailure {
+  hipError_t err;
+};
+
+// Tuning knobs, read once: RISM3D_ZSTAR_LINES (kx columns per zstar
+// workgroup, 2..16) and RISM3D_ZSTAR_ORDER (0..3, see zstar_reg).
+inline int env_int(const char* name, int dflt) {
+  const char* v = std::getenv(name);
+  return v ? std::atoi(v) : dflt;
+}
+
+template <typename T> constexpr int y_lines() { return 128 / (int)sizeof(cpx<T>); }
+
+template <typename T>
+int zstar_lines(int N2, int m) {
+  // 8 kx columns per workgroup (64 B FP32, 128 B FP64 rows): at 128^3 the
+  // FP32 pass ran 1.7 ms with 8 against 2.25 ms with 16 and 2.3 ms with 4
+  // (64 solutes, m = 3; occupancy against row length)
+  int L = 8;
+  const int want = env_int("RISM3D_ZSTAR_LINES", 0);
+  if (want == 2 || want == 4 || want == 8 || want == 16) L = want;
+  while (L > 2 && (size_t)m * L * lstride_for(N2) * sizeof(cpx<T>) > 64 * 1024) L /= 2;
+  return L;
+}
+
+// zstar_reg for the solute residual with 3 or 5 solvent sites (RISM3D_ZSTAR_LDS=1 keeps
+// the all-sites-in-LDS kernel), zstar otherwise.
+inline bool use_zreg(const GridArgs& g) {
+  static const int lds_only = env_int("RISM3D_ZSTAR_LDS", 0);
+  return !lds_only && g.special == 0 && (g.m == 3 || g.m == 5);
+}
+
+// The FP32 residual on xy planes (closure_r2c_xy, zstar, c2r_xy_resid:
+// three launches, the y transforms inside the plane kernels) when the
+// planes are square with 64, 96 or 128 points per side; otherwise, and in
+// FP64 (a 128^2 plane would take 133 KB of LDS), the five-launch chain.
+// RISM3D_PLANES=0 keeps the five-launch chain in FP32 too.  The plane
+// kernels write W y-major with the Nyquist column apart (GridArgs::ylay),
+// which only zstar_reg reads (3 or 5 solvent sites).
+inline bool use_planes(const GridArgs& g, bool fp32, int on) {
+  return on && fp32 && g.special == 0 && g.N0 == g.N1 &&
+         (g.N0 == 64 || g.N0 == 96 || g.N0 == 128) && use_zreg(g);
+}
+
+template <typename T>
+void launch_closure_r2c(int N0, dim3 grid, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
+                        const cpx<T>* twh, const cpx<T>* twf, int hist);
+template <typename T>
+void launch_c2r_resid(int N0, dim3 grid, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
+                      const cpx<T>* twh, const cpx<T>* twf, int hist);
+template <typename T, bool INV>
+void launch_fft_y(int N1, dim3 grid, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
+                  const cpx<T>* tw);
+template <typename T>
+void launch_zstar(int N2, int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd,
+                  const GridArgs& g, const cpx<T>* tw, const T* chi, const T* tau);
+template <typename T>
+void launch_planes(bool inv, int B, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
+                   const cpx<T>* twh, const cpx<T>* twf, const cpx<T>* twy, int hist);
+
+}  // namespace rism

@@ -21,6 +21,7 @@
 
 #include "../../include/rism3d.h"
 
+#include "chain_launch.hpp"
 #include "kernels.hip"
 
 // The fixed device scratch of rism3d_residual_noalloc: every device buffer
@@ -43,219 +44,10 @@ namespace {
     }                                                                                    \
   } while (0)
 
-struct HipFailure {
-  hipError_t err;
-};
-
 bool supported_n(int n) {
   switch (n) {
     case 32: case 48: case 64: case 96: case 128: case 192: case 256: case 384: return true;
     default: return false;
-  }
-}
-
-// ----------------------------------------------------- kernel dispatch
-#define RISM_FOR_N(X) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384)
-
-// The history loads of the closure and residual kernels are unrolled over
-// H slots held in registers: the smallest of 8, 10 and MAX_DIIS that holds
-// every solute's history (at 10 slots the residual kernel keeps 80 fewer
-// bytes per lane in flight than at 16).
-template <typename T>
-void launch_closure_r2c(int N0, dim3 grid, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
-                        const cpx<T>* twh, const cpx<T>* twf, int hist) {
-  if (hist <= 8) {
-    switch (N0) {
-#define X(n) case n: hipLaunchKernelGGL((closure_r2c_x<T, n, 8>), grid, dim3(NT), 0, s, sd, g, twh, twf); break;
-      RISM_FOR_N(X)
-#undef X
-    }
-    return;
-  }
-  if (hist <= 10) {
-    switch (N0) {
-#define X(n) case n: hipLaunchKernelGGL((closure_r2c_x<T, n, 10>), grid, dim3(NT), 0, s, sd, g, twh, twf); break;
-      RISM_FOR_N(X)
-#undef X
-    }
-    return;
-  }
-  switch (N0) {
-#define X(n) case n: hipLaunchKernelGGL((closure_r2c_x<T, n, MAX_DIIS>), grid, dim3(NT), 0, s, sd, g, twh, twf); break;
-    RISM_FOR_N(X)
-#undef X
-  }
-}
-template <typename T>
-void launch_c2r_resid(int N0, dim3 grid, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
-                      const cpx<T>* twh, const cpx<T>* twf, int hist) {
-  if (hist <= 8) {
-    switch (N0) {
-#define X(n) case n: hipLaunchKernelGGL((c2r_x_resid<T, n, 8>), grid, dim3(NT), 0, s, sd, g, twh, twf); break;
-      RISM_FOR_N(X)
-#undef X
-    }
-    return;
-  }
-  if (hist <= 10) {
-    switch (N0) {
-#define X(n) case n: hipLaunchKernelGGL((c2r_x_resid<T, n, 10>), grid, dim3(NT), 0, s, sd, g, twh, twf); break;
-      RISM_FOR_N(X)
-#undef X
-    }
-    return;
-  }
-  switch (N0) {
-#define X(n) case n: hipLaunchKernelGGL((c2r_x_resid<T, n, MAX_DIIS>), grid, dim3(NT), 0, s, sd, g, twh, twf); break;
-    RISM_FOR_N(X)
-#undef X
-  }
-}
-template <typename T> constexpr int y_lines() { return 128 / (int)sizeof(cpx<T>); }
-template <typename T, bool INV>
-void launch_fft_y(int N1, dim3 grid, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
-                  const cpx<T>* tw) {
-  constexpr int LN = y_lines<T>();
-  switch (N1) {
-#define X(n) case n: hipLaunchKernelGGL((fft_y<T, n, LN, INV>), grid, dim3(NT), 0, s, sd, g, tw); break;
-    RISM_FOR_N(X)
-#undef X
-  }
-}
-template <typename T, int LINES>
-void launch_zstar_l(int N2, dim3 grid, size_t lds, hipStream_t s, const SoluteDesc* sd,
-                    const GridArgs& g, const cpx<T>* tw, const T* chi, const T* tau) {
-  switch (N2) {
-#define X(n) case n: hipLaunchKernelGGL((zstar<T, n, LINES>), grid, dim3(NT), lds, s, sd, g, tw, chi, tau); break;
-    RISM_FOR_N(X)
-#undef X
-  }
-}
-// Tuning knobs, read once: RISM3D_ZSTAR_LINES (kx columns per zstar
-// workgroup, 2..16) and RISM3D_ZSTAR_ORDER (0..3, see zstar_reg).
-int env_int(const char* name, int dflt) {
-  const char* v = std::getenv(name);
-  return v ? std::atoi(v) : dflt;
-}
-template <typename T>
-int zstar_lines(int N2, int m) {
-  // 8 kx columns per workgroup (64 B FP32, 128 B FP64 rows): at 128^3 the
-  // FP32 pass ran 1.7 ms with 8 against 2.25 ms with 16 and 2.3 ms with 4
-  // (64 solutes, m = 3; occupancy against row length)
-  int L = 8;
-  const int want = env_int("RISM3D_ZSTAR_LINES", 0);
-  if (want == 2 || want == 4 || want == 8 || want == 16) L = want;
-  while (L > 2 && (size_t)m * L * lstride_for(N2) * sizeof(cpx<T>) > 64 * 1024) L /= 2;
-  return L;
-}
-template <typename T, int N2, int NTZ = NT>
-void launch_zreg_n(int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
-                   const cpx<T>* tw, const T* chi, const T* tau) {
-  // NTZ threads: the same points per thread over NTZ / NT times the columns
-  constexpr int L = zreg_lines<T, N2>() * (NTZ / NT);
-  // In FP32 the Nyquist column kx = N0/2 gets a launch of its own (NYQ,
-  // LINES rows per workgroup) when the tiles of LINES columns end just
-  // before it, instead of a tile that holds it alone (one workgroup in five
-  // at N0 = 128): 1.19 -> 1.08 ms per pass at 64 x 128^3 (2, 4, 8 or 16
-  // rows per Nyquist workgroup alike).  In FP64, and in the y passes, the
-  // separate launch cost more than the tile it replaced.  RISM3D_NYQ=0
-  // keeps it in the last tile (g.nyq).
-  const bool split = g.nyq && sizeof(T) == 4 && NX > 1 && (NX - 1) % L == 0;
-  if (g.ylay && !split) {  // evaluate forces the split for the plane chain
-    std::fprintf(stderr, "rism3d: y-major spectra need the Nyquist launch\n");
-    throw HipFailure{hipErrorInvalidValue};
-  }
-  const int tiles = split ? (NX - 1) / L : (NX + L - 1) / L;
-  GridArgs gz = g;
-  if (gz.zorder == 2 && (tiles * N1) % 8 != 0) gz.zorder = 1;  // whole tiles per XCD
-  if (gz.zorder == 3 && N1 % 8 != 0) gz.zorder = 1;             // whole rows per XCD
-  gz.zB = B;
-  gz.ztiles = tiles;
-  const dim3 grid = gz.zorder >= 2 ? dim3(tiles * N1 * B)
-                  : gz.zorder ? dim3(tiles, N1, B) : dim3(B, tiles, N1);
-  const dim3 gn((N1 + L - 1) / L, 1, B);
-  if (g.m == 3) {
-    hipLaunchKernelGGL((zstar_reg<T, N2, L, 3, false, NTZ>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
-    if (split) hipLaunchKernelGGL((zstar_reg<T, N2, L, 3, true, NTZ>), gn, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
-  } else {
-    hipLaunchKernelGGL((zstar_reg<T, N2, L, 5, false, NTZ>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
-    if (split) hipLaunchKernelGGL((zstar_reg<T, N2, L, 5, true, NTZ>), gn, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
-  }
-}
-// The FP32 residual on xy planes (closure_r2c_xy, zstar, c2r_xy_resid:
-// three launches, the y transforms inside the plane kernels) when the
-// planes are square with 64, 96 or 128 points per side; otherwise, and in
-// FP64 (a 128^2 plane would take 133 KB of LDS), the five-launch chain.
-// RISM3D_PLANES=0 keeps the five-launch chain in FP32 too.  The plane
-// kernels write W y-major with the Nyquist column apart (GridArgs::ylay),
-// which only zstar_reg reads (3 or 5 solvent sites).
-bool use_zreg(const GridArgs& g);
-bool use_planes(const GridArgs& g, bool fp32, int on) {
-  return on && fp32 && g.special == 0 && g.N0 == g.N1 &&
-         (g.N0 == 64 || g.N0 == 96 || g.N0 == 128) && use_zreg(g);
-}
-template <typename T, int N, int H>
-void launch_planes_h(bool inv, dim3 grid, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
-                     const cpx<T>* twh, const cpx<T>* twf, const cpx<T>* twy) {
-  if (inv)
-    hipLaunchKernelGGL((c2r_xy_resid<T, N, N, H>), grid, dim3(NTP), 0, s, sd, g, twh, twf, twy);
-  else
-    hipLaunchKernelGGL((closure_r2c_xy<T, N, N, H>), grid, dim3(NTP), 0, s, sd, g, twh, twf, twy);
-}
-template <typename T, int N>
-void launch_planes_n(bool inv, dim3 grid, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
-                     const cpx<T>* twh, const cpx<T>* twf, const cpx<T>* twy, int hist) {
-  if (hist <= 8) launch_planes_h<T, N, 8>(inv, grid, s, sd, g, twh, twf, twy);
-  else if (hist <= 10) launch_planes_h<T, N, 10>(inv, grid, s, sd, g, twh, twf, twy);
-  else launch_planes_h<T, N, MAX_DIIS>(inv, grid, s, sd, g, twh, twf, twy);
-}
-// Grid: x = z plane, y = site, z = solute.
-template <typename T>
-void launch_planes(bool inv, int B, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
-                   const cpx<T>* twh, const cpx<T>* twf, const cpx<T>* twy, int hist) {
-  const dim3 grid(g.N2, g.m, B);
-  switch (g.N0) {
-    case 64: launch_planes_n<T, 64>(inv, grid, s, sd, g, twh, twf, twy, hist); break;
-    case 96: launch_planes_n<T, 96>(inv, grid, s, sd, g, twh, twf, twy, hist); break;
-    case 128: launch_planes_n<T, 128>(inv, grid, s, sd, g, twh, twf, twy, hist); break;
-  }
-}
-
-// zstar_reg for the solute residual with 3 or 5 solvent sites (RISM3D_ZSTAR_LDS=1 keeps
-// the all-sites-in-LDS kernel), zstar otherwise.
-bool use_zreg(const GridArgs& g) {
-  static const int lds_only = env_int("RISM3D_ZSTAR_LDS", 0);
-  return !lds_only && g.special == 0 && (g.m == 3 || g.m == 5);
-}
-template <typename T>
-void launch_zstar(int N2, int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd,
-                  const GridArgs& g, const cpx<T>* tw, const T* chi, const T* tau) {
-  if (use_zreg(g)) {
-    if (g.zwide && sizeof(T) == 4 && N2 <= 128) {  // 512 threads over 32 kx columns
-      switch (N2) {
-        case 32: launch_zreg_n<T, 32, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
-        case 48: launch_zreg_n<T, 48, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
-        case 64: launch_zreg_n<T, 64, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
-        case 96: launch_zreg_n<T, 96, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
-        case 128: launch_zreg_n<T, 128, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
-      }
-      return;
-    }
-    switch (N2) {
-#define X(n) case n: launch_zreg_n<T, n>(NX, N1, B, s, sd, g, tw, chi, tau); break;
-      RISM_FOR_N(X)
-#undef X
-    }
-    return;
-  }
-  const int L = zstar_lines<T>(N2, g.m);
-  const size_t lds = (size_t)g.m * L * lstride_for(N2) * sizeof(cpx<T>);
-  const dim3 grid = g.zorder ? dim3((NX + L - 1) / L, N1, B) : dim3(B, (NX + L - 1) / L, N1);
-  switch (L) {
-    case 2: launch_zstar_l<T, 2>(N2, grid, lds, s, sd, g, tw, chi, tau); break;
-    case 4: launch_zstar_l<T, 4>(N2, grid, lds, s, sd, g, tw, chi, tau); break;
-    case 8: launch_zstar_l<T, 8>(N2, grid, lds, s, sd, g, tw, chi, tau); break;
-    default: launch_zstar_l<T, 16>(N2, grid, lds, s, sd, g, tw, chi, tau); break;
   }
 }
 
