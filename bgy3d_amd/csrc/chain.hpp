@@ -870,7 +870,9 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
 // -------------------------------------- 5. x c2r fused with the residual
 // t' = c2r(...), r = t' - t, u = t + lam r, and per workgroup the partial
 // max|r|, sum r^2 and dots <r, r_j> with the history (MDIIS Gram row), to
-// part[(site * gridDim.x + blockIdx.x) * NPART + q].  Grid as closure_r2c_x.
+// part[q * nparts + site * gridDim.x + blockIdx.x], nparts = m gridDim.x: the
+// partials of one quantity together, as reduce_resid reads them.  Grid as
+// closure_r2c_x.
 template <typename T, int N0, int H>
 __global__ void __launch_bounds__(NT)
 c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
@@ -1078,7 +1080,7 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
     const int q = threadIdx.x;
     double a = red[q][0];
     for (int i = 1; i < NT / 64; ++i) a = (q == 0) ? fmax(a, red[q][i]) : a + red[q][i];
-    gst(d.part + ((int64_t)site * gridDim.x + blockIdx.x) * NPART + q, a);
+    gst(d.part + (int64_t)q * (gridDim.x * gridDim.y) + site * gridDim.x + blockIdx.x, a);
   }
 }
 
@@ -1169,8 +1171,8 @@ closure_r2c_xy(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __re
 // Z_{N0/2-k} from bins k and N0/2 - k; Im of the DC and Nyquist bins
 // dropped, as FFTW's c2r does), the inverse N0/2-point row FFTs, then
 // r = t' - t (or the mode's form), u = t + lam r and the partials max|r|,
-// sum r^2, <r, r_j> as c2r_x_resid, one partial row per plane at
-// part[(site * N2 + z) * NPART + q].  Grid as closure_r2c_xy.
+// sum r^2, <r, r_j> as c2r_x_resid, one partial per plane and quantity at
+// part[q * m N2 + site * N2 + z].  Grid as closure_r2c_xy.
 template <typename T, int N0, int N1, int H>
 __global__ void __launch_bounds__(NTP)
 c2r_xy_resid(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ tw_half,
@@ -1374,7 +1376,7 @@ c2r_xy_resid(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __rest
     const int q = threadIdx.x;
     double a = red[q][0];
     for (int i = 1; i < NTP / 64; ++i) a = (q == 0) ? fmax(a, red[q][i]) : a + red[q][i];
-    gst(d.part + ((int64_t)site * gridDim.x + blockIdx.x) * NPART + q, a);
+    gst(d.part + (int64_t)q * (gridDim.x * gridDim.y) + site * gridDim.x + blockIdx.x, a);
   }
 }
 

@@ -558,7 +558,7 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
     g.nyq = 1;
     if (g.zwide && (g.NX - 1) % 32 != 0) g.zwide = 0;
   }
-  const int nparts = planes ? g.m * g.N2 : pb.nparts;  // partial rows per solute
+  const int nparts = planes ? g.m * g.N2 : resid_grid_x(g) * g.m;  // partials per quantity
   auto chain = [&]() {
     if (planes) {
       using T = float;
@@ -584,7 +584,9 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
       mark(3, 0); launch_fft_y<T, true>(g.N1, gy, pb.s, dsd, g, pb.tw.d[2].p); mark(3, 1);
       mark(4, 0); launch_c2r_resid<T>(g.N0, gx, pb.s, dsd, g, pb.tw.d[1].p, pb.tw.d[0].p, hist); mark(4, 1);
     }
-    hipLaunchKernelGGL(reduce_resid, dim3(pb.B), dim3(NT), 0, pb.s, dsd, nparts, pb.d_out.p);
+    // 2 + the history width this launch (or graph, captured per width) serves
+    const int nq = 2 + (hist <= 8 ? 8 : (hist <= 10 ? 10 : MAX_DIIS));
+    hipLaunchKernelGGL(reduce_resid, dim3(nq, pb.B), dim3(NTR), 0, pb.s, dsd, nparts, pb.d_out.p);
     if (step)
       hipLaunchKernelGGL(mdiis_step, dim3(pb.B), dim3(64), 0, pb.s, pb.d_out.p, pb.d_mdiis.p, dsd,
                          pb.h_status.p);
