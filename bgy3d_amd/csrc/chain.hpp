@@ -562,8 +562,7 @@ zstar(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ 
           lds[(s * LINES + l) * LS + lpos(z)] = cpx<T>{T(U * sgn * g.inv_L3), T(0)};
         continue;
       }
-      if (g.msol <= 3) oz_pairs<T, 3, LINES, LS>(lds, g, chi3, kk, l, z, sgn, U);
-      else oz_pairs<T, MAX_SITES, LINES, LS>(lds, g, chi3, kk, l, z, sgn, U);
+      oz_pairs<T, MAX_SITES, LINES, LS>(lds, g, chi3, kk, l, z, sgn, U);
     }
   } else {
   const cpx<T>* Fs = static_cast<const cpx<T>*>(d.Fs);
@@ -634,6 +633,99 @@ __device__ __forceinline__ double warp_max(double v) {
   return v;
 }
 
+// oz_pairs for a compile-time site count MS, the MS (MS + 1) / 2 pair spectra
+// of the point in registers (c, overwritten with T), w the omega of the
+// off-diagonal pairs (1 on the diagonal).  Every loop unrolls and the row
+// exchanges are selects, so nothing is indexed at run time.
+template <int MS>
+__device__ __forceinline__ void oz_point(cpx<double> (&c)[MS * (MS + 1) / 2],
+                                         const double (&w)[MS * (MS + 1) / 2], const GridArgs& g,
+                                         double sgn, double U) {
+  auto pr = [](int i, int j) { return i >= j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i; };
+  cpx<double> A[MS][MS], B[MS][MS];
+#pragma unroll
+  for (int i = 0; i < MS; ++i)
+#pragma unroll
+    for (int j = 0; j <= i; ++j) {  // C = h^3 c s - beta q_i q_j U
+      cpx<double>& v = c[pr(i, j)];
+      v = cpx<double>{v.re * g.h3 * sgn - g.beta * (g.q[i] * g.q[j]) * U, v.im * g.h3 * sgn};
+    }
+#pragma unroll
+  for (int i = 0; i < MS; ++i)
+#pragma unroll
+    for (int j = 0; j < MS; ++j) {  // W C, A = 1 - rho W C
+      cpx<double> a = {0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < MS; ++q) a = cadd(a, cscale(c[pr(q, j)], w[pr(i, q)]));
+      B[i][j] = a;
+      A[i][j] = cpx<double>{(i == j ? 1.0 : 0.0) - g.rho * a.re, -g.rho * a.im};
+    }
+#pragma unroll
+  for (int i = 0; i < MS; ++i) {  // B = W C W, row by row
+    cpx<double> row[MS];
+#pragma unroll
+    for (int j = 0; j < MS; ++j) row[j] = B[i][j];
+#pragma unroll
+    for (int j = 0; j < MS; ++j) {
+      cpx<double> b = {0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < MS; ++q) b = cadd(b, cscale(row[q], w[pr(q, j)]));
+      B[i][j] = b;
+    }
+  }
+  // Gaussian elimination with partial pivoting, A X = B
+#pragma unroll
+  for (int col = 0; col < MS; ++col) {
+    int piv = col;
+    double best = A[col][col].re * A[col][col].re + A[col][col].im * A[col][col].im;
+#pragma unroll
+    for (int r = col + 1; r < MS; ++r) {
+      const double a2 = A[r][col].re * A[r][col].re + A[r][col].im * A[r][col].im;
+      if (a2 > best) { best = a2; piv = r; }
+    }
+#pragma unroll
+    for (int r = col + 1; r < MS; ++r) {
+      const bool sw = piv == r;
+#pragma unroll
+      for (int q = 0; q < MS; ++q) {
+        const cpx<double> a0 = A[col][q], a1 = A[r][q], b0 = B[col][q], b1 = B[r][q];
+        A[col][q] = {sw ? a1.re : a0.re, sw ? a1.im : a0.im};
+        A[r][q] = {sw ? a0.re : a1.re, sw ? a0.im : a1.im};
+        B[col][q] = {sw ? b1.re : b0.re, sw ? b1.im : b0.im};
+        B[r][q] = {sw ? b0.re : b1.re, sw ? b0.im : b1.im};
+      }
+    }
+    const double den = A[col][col].re * A[col][col].re + A[col][col].im * A[col][col].im;
+    const cpx<double> inv = {A[col][col].re / den, -A[col][col].im / den};
+#pragma unroll
+    for (int r = col + 1; r < MS; ++r) {
+      const cpx<double> f = cmul(A[r][col], inv);
+#pragma unroll
+      for (int q = col + 1; q < MS; ++q) A[r][q] = csub(A[r][q], cmul(f, A[col][q]));
+#pragma unroll
+      for (int q = 0; q < MS; ++q) B[r][q] = csub(B[r][q], cmul(f, B[col][q]));
+    }
+    A[col][col] = inv;  // 1 / pivot, for the back substitution
+  }
+#pragma unroll
+  for (int col = MS - 1; col >= 0; --col)
+#pragma unroll
+    for (int q = 0; q < MS; ++q) {
+      cpx<double> x = B[col][q];
+#pragma unroll
+      for (int r = col + 1; r < MS; ++r) x = csub(x, cmul(A[col][r], B[r][q]));
+      B[col][q] = cmul(x, A[col][col]);
+    }
+#pragma unroll
+  for (int i = 0; i < MS; ++i)
+#pragma unroll
+    for (int j = 0; j <= i; ++j) {  // T = ((X - C) - beta q_i q_j U) s / L^3
+      cpx<double>& v = c[pr(i, j)];
+      v = cpx<double>{((B[i][j].re - v.re) - g.beta * (g.q[i] * g.q[j]) * U) * sgn * g.inv_L3,
+                      (B[i][j].im - v.im) * sgn * g.inv_L3};
+    }
+}
+
 // --------------------------- 3b. zstar with the spectra held in registers
 // Mode 3: forward z FFTs only; mode 4: inverse z FFTs only.
 // The solute residual's k-space step (modes 0-7 of zstar, special 0) for a
@@ -643,6 +735,10 @@ __device__ __forceinline__ double warp_max(double v) {
 // workgroup is 1/MS of zstar's, so a 128-byte row of kx columns (16 FP32
 // or 8 FP64) fits at high occupancy.  Same arithmetic as zstar, point by
 // point.  Grid as zstar.
+// OZ > 0 (FP64, special 1): the solvent-solvent step of OZ sites instead,
+// MS = OZ (OZ + 1) / 2 pairs (oz_point).  zstar's oz_pairs keeps its matrices
+// in scratch (their loops run to a run-time site count) and took 60% of a
+// three-site pass: 142 us at 64^3, here 25 us (43 MB of spectra and tables).
 template <typename T, int N2>
 constexpr int zreg_lines() {
   int L = 128 / (int)sizeof(cpx<T>);
@@ -651,7 +747,7 @@ constexpr int zreg_lines() {
   return L;
 }
 
-template <typename T, int N2, int LINES, int MS, bool NYQ, int NTZ = NT>
+template <typename T, int N2, int LINES, int MS, bool NYQ, int NTZ = NT, int OZ = 0>
 __global__ void __launch_bounds__(NTZ)
 zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ tw,
           const T* __restrict__ chi3, const T* __restrict__ tau3) {
@@ -784,6 +880,37 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
   if (d.mode == 3) return;
   const bool linear = d.mode != 0;  // chi convolution only
   const cpx<T>* Fs = static_cast<const cpx<T>*>(d.Fs);
+  if constexpr (OZ > 0) {
+    static_assert(MS == OZ * (OZ + 1) / 2 && !NYQ && sizeof(T) == 8, "site pairs, FP64");
+    const int iy = (y <= g.N1 / 2) ? y : y - g.N1;
+#pragma unroll
+    for (int p = 0; p < PPT; ++p) {
+      const int e = tid + p * NTZ;
+      const int z = e / LINES, l = e - z * LINES;
+      if (d.mode == 4 || !(PPT * NTZ == PTS || e < PTS) || l >= nl) continue;
+      const uint32_t kk = (uint32_t)(base + z * zs + l);
+      const int iz = (z <= N2 / 2) ? z : z - N2, ix = kx0 + l;
+      const double sgn = ((ix + iy + iz) & 1) ? -1.0 : 1.0;
+      // the unit long-range Coulomb as zstar forms it
+      const double kabs = sqrt(kmag2(ix * g.dkx, iy * g.dky, iz * g.dkz));
+      const double k2 = kabs * kabs;
+      const double U = k2 == 0.0 ? 0.0
+          : (4 * M_PI * EPSILON0INV) * exp(-k2 / (4 * G_COULOMB * G_COULOMB)) / k2;
+      double w[MS];
+      cpx<double> v[MS];
+#pragma unroll
+      for (int i = 0; i < OZ; ++i)
+#pragma unroll
+        for (int j = 0; j <= i; ++j) {
+          const int q = i * (i + 1) / 2 + j;
+          w[q] = i == j ? 1.0 : gld(at32(chi3 + q * g.K, kk));
+          v[q] = c[q][p];
+        }
+      oz_point<OZ>(v, w, g, sgn, U);
+#pragma unroll
+      for (int q = 0; q < MS; ++q) c[q][p] = v[q];
+    }
+  } else
 #pragma unroll
   for (int p = 0; p < PPT; ++p) {
     const int e = tid + p * NTZ;

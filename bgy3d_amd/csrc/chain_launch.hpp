@@ -34,11 +34,14 @@ int zstar_lines(int N2, int m) {
   return L;
 }
 
-// zstar_reg for the solute residual with 3 or 5 solvent sites (RISM3D_ZSTAR_LDS=1 keeps
-// the all-sites-in-LDS kernel), zstar otherwise.
+// zstar_reg for the solute residual with 3 or 5 solvent sites and for the 3D
+// solvent of at most 3 sites, whose points fit in registers (6 pairs: 24 to
+// 48 registers a thread; 4 sites are 10 pairs); zstar otherwise, and for all
+// with RISM3D_ZSTAR_LDS=1.
 inline bool use_zreg(const GridArgs& g) {
   static const int lds_only = env_int("RISM3D_ZSTAR_LDS", 0);
-  return !lds_only && g.special == 0 && (g.m == 3 || g.m == 5);
+  return !lds_only && ((g.special == 0 && (g.m == 3 || g.m == 5)) ||
+                       (g.special == 1 && g.msol <= 3));
 }
 
 // The FP32 residual on xy planes (closure_r2c_xy, zstar, c2r_xy_resid:

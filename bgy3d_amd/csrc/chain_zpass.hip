@@ -46,6 +46,17 @@ void launch_zreg_n(int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd, c
   const dim3 grid = gz.zorder >= 2 ? dim3(tiles * N1 * B)
                   : gz.zorder ? dim3(tiles, N1, B) : dim3(B, tiles, N1);
   const dim3 gn((N1 + L - 1) / L, 1, B);
+  if constexpr (sizeof(T) == 8 && NTZ == NT) {
+    if (g.special == 1) {
+      if (g.msol == 1)
+        hipLaunchKernelGGL((zstar_reg<T, N2, L, 1, false, NTZ, 1>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
+      else if (g.msol == 2)
+        hipLaunchKernelGGL((zstar_reg<T, N2, L, 3, false, NTZ, 2>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
+      else
+        hipLaunchKernelGGL((zstar_reg<T, N2, L, 6, false, NTZ, 3>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
+      return;
+    }
+  }
   if (g.m == 3) {
     hipLaunchKernelGGL((zstar_reg<T, N2, L, 3, false, NTZ>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
     if (split) hipLaunchKernelGGL((zstar_reg<T, N2, L, 3, true, NTZ>), gn, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);

@@ -326,3 +326,23 @@ def test_cli_solvent_3d(tmp_path, capsys, monkeypatch):
     assert abs(mu["HNC"] - ref["free-energy-hnc"]) < 1e-6
     assert "q_v = " in text and "<ρ_v|U_u> = " in text
     assert (tmp_path / "g0.bin").exists() and (tmp_path / "g2.bin").exists()
+
+
+@pytest.mark.parametrize("name,rho,N", [("OW", 0.02, 32), ("hydrogen chloride", 0.012, 48),
+                                        ("hydrogen chloride", 0.012, 64), ("water", RHO, 96),
+                                        ("water", RHO, 128)])
+def test_few_site_solvent_root_is_the_oracles(name, rho, N):
+    """The per-k OZ solve with the pairs in registers (1, 2 and 3 sites; z
+    lines whose points stay in registers or pass through LDS): the
+    converged t is the oracle's root too, max|F_oracle(t)| <= 1e-9 (1e-11
+    asked, the rest rounding of F terms of order 100)."""
+    print(f"case solvent3d {name} n{N}", flush=True)
+    from bgy3d_amd import rism3d as R
+    from bgy3d_amd.solutes import find_molecule
+    mol = find_molecule(name)
+    out = R.hnc3d_run_solvent(name, _settings(N, 0.15 * N, rho=rho, **{"norm-tol": 1e-11}))
+    assert out["status"] == "OK"
+    pd = O.Problem.from_cli(0.15 * N, N, BETA, rho, closure=C.KH, rmax=40.0, nrad=16 * N)
+    f = S3.Solvent3D(pd, mol).iterate(out["t"])
+    print(f"  iters {out['iterations']} max|F_oracle| {np.max(np.abs(f)):.2e}", flush=True)
+    assert np.max(np.abs(f)) <= 1e-9
