@@ -747,66 +747,73 @@ constexpr int zreg_lines() {
   return L;
 }
 
-template <typename T, int N2, int LINES, int MS, bool NYQ, int NTZ = NT, int OZ = 0>
+template <typename T, int N2, int LINES, int MS, int NTZ = NT, int OZ = 0>
 __global__ void __launch_bounds__(NTZ)
 zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ tw,
           const T* __restrict__ chi3, const T* __restrict__ tau3) {
   constexpr int PTS = N2 * LINES;
   constexpr int PPT = (PTS + NTZ - 1) / NTZ;
   __shared__ cpx<T> lds[PTS];  // interleaved: point z of line l at z * LINES + l
-  // Block order.  zorder 2 (1D grid): consecutive blocks go to the XCDs in
+  // Block order of the 1D grid.  First the Nyquist blocks of a split launch
+  // (nyq: lines are LINES rows ky of the column kx = N0/2), whose scattered
+  // accesses then run beside the tiles instead of after them; a launch of
+  // their own took 98 us beside 174 us at 192^3 with 5 sites and 27 beside
+  // 285 us at 24 x 128^3 (FP32); the one launch 192 and 295.  Then the tiles:
+  // zorder 2: consecutive blocks go to the XCDs in
   // turn, and each XCD walks all solutes of one (ky, kx tile) before the
   // next, so the tile's chi and tau stay in that XCD's L2 for every solute.
-  // zorder 3 (1D grid): XCD x owns the rows ky = x (mod 8) and walks every
+  // zorder 3: XCD x owns the rows ky = x (mod 8) and walks every
   // solute of a row, the row's kx tiles back to back, so each z line's
   // columns are read by neighbouring workgroups at once (whole rows of the
   // z planes instead of one tile's 128 bytes) and the row's chi and tau
   // stay in the XCD's L2 across solutes.
-  // zorder 1: x = kx tile, y = ky, z = solute; zorder 0: x = solute,
-  // y = kx tile, z = ky.
+  // zorder 1: kx tile fastest, then ky, then the solute; zorder 0: solute
+  // fastest, then the kx tile.
   int b, tile, ky;
-  if (NYQ) {
-    b = blockIdx.z;
+  const int nnyq = g.nyqb * g.zB;
+  const bool nyq = (int)blockIdx.x < nnyq;
+  if (nyq) {
+    b = blockIdx.x / g.nyqb;
     tile = 0;
-    ky = blockIdx.x * LINES;
-  } else if (g.zorder == 3) {
-    const int lin = blockIdx.x, xcd = lin & 7, slot = lin >> 3;
-    tile = slot % g.ztiles;
-    b = (slot / g.ztiles) % g.zB;
-    ky = (slot / (g.ztiles * g.zB)) * 8 + xcd;
-  } else if (g.zorder == 2) {
-    const int lin = blockIdx.x, xcd = lin & 7, slot = lin >> 3;
-    const int gt = (slot / g.zB) * 8 + xcd;  // global tile, ky-major
-    b = slot - (slot / g.zB) * g.zB;
-    tile = gt % g.ztiles;
-    ky = gt / g.ztiles;
-  } else if (g.zorder == 1) {
-    b = blockIdx.z;
-    tile = blockIdx.x;
-    ky = blockIdx.y;
+    ky = (blockIdx.x - b * g.nyqb) * LINES;
   } else {
-    b = blockIdx.x;
-    tile = blockIdx.y;
-    ky = blockIdx.z;
+    const int lin = blockIdx.x - nnyq, xcd = lin & 7, slot = lin >> 3;
+    if (g.zorder == 3) {
+      tile = slot % g.ztiles;
+      b = (slot / g.ztiles) % g.zB;
+      ky = (slot / (g.ztiles * g.zB)) * 8 + xcd;
+    } else if (g.zorder == 2) {
+      const int gt = (slot / g.zB) * 8 + xcd;  // global tile, ky-major
+      b = slot - (slot / g.zB) * g.zB;
+      tile = gt % g.ztiles;
+      ky = gt / g.ztiles;
+    } else if (g.zorder == 1) {
+      tile = lin % g.ztiles;
+      ky = (lin / g.ztiles) % g.N1;
+      b = lin / (g.ztiles * g.N1);
+    } else {
+      b = lin % g.zB;
+      tile = (lin / g.zB) % g.ztiles;
+      ky = lin / (g.zB * g.ztiles);
+    }
   }
   const SoluteDesc& d = sd[b];
   if (!d.active) return;
-  // NYQ: lines are the rows y0 + l of the Nyquist column kx = N0/2 (grid
-  // x = ceil(N1 / LINES), y = 1, z = solute); otherwise the kx columns
-  // kx0 + l of row y.
+  // nyq: lines are the rows y0 + l of the Nyquist column kx = N0/2;
+  // otherwise the kx columns kx0 + l of row y.
   const int y = ky;
-  const int kx0 = NYQ ? g.NX - 1 : tile * LINES;
+  const int kx0 = nyq ? g.NX - 1 : tile * LINES;
   // element offsets below 2^32 bytes from per-workgroup bases (at32): the
   // tables and Fs from their starts, W from its site's
   const int zs = g.N1 * g.NH;         // z stride (Fs, chi, tau)
-  const int ls = NYQ ? g.NH : 1;      // line stride
+  const int ls = nyq ? g.NH : 1;      // line stride
   const int base = y * g.NH + kx0;
   // W: the same index unless ylay (y-major rows, compact Nyquist column)
   int wz = zs, wl = ls;
   int64_t wsite = g.K;
   cpx<T>* W = static_cast<cpx<T>*>(d.W) + base;
   if (g.ylay) {
-    if (NYQ) {
+    if (nyq) {
       W = static_cast<cpx<T>*>(d.W) + g.m * g.K + y;
       wz = g.N1;
       wl = 1;
@@ -816,7 +823,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
       wz = g.NH;
     }
   }
-  const int nl = NYQ ? min(LINES, g.N1 - y) : min(LINES, g.NX - kx0);  // valid lines
+  const int nl = nyq ? min(LINES, g.N1 - y) : min(LINES, g.NX - kx0);  // valid lines
   const int tid = threadIdx.x;
   cpx<T> c[MS][PPT];
   // every site's loads first, staged in its registers of c (its FFT result
@@ -881,7 +888,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
   const bool linear = d.mode != 0;  // chi convolution only
   const cpx<T>* Fs = static_cast<const cpx<T>*>(d.Fs);
   if constexpr (OZ > 0) {
-    static_assert(MS == OZ * (OZ + 1) / 2 && !NYQ && sizeof(T) == 8, "site pairs, FP64");
+    static_assert(MS == OZ * (OZ + 1) / 2 && sizeof(T) == 8, "site pairs, FP64");
     const int iy = (y <= g.N1 / 2) ? y : y - g.N1;
 #pragma unroll
     for (int p = 0; p < PPT; ++p) {
@@ -919,15 +926,15 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
     if (l >= nl) continue;
     const uint32_t kk = (uint32_t)(base + z * zs + l * ls);  // k-grid index of this point
     cpx<T> fs = {T(0), T(0)};
-    if (!linear) fs = ldc(at32(Fs, (uint32_t)fs_index<T>(g, z, NYQ ? y + l : y, kx0 + (NYQ ? 0 : l))));
+    if (!linear) fs = ldc(at32(Fs, (uint32_t)fs_index<T>(g, z, nyq ? y + l : y, kx0 + (nyq ? 0 : l))));
     cpx<T> uc = {T(0), T(0)};
     if (!g.renorm && !linear) {
       // u_c(k) = 4 pi eps0^-1 exp(-k^2/4G^2)/k^2 F(k) s(k), 0 at k = 0
       // (bgy3d-force.h:140-147, bgy3d-solutes.c:767-792).
       const int iz = (z <= N2 / 2) ? z : z - N2;
-      const int yl = NYQ ? y + l : y;
+      const int yl = nyq ? y + l : y;
       const int iy = (yl <= g.N1 / 2) ? yl : yl - g.N1;
-      const double k2 = kmag2((NYQ ? kx0 : kx0 + l) * g.dkx, iy * g.dky, iz * g.dkz);
+      const double k2 = kmag2((nyq ? kx0 : kx0 + l) * g.dkx, iy * g.dky, iz * g.dkz);
       const double shape = (k2 == 0.0) ? 0.0
           : (4 * M_PI * EPSILON0INV) * exp(-k2 / (4 * G_COULOMB * G_COULOMB)) / k2;
       uc = cscale(fs, T(shape));

@@ -25,13 +25,12 @@ void launch_zreg_n(int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd, c
                    const cpx<T>* tw, const T* chi, const T* tau) {
   // NTZ threads: the same points per thread over NTZ / NT times the columns
   constexpr int L = zreg_lines<T, N2>() * (NTZ / NT);
-  // In FP32 the Nyquist column kx = N0/2 gets a launch of its own (NYQ,
-  // LINES rows per workgroup) when the tiles of LINES columns end just
-  // before it, instead of a tile that holds it alone (one workgroup in five
-  // at N0 = 128): 1.19 -> 1.08 ms per pass at 64 x 128^3 (2, 4, 8 or 16
-  // rows per Nyquist workgroup alike).  In FP64, and in the y passes, the
-  // separate launch cost more than the tile it replaced.  RISM3D_NYQ=0
-  // keeps it in the last tile (g.nyq).
+  // In FP32 the Nyquist column kx = N0/2 gets blocks of its own (LINES rows
+  // each) when the tiles of LINES columns end just before it, instead of a
+  // tile that holds it alone (one workgroup in five at N0 = 128): 1.19 ->
+  // 1.08 ms per pass at 64 x 128^3.  In FP64 in rows, and in the y passes,
+  // that cost more than the tile it replaced.  RISM3D_NYQ=0 keeps it in the
+  // last tile (g.nyq).
   const bool split = g.nyq && sizeof(T) == 4 && NX > 1 && (NX - 1) % L == 0;
   if (g.ylay && !split) {  // evaluate forces the split for the plane chain
     std::fprintf(stderr, "rism3d: y-major spectra need the Nyquist launch\n");
@@ -43,26 +42,23 @@ void launch_zreg_n(int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd, c
   if (gz.zorder == 3 && N1 % 8 != 0) gz.zorder = 1;             // whole rows per XCD
   gz.zB = B;
   gz.ztiles = tiles;
-  const dim3 grid = gz.zorder >= 2 ? dim3(tiles * N1 * B)
-                  : gz.zorder ? dim3(tiles, N1, B) : dim3(B, tiles, N1);
-  const dim3 gn((N1 + L - 1) / L, 1, B);
+  gz.nyqb = split ? (N1 + L - 1) / L : 0;
+  const dim3 grid(((size_t)tiles * N1 + gz.nyqb) * B);
   if constexpr (sizeof(T) == 8 && NTZ == NT) {
     if (g.special == 1) {
       if (g.msol == 1)
-        hipLaunchKernelGGL((zstar_reg<T, N2, L, 1, false, NTZ, 1>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
+        hipLaunchKernelGGL((zstar_reg<T, N2, L, 1, NTZ, 1>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
       else if (g.msol == 2)
-        hipLaunchKernelGGL((zstar_reg<T, N2, L, 3, false, NTZ, 2>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
+        hipLaunchKernelGGL((zstar_reg<T, N2, L, 3, NTZ, 2>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
       else
-        hipLaunchKernelGGL((zstar_reg<T, N2, L, 6, false, NTZ, 3>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
+        hipLaunchKernelGGL((zstar_reg<T, N2, L, 6, NTZ, 3>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
       return;
     }
   }
   if (g.m == 3) {
-    hipLaunchKernelGGL((zstar_reg<T, N2, L, 3, false, NTZ>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
-    if (split) hipLaunchKernelGGL((zstar_reg<T, N2, L, 3, true, NTZ>), gn, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
+    hipLaunchKernelGGL((zstar_reg<T, N2, L, 3, NTZ>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
   } else {
-    hipLaunchKernelGGL((zstar_reg<T, N2, L, 5, false, NTZ>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
-    if (split) hipLaunchKernelGGL((zstar_reg<T, N2, L, 5, true, NTZ>), gn, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
+    hipLaunchKernelGGL((zstar_reg<T, N2, L, 5, NTZ>), grid, dim3(NTZ), 0, s, sd, gz, tw, chi, tau);
   }
 }
 template <typename T>

@@ -133,8 +133,8 @@ struct GridArgs {
   int closure;         // enum rism3d_closure
   int pse_order;       // n of PSE-n, 1 for KH
   int zorder;          // zstar grid order (see zstar_reg)
-  int zB, ztiles;      // zorder 2: solutes and kx tiles of the launch
-  int nyq;             // FP32 z pass: the Nyquist column in a launch of its own
+  int zB, ztiles;      // z pass: solutes and kx tiles of the launch
+  int nyq;             // FP32 z pass: the Nyquist column in blocks of its own
   int zwide;           // FP32 z pass at N2 <= 128: 32 kx columns, 512 threads
   // ylay (the FP32 xy-plane chain): W is y-major, point (site, ky, z, kx <
   // N0/2) at site K + ky N2 NH + z NH + kx, so that the z pass reads whole
@@ -142,7 +142,7 @@ struct GridArgs {
   // behind the sites, (site, z, ky) at m K + site N1 N2 + z N1 + ky (cpx<T>
   // units).  0: W is z-major like the tables, [site][z][ky][NH].
   int ylay;
-  int pad_ylay_;
+  int nyqb;            // z pass: Nyquist blocks per solute (0: in the last tile)
   double q[MAX_SITES]; // solvent charges
   // zstar variants (0 solute residual): 1 solvent-solvent OZ on site-site
   // pairs (msol sites, pair p = i(i+1)/2 + j), 2 Poisson potential of a
