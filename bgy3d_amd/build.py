@@ -28,7 +28,7 @@ HIP_FLAGS = [
 UNITS = [("solver", "solver.hip", HIP_FLAGS), ("rism1d", "rism1d.cpp", None)] + [
     (f"{src}_{t[0]}", f"{src}.hip", HIP_FLAGS + [f"-DRISM_T={t}"])
     for src, types in (("chain_rows", ("double", "float")), ("chain_zpass", ("double", "float")),
-                       ("chain_planes", ("float",)))
+                       ("chain_planes", ("double", "float")))
     for t in types]
 
 

@@ -1,5 +1,6 @@
 // gfx950 kernels of the 3D-RISM residual F(t) = (chi - 1) * c(t) - t and
-// its setup / post-processing.  One residual evaluation is five launches:
+// its setup / post-processing.  One residual evaluation is five launches,
+// or three on xy planes (closure_r2c_xy, zstar, c2r_xy_resid):
 //
 //   1. closure_r2c_x : c = closure(beta v, t) fused into the x-axis r2c
 //   2. fft_y         : forward c2c along y
@@ -187,7 +188,8 @@ __device__ __forceinline__ Vec16<float> st_hist(const SoluteDesc& d, int64_t idx
 // z-major rows of NH like the tables in FP64; in FP32 y-major rows of
 // N0/2 bins (the layout of the plane chain's spectra) and the Nyquist
 // column kx = N0/2 compact behind them, so that the z pass reads it
-// as it reads the spectra.
+// as it reads the spectra.  (FP64 has that compact column too, at the same
+// place, for the z pass's Nyquist blocks.)
 template <typename T>
 __device__ __forceinline__ int64_t fs_index(const GridArgs& g, int z, int y, int x) {
   if constexpr (sizeof(T) == 8) return ((int64_t)z * g.N1 + y) * g.NH + x;
@@ -823,6 +825,15 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
       wz = g.NH;
     }
   }
+  // the tables: z-major rows, and the Nyquist column of each compact behind
+  // them all, (z, ky) at z N1 + ky, where a Nyquist block's lines are
+  // contiguous (8 bytes of each 128-byte line otherwise: at B = 1 such a
+  // block was the pass's last, 50 us against 33 for the rows at 96^3 in FP64)
+  constexpr int NTAB = OZ > 0 ? MS : MS * (MS + 1) / 2;  // chi3's tables
+  const int64_t tsite = nyq ? (int64_t)g.N1 * g.N2 : g.K;
+  const T* chit = nyq ? chi3 + NTAB * g.K : chi3;
+  const T* taut = nyq ? tau3 + MS * g.K : tau3;
+  const int tbase = nyq ? y : base, tz = nyq ? g.N1 : zs;
   const int nl = nyq ? min(LINES, g.N1 - y) : min(LINES, g.NX - kx0);  // valid lines
   const int tid = threadIdx.x;
   cpx<T> c[MS][PPT];
@@ -889,14 +900,15 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
   const cpx<T>* Fs = static_cast<const cpx<T>*>(d.Fs);
   if constexpr (OZ > 0) {
     static_assert(MS == OZ * (OZ + 1) / 2 && sizeof(T) == 8, "site pairs, FP64");
-    const int iy = (y <= g.N1 / 2) ? y : y - g.N1;
 #pragma unroll
     for (int p = 0; p < PPT; ++p) {
       const int e = tid + p * NTZ;
       const int z = e / LINES, l = e - z * LINES;
       if (d.mode == 4 || !(PPT * NTZ == PTS || e < PTS) || l >= nl) continue;
-      const uint32_t kk = (uint32_t)(base + z * zs + l);
-      const int iz = (z <= N2 / 2) ? z : z - N2, ix = kx0 + l;
+      const uint32_t kk = (uint32_t)(tbase + z * tz + l);
+      const int iz = (z <= N2 / 2) ? z : z - N2, ix = nyq ? kx0 : kx0 + l;
+      const int yl = nyq ? y + l : y;
+      const int iy = (yl <= g.N1 / 2) ? yl : yl - g.N1;
       const double sgn = ((ix + iy + iz) & 1) ? -1.0 : 1.0;
       // the unit long-range Coulomb as zstar forms it
       const double kabs = sqrt(kmag2(ix * g.dkx, iy * g.dky, iz * g.dkz));
@@ -910,7 +922,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
 #pragma unroll
         for (int j = 0; j <= i; ++j) {
           const int q = i * (i + 1) / 2 + j;
-          w[q] = i == j ? 1.0 : gld(at32(chi3 + q * g.K, kk));
+          w[q] = i == j ? 1.0 : gld(at32(chit + q * tsite, kk));
           v[q] = c[q][p];
         }
       oz_point<OZ>(v, w, g, sgn, U);
@@ -924,9 +936,11 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
     if (d.mode == 4 || !(PPT * NTZ == PTS || e < PTS)) continue;
     const int z = e / LINES, l = e - z * LINES;
     if (l >= nl) continue;
-    const uint32_t kk = (uint32_t)(base + z * zs + l * ls);  // k-grid index of this point
+    const uint32_t kk = (uint32_t)(tbase + z * tz + l);  // this point in the tables
     cpx<T> fs = {T(0), T(0)};
-    if (!linear) fs = ldc(at32(Fs, (uint32_t)fs_index<T>(g, z, nyq ? y + l : y, kx0 + (nyq ? 0 : l))));
+    if (!linear)
+      fs = ldc(at32(Fs, nyq ? (uint32_t)(g.K + z * g.N1 + y + l)
+                            : (uint32_t)fs_index<T>(g, z, y, kx0 + l)));
     cpx<T> uc = {T(0), T(0)};
     if (!g.renorm && !linear) {
       // u_c(k) = 4 pi eps0^-1 exp(-k^2/4G^2)/k^2 F(k) s(k), 0 at k = 0
@@ -944,7 +958,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
     }
     T chi[MS * (MS + 1) / 2];
 #pragma unroll
-    for (int q = 0; q < MS * (MS + 1) / 2; ++q) chi[q] = gld(at32(chi3 + q * g.K, kk));
+    for (int q = 0; q < MS * (MS + 1) / 2; ++q) chi[q] = gld(at32(chit + q * tsite, kk));
     cpx<T> out[MS];
 #pragma unroll
     for (int i = 0; i < MS; ++i) {
@@ -960,7 +974,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
         out[i] = cscale(acc, T(g.a_scale));
       } else if (g.renorm) {
         // (h^3/L^3) sum_j chi_ij C_j - (beta/eps0/L^3) tau_i F s  (hnc3d.c:1245-1268)
-        const T tau = gld(at32(tau3 + i * g.K, kk)) * T(g.tau_scale);
+        const T tau = gld(at32(taut + i * tsite, kk)) * T(g.tau_scale);
         out[i] = csub(cscale(acc, T(g.a_scale)), cscale(fs, tau));
       } else {
         out[i] = cscale(csub(acc, cscale(uc, T(g.beta * g.q[i]))), T(g.inv_L3));
@@ -1218,15 +1232,19 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
   }
 }
 
-// ------------------------------- 1' and 5'. the xy-plane pair (FP32)
-// The FP32 residual in three launches: closure_r2c_xy, zstar, c2r_xy_resid.
+// ----------------------------------- 1' and 5'. the xy-plane pair
+// The residual in three launches: closure_r2c_xy, zstar, c2r_xy_resid.
 // A workgroup owns one z plane of one site of one solute: N1 rows of N0
 // points, whose half spectrum (N1 rows of N0/2 + 1 bins, 66.5 KB in FP32
 // at 128^2) stays in LDS between the x and the y transforms, so the y pass
 // of the five-launch chain costs no HBM traffic.  Rows of the plane are at
 // stride LS = N0/2 + 1 in LDS; the row FFTs run on the first N0/2 points of
 // each row, the column FFTs on all N0/2 + 1 columns.
-constexpr int NTP = 512;  // threads of a plane workgroup
+// Threads of a plane workgroup.
+template <typename T, int N0, int N1>
+constexpr int plane_threads() {
+  return 512;
+}
 
 // t, c = closure(beta v, t) as closure_r2c_x over the plane, the N0-point
 // r2c of every row (N0/2-point FFT of z_n = c_2n + i c_2n+1 and the split,
@@ -1234,9 +1252,10 @@ constexpr int NTP = 512;  // threads of a plane workgroup
 // every kx column along y; the plane's rows [y][kx] go to W.
 // Grid: x = z plane (N2), y = site, z = solute.
 template <typename T, int N0, int N1, int H>
-__global__ void __launch_bounds__(NTP)
+__global__ void __launch_bounds__((plane_threads<T, N0, N1>()))
 closure_r2c_xy(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ tw_half,
                const cpx<T>* __restrict__ tw_full, const cpx<T>* __restrict__ tw_y) {
+  constexpr int NTP = plane_threads<T, N0, N1>();
   constexpr int M = N0 / 2, LS = M + 1, PLANE = N0 * N1, HP = M / 2 + 1;
   constexpr int VW = Vec16<T>::W;
   static_assert(PLANE % VW == 0, "whole vectors");
@@ -1308,9 +1327,10 @@ closure_r2c_xy(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __re
 // sum r^2, <r, r_j> as c2r_x_resid, one partial per plane and quantity at
 // part[q * m N2 + site * N2 + z].  Grid as closure_r2c_xy.
 template <typename T, int N0, int N1, int H>
-__global__ void __launch_bounds__(NTP)
+__global__ void __launch_bounds__((plane_threads<T, N0, N1>()))
 c2r_xy_resid(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ tw_half,
              const cpx<T>* __restrict__ tw_full, const cpx<T>* __restrict__ tw_y) {
+  constexpr int NTP = plane_threads<T, N0, N1>();
   constexpr int M = N0 / 2, LS = M + 1, PLANE = N0 * N1, HP = M / 2 + 1;
   constexpr int VW = Vec16<T>::W;
   static_assert(PLANE % VW == 0, "whole vectors");

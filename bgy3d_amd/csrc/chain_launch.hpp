@@ -44,16 +44,22 @@ inline bool use_zreg(const GridArgs& g) {
                        (g.special == 1 && g.msol <= 3));
 }
 
-// The FP32 residual on xy planes (closure_r2c_xy, zstar, c2r_xy_resid:
-// three launches, the y transforms inside the plane kernels) when the
-// planes are square with 64, 96 or 128 points per side; otherwise, and in
-// FP64 (a 128^2 plane would take 133 KB of LDS), the five-launch chain.
-// RISM3D_PLANES=0 keeps the five-launch chain in FP32 too.  The plane
-// kernels write W y-major with the Nyquist column apart (GridArgs::ylay),
-// which only zstar_reg reads (3 or 5 solvent sites).
-inline bool use_planes(const GridArgs& g, bool fp32, int on) {
-  return on && fp32 && g.special == 0 && g.N0 == g.N1 &&
-         (g.N0 == 64 || g.N0 == 96 || g.N0 == 128) && use_zreg(g);
+// The residual of B solutes on xy planes (closure_r2c_xy, zstar,
+// c2r_xy_resid: three launches, the y transforms inside the plane kernels)
+// when the planes are square, otherwise (and with RISM3D_PLANES=0) the
+// five-launch chain.  FP32: 64, 96 or 128 points per side.  FP64: up to 64
+// points always; planes of 96 and 128 points take 75 and 133 KB of LDS, two
+// and one workgroup per CU, and need about four workgroups per CU to fill
+// the chip (us per FP64 pass, rows against planes: 32^3 47 and 30, 64^3 72
+// and 59, 24 x 64^3 1006 and 841; 96^3 157 and 164 for one solute, 519 and
+// 483 for 4, 3355 and 2820 for 24; 128^3 339 and 358, 1188 and 1138, 7932
+// and 6855).  The plane kernels write W y-major with the Nyquist column
+// apart (GridArgs::ylay), which only zstar_reg reads.
+inline bool use_planes(const GridArgs& g, int B, bool fp32, int on) {
+  if (!on || g.N0 != g.N1 || !use_zreg(g)) return false;
+  if (fp32) return g.N0 == 64 || g.N0 == 96 || g.N0 == 128;
+  if (g.N0 <= 64) return true;
+  return (g.N0 == 96 || g.N0 == 128) && (int64_t)g.m * g.N2 * B >= 1024;
 }
 
 template <typename T>

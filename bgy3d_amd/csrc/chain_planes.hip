@@ -11,9 +11,9 @@ template <typename T, int N, int H>
 void launch_planes_h(bool inv, dim3 grid, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
                      const cpx<T>* twh, const cpx<T>* twf, const cpx<T>* twy) {
   if (inv)
-    hipLaunchKernelGGL((c2r_xy_resid<T, N, N, H>), grid, dim3(NTP), 0, s, sd, g, twh, twf, twy);
+    hipLaunchKernelGGL((c2r_xy_resid<T, N, N, H>), grid, dim3((plane_threads<T, N, N>())), 0, s, sd, g, twh, twf, twy);
   else
-    hipLaunchKernelGGL((closure_r2c_xy<T, N, N, H>), grid, dim3(NTP), 0, s, sd, g, twh, twf, twy);
+    hipLaunchKernelGGL((closure_r2c_xy<T, N, N, H>), grid, dim3((plane_threads<T, N, N>())), 0, s, sd, g, twh, twf, twy);
 }
 template <typename T, int N>
 void launch_planes_n(bool inv, dim3 grid, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
@@ -27,6 +27,10 @@ template <typename T>
 void launch_planes(bool inv, int B, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
                    const cpx<T>* twh, const cpx<T>* twf, const cpx<T>* twy, int hist) {
   const dim3 grid(g.N2, g.m, B);
+  if constexpr (sizeof(T) == 8) {
+    if (g.N0 == 32) return launch_planes_n<T, 32>(inv, grid, s, sd, g, twh, twf, twy, hist);
+    if (g.N0 == 48) return launch_planes_n<T, 48>(inv, grid, s, sd, g, twh, twf, twy, hist);
+  }
   switch (g.N0) {
     case 64: launch_planes_n<T, 64>(inv, grid, s, sd, g, twh, twf, twy, hist); break;
     case 96: launch_planes_n<T, 96>(inv, grid, s, sd, g, twh, twf, twy, hist); break;

@@ -31,7 +31,7 @@ void launch_zreg_n(int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd, c
   // 1.08 ms per pass at 64 x 128^3.  In FP64 in rows, and in the y passes,
   // that cost more than the tile it replaced.  RISM3D_NYQ=0 keeps it in the
   // last tile (g.nyq).
-  const bool split = g.nyq && sizeof(T) == 4 && NX > 1 && (NX - 1) % L == 0;
+  const bool split = g.nyq && (sizeof(T) == 4 || g.ylay) && NX > 1 && (NX - 1) % L == 0;
   if (g.ylay && !split) {  // evaluate forces the split for the plane chain
     std::fprintf(stderr, "rism3d: y-major spectra need the Nyquist launch\n");
     throw HipFailure{hipErrorInvalidValue};

@@ -78,6 +78,19 @@ ktab3(GridArgs g, const double* __restrict__ chi_tab, const double* __restrict__
   }
 }
 
+// The Nyquist column kx = N0/2 of n tables [n][K] once more behind them,
+// [n][N2][N1], as the z pass's Nyquist blocks read it.  Grid: x = chunks of
+// N1 N2, y = table.
+template <typename T>
+__global__ void __launch_bounds__(NT)
+nyq_tables(GridArgs g, T* __restrict__ tab) {
+  const int64_t n12 = (int64_t)g.N1 * g.N2;
+  const T* src = tab + blockIdx.y * g.K + (g.NX - 1);
+  T* dst = tab + gridDim.y * g.K + blockIdx.y * n12;
+  for (int64_t j = blockIdx.x * (int64_t)NT + threadIdx.x; j < n12; j += (int64_t)gridDim.x * NT)
+    dst[j] = src[j * g.NH];
+}
+
 // Fixed-order reduction of the residual-workgroup partials of each solute.
 // Grid: x = quantity (2 + the history width of the pass at least), y =
 // solute.  out[b * NPART + q]: max|r|, ||r||^2, <r, r_j>.  One workgroup per
@@ -675,6 +688,7 @@ form_factor(const SitesDesc* __restrict__ sites, GridArgs g, cpx<double>* const*
     }
     const double sign = ((x + iy + iz) & 1) ? -1.0 : 1.0;
     fs64[blockIdx.y][e] = cpx<double>{sign * re, sign * im};
+    if (x == g.NX - 1) fs64[blockIdx.y][g.K + (int64_t)z * g.N1 + y] = cpx<double>{sign * re, sign * im};
     if (fs32)
       fs32[blockIdx.y][fs_index<float>(g, z, y, x)] =
           cpx<float>{(float)(sign * re), (float)(sign * im)};

@@ -413,7 +413,7 @@ struct Problem {
   DevBuf<double> d_out;                 // B * NPART
   DevBuf<void*> d_cdst, d_csrc;         // precision hand-over copies
   DevBuf<int> d_cmask;
-  int nparts = 0;
+  int nparts = 0;  // partials per quantity: workgroups of the residual kernel at most
   std::vector<SoluteState> st;
   PinnedRing up;    // descriptor uploads
   PinnedRing down;  // norms and Gram rows
@@ -459,11 +459,11 @@ struct Problem {
   // ([0] FP64, [1] FP32): defaults from the environment, or the autotuner's
   // choice (tune)
   struct Knobs {
-    int planes;  // FP32 chain on xy planes (use_planes)
+    int planes;  // chain on xy planes (use_planes)
     int zorder;  // z-pass block order (zstar_reg)
     int zwide;   // z-pass tile of 32 kx columns over 512 threads (FP32)
     int nyq;     // Nyquist column in a launch of its own (FP32)
-  } knob[2] = {{0, env_int("RISM3D_ZSTAR_ORDER", 3), 0, 0},
+  } knob[2] = {{env_int("RISM3D_PLANES", 1), env_int("RISM3D_ZSTAR_ORDER", 3), 0, 0},
                {env_int("RISM3D_PLANES", 1), env_int("RISM3D_ZSTAR_ORDER", 3),
                 env_int("RISM3D_ZSTAR_WIDE", 0), env_int("RISM3D_NYQ", 1)}};
   int noalloc = 0;  // buffers from the fixed scratch: no pinned staging, no graphs
@@ -515,6 +515,13 @@ int resid_grid_x(const GridArgs& g) {
   return (g.N1 * g.N2 + rows - 1) / rows;
 }
 
+// Points of a spectrum or table with the Nyquist column apart: the rows and
+// that column, compact.
+int64_t w_points(const GridArgs& g) { return g.K + (int64_t)g.N1 * g.N2; }
+dim3 nyq_grid(const GridArgs& g, int tables) {
+  return dim3((unsigned)std::min<int64_t>(1024, ((int64_t)g.N1 * g.N2 + NT - 1) / NT), tables);
+}
+
 // History slots the closure and residual kernels must unroll for this batch.
 int hist_of(const std::vector<SoluteDesc>& sd) {
   int h = 0;
@@ -550,7 +557,7 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
     if (pf.on) HIPCHK(hipEventRecord(pf.ev[k][which], pb.s));
   };
   const int hist = step ? hist2 : hist_of(sd);
-  const bool planes = use_planes(g, fp32, kn.planes);
+  const bool planes = use_planes(g, pb.B, fp32, kn.planes);
   if (planes) {
     // y-major spectra, the Nyquist column in the z pass's launch of its
     // own (32-column tiles only where they end at it)
@@ -560,11 +567,16 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
   }
   const int nparts = planes ? g.m * g.N2 : resid_grid_x(g) * g.m;  // partials per quantity
   auto chain = [&]() {
-    if (planes) {
+    if (planes && fp32) {
       using T = float;
       mark(0, 0); launch_planes<T>(false, pb.B, pb.s, dsd, g, pb.tw.f[1].p, pb.tw.f[0].p, pb.tw.f[2].p, hist); mark(0, 1);
       mark(2, 0); launch_zstar<T>(g.N2, g.NX, g.N1, pb.B, pb.s, dsd, g, pb.tw.f[3].p, pb.chi3f.p, pb.tau3f.p); mark(2, 1);
       mark(4, 0); launch_planes<T>(true, pb.B, pb.s, dsd, g, pb.tw.f[1].p, pb.tw.f[0].p, pb.tw.f[2].p, hist); mark(4, 1);
+    } else if (planes) {
+      using T = double;
+      mark(0, 0); launch_planes<T>(false, pb.B, pb.s, dsd, g, pb.tw.d[1].p, pb.tw.d[0].p, pb.tw.d[2].p, hist); mark(0, 1);
+      mark(2, 0); launch_zstar<T>(g.N2, g.NX, g.N1, pb.B, pb.s, dsd, g, pb.tw.d[3].p, pb.chi3.p, pb.tau3.p); mark(2, 1);
+      mark(4, 0); launch_planes<T>(true, pb.B, pb.s, dsd, g, pb.tw.d[1].p, pb.tw.d[0].p, pb.tw.d[2].p, hist); mark(4, 1);
     } else if (fp32) {
       using T = float;
       constexpr int LN = y_lines<T>();
@@ -696,16 +708,18 @@ void tune(Problem& pb, bool fp32, int verbose) {
     }
   }
   std::vector<Problem::Knobs> cand{pb.knob[fp32 ? 1 : 0]};  // the built-in one first
-  const bool can_planes = fp32 && use_planes(g0, true, 1);
+  const bool can_planes = !fp32 || use_planes(g0, pb.B, true, 1);
   const bool can_wide = fp32 && g0.N2 <= 128 && use_zreg(g0);
   for (int planes : {1, 0})
     for (int zorder : {3, 2, 1})
       for (int zwide : {0, 1})
         for (int nyq : {1, 0}) {
           if ((planes && !can_planes) || (zwide && !can_wide) || (!fp32 && (nyq || zwide)) ||
-              (planes && !nyq))  // the plane chain always splits the Nyquist column off
+              (planes && !nyq && fp32))  // the plane chain always splits the Nyquist column off
             continue;
           const Problem::Knobs& d0 = cand[0];
+          // FP64 keeps its rounding: the planes as built in
+          if (!fp32 && planes != d0.planes) continue;
           if (planes == d0.planes && zorder == d0.zorder && zwide == d0.zwide && nyq == d0.nyq)
             continue;
           cand.push_back({planes, zorder, zwide, nyq});
@@ -2142,7 +2156,7 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
   make_twiddles(pb.tw, pb.N, pb.s);
 
   // omega_ij(k) in the chi3 slots of the pairs
-  pb.chi3 = DevBuf<double>((size_t)np * g.K);
+  pb.chi3 = DevBuf<double>((size_t)np * w_points(g));
   {
     std::vector<double> rij(np, 0.0);
     for (int i = 0; i < m; ++i)
@@ -2155,16 +2169,17 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
     HIPCHK(hipMemcpy(d_rij.p, rij.data(), np * 8, hipMemcpyHostToDevice));
     const int ck = (int)std::min<int64_t>(4096, (g.K + NT - 1) / NT);
     hipLaunchKernelGGL(omega3, dim3(ck, np), dim3(NT), 0, pb.s, g, pd->L[0], d_rij.p, pb.chi3.p);
+    hipLaunchKernelGGL(nyq_tables<double>, nyq_grid(g, np), dim3(NT), 0, pb.s, g, pb.chi3.p);
     HIPCHK(hipStreamSynchronize(pb.s));
   }
   pb.st.resize(1);
-  pb.nparts = resid_grid_x(g) * np;
+  pb.nparts = np * std::max(resid_grid_x(g), g.N2);
   auto& s0 = pb.st[0];
   s0.U = DevBuf<double>((size_t)pb.D * pb.mP);
   s0.R = DevBuf<double>((size_t)pb.D * pb.mP);
   s0.t64 = DevBuf<double>(pb.mP);
   s0.bv64 = DevBuf<double>(pb.mP);
-  s0.W = DevBuf<cpx<double>>((size_t)np * g.K);
+  s0.W = DevBuf<cpx<double>>((size_t)np * w_points(g));
   s0.part = DevBuf<double>((size_t)pb.nparts * NPART);
   pb.d_sd = DevBuf<SoluteDesc>(1);
   pb.d_out = DevBuf<double>(NPART);
@@ -2353,17 +2368,17 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
     // --solvent-3d: chi - 1 of a 3D solvent solve on this grid
     // (solvent_kernel_file, hnc3d.c:1434-1437, 1572-1590), no tau
     const size_t np = (size_t)m * (m + 1) / 2;
-    pb.chi3 = DevBuf<double>(np * g.K);
-    pb.chi3f = DevBuf<float>(np * g.K);
-    pb.tau3 = DevBuf<double>((size_t)m * g.K);
-    pb.tau3f = DevBuf<float>((size_t)m * g.K);
+    pb.chi3 = DevBuf<double>(np * w_points(g));
+    pb.chi3f = DevBuf<float>(np * w_points(g));
+    pb.tau3 = DevBuf<double>((size_t)m * w_points(g));
+    pb.tau3f = DevBuf<float>((size_t)m * w_points(g));
     HIPCHK(hipMemcpy2DAsync(pb.chi3.p, g.NH * 8, in.opt.chi3d, g.NX * 8, g.NX * 8,
                             np * g.N1 * g.N2, hipMemcpyHostToDevice, pb.s));
     const int ck = (int)std::min<int64_t>(4096, (np * g.K + NT - 1) / NT);
     hipLaunchKernelGGL(to_f32, dim3(ck), dim3(NT), 0, pb.s, pb.chi3f.p, pb.chi3.p,
                        (int64_t)(np * g.K));
-    HIPCHK(hipMemsetAsync(pb.tau3.p, 0, (size_t)m * g.K * 8, pb.s));
-    HIPCHK(hipMemsetAsync(pb.tau3f.p, 0, (size_t)m * g.K * 4, pb.s));
+    HIPCHK(hipMemsetAsync(pb.tau3.p, 0, pb.tau3.n * 8, pb.s));
+    HIPCHK(hipMemsetAsync(pb.tau3f.p, 0, pb.tau3f.n * 4, pb.s));
   } else {
   std::vector<double> chi_tab((size_t)m * (m + 1) / 2 * nrad), tau_tab((size_t)m * nrad);
   for (int i = 0; i < m; ++i)
@@ -2386,21 +2401,25 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
   HIPCHK(hipMemcpyAsync(pb.tau_tab.p, tau_tab.data(), tau_tab.size() * 8, hipMemcpyHostToDevice, pb.s));
   {
     const size_t np = (size_t)m * (m + 1) / 2;
-    pb.chi3 = DevBuf<double>(np * g.K);
-    pb.chi3f = DevBuf<float>(np * g.K);
-    pb.tau3 = DevBuf<double>((size_t)m * g.K);
-    pb.tau3f = DevBuf<float>((size_t)m * g.K);
+    pb.chi3 = DevBuf<double>(np * w_points(g));
+    pb.chi3f = DevBuf<float>(np * w_points(g));
+    pb.tau3 = DevBuf<double>((size_t)m * w_points(g));
+    pb.tau3f = DevBuf<float>((size_t)m * w_points(g));
     const int ck = (int)std::min<int64_t>(4096, (g.K + NT - 1) / NT);
     hipLaunchKernelGGL(ktab3, dim3(ck), dim3(NT), 0, pb.s, g, pb.chi_tab.p, pb.tau_tab.p,
                        pb.chi3.p, pb.chi3f.p, pb.tau3.p, pb.tau3f.p);
+    hipLaunchKernelGGL(nyq_tables<double>, nyq_grid(g, m), dim3(NT), 0, pb.s, g, pb.tau3.p);
+    hipLaunchKernelGGL(nyq_tables<float>, nyq_grid(g, m), dim3(NT), 0, pb.s, g, pb.tau3f.p);
   }
   }
+  hipLaunchKernelGGL(nyq_tables<double>, nyq_grid(g, m * (m + 1) / 2), dim3(NT), 0, pb.s, g, pb.chi3.p);
+  hipLaunchKernelGGL(nyq_tables<float>, nyq_grid(g, m * (m + 1) / 2), dim3(NT), 0, pb.s, g, pb.chi3f.p);
 
   // per-solute buffers
   const int B = in.B;
   pb.st.resize(B);
-  pb.nparts = resid_grid_x(g) * m;
-  const int64_t mK = (int64_t)m * g.K;
+  pb.nparts = m * std::max(resid_grid_x(g), g.N2);
+  const int64_t mK = (int64_t)m * w_points(g);
   std::vector<SitesDesc> sites(B);
   std::vector<double*> bv64p(B), tp(B), gp(B);
   std::vector<float*> bv32p(B);
@@ -2421,8 +2440,8 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
       s.t32b = DevBuf<float>(pb.mP);
     }
     s.W = DevBuf<cpx<double>>(mK);
-    s.fs64 = DevBuf<cpx<double>>(g.K);
-    if (pb.mixed) s.fs32 = DevBuf<cpx<float>>(g.K + (int64_t)g.N1 * g.N2);  // fs_index
+    s.fs64 = DevBuf<cpx<double>>(w_points(g));
+    if (pb.mixed) s.fs32 = DevBuf<cpx<float>>(w_points(g));  // fs_index
     s.part = DevBuf<double>((size_t)pb.nparts * NPART);
     s.n_sites = in.n_sites[b];
     auto& sh = site_host[b];
@@ -2759,9 +2778,10 @@ size_t noalloc_bytes(const rism3d_problem& pd, int m, int n, bool mixed) {
   size_t b = 0;
   for (size_t len : {N0, N0 / 2, N1, N2}) b += al(len * 16) + al(len * 8);  // twiddles
   b += al(np * nrad * 8) + al(m * nrad * 8);                       // 1D tables
-  b += al(np * K * 8) + al(np * K * 4) + al(m * K * 8) + al(m * K * 4);  // 3D tables
-  b += 4 * al(mP * 8) + al(m * K * 16) + al(K * 16);  // U, R, t, beta v; W; F s
-  if (mixed) b += 4 * al(mP * 4) + al(mP * 8) + al((K + N1 * N2) * 8);
+  const size_t Kw = K + N1 * N2;  // with the Nyquist column apart
+  b += al(np * Kw * 8) + al(np * Kw * 4) + al(m * Kw * 8) + al(m * Kw * 4);  // 3D tables
+  b += 4 * al(mP * 8) + al(m * Kw * 16) + al(Kw * 16);  // U, R, t, beta v; W; F s
+  if (mixed) b += 4 * al(mP * 4) + al(mP * 8) + al(Kw * 8);
   b += al(N1 * N2 * m * NPART * 8) + al((size_t)std::max(n, 0) * 6 * 8);
   b += al(sizeof(SoluteDesc)) + al(sizeof(SitesDesc)) + al(NPART * 8) + 3 * al(8);
   b += al(3 * (size_t)m * 8) + 4 * al(8);  // setup descriptors
