@@ -1040,15 +1040,6 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
   const cpx<T>* W = static_cast<const cpx<T>*>(d.W) + site * g.K + (int64_t)row0 * g.NH;
   const int64_t off = site * g.P + (int64_t)row0 * N0;
   constexpr int VW = Vec16<T>::W;
-  // FP32 defect-correction passes over whole tiles: the streams this
-  // thread reads after the inverse FFT (t, F(t_b), the BF16 residual
-  // history) are loaded together with the spectrum, so those loads overlap
-  // the FFT instead of following it.  ITP vectors per thread.
-  constexpr int ITP = (ROWS * N0) / (NT * VW);
-  constexpr bool PREF = sizeof(T) == 4 && ITP * NT * VW == ROWS * N0 && ITP <= 2;
-  const bool pref = PREF && (d.r16 != 0 || d.r8 != 0) && d.mode == 5 && vrows == ROWS;
-  Vec16<T> ptv[PREF ? ITP : 1], pfb[PREF ? ITP : 1];
-  BF4 prh[PREF ? ITP : 1][H];
   {
     // all loads first; rows past the last one read the last row's address
     // and are zeroed
@@ -1061,19 +1052,6 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
         const int row = e / (M + 1);
         const int k = e - row * (M + 1);
         v[p] = ldc(W + min(row, vrows - 1) * g.NH + k);
-      }
-    }
-    if constexpr (PREF) {
-      if (pref) {
-#pragma unroll
-        for (int it = 0; it < ITP; ++it) {
-          const int64_t e = off + threadIdx.x * VW + it * NT * VW;
-          ptv[it] = ld16(static_cast<const T*>(d.t) + e);
-          pfb[it] = ld16(static_cast<const T*>(d.fb) + e);
-#pragma unroll
-          for (int j = 0; j < H; ++j)
-            if (j < d.ndot) prh[it][j] = ld_hist(d, d.rh[j], e);
-        }
       }
     }
 #pragma unroll
@@ -1107,8 +1085,12 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
 #pragma unroll
   for (int j = 0; j < H; ++j) dot[j] = 0.0;
   const int mode = d.mode;
-  // one vector of VW points at e: t, F(t_b) (mode 5) and the history rh
-  auto point = [&](int e, const Vec16<T>& tv, const Vec16<T>& f, const Vec16<T>* rh) {
+  // one vector of VW points at e: t, F(t_b) (mode 5) and the history r_j
+  // (rhj(j), unpacked on use)
+  auto point = [&](int e, const Vec16<T>& tv, const Vec16<T>& f, auto&& rhj) {
+    Vec16<T> uo;  // u16: the u the new one replaces (loaded first, used last)
+    if constexpr (sizeof(T) == 4)
+      if (d.u16 && un) uo = ld16(un + e);
     Vec16<T> z;  // t' at points e.. of row e / N0: z_n = t'_{2n} + i t'_{2n+1}
     {
       const cpx<T>* zrow = zb + (e / N0) * LSM;
@@ -1138,7 +1120,6 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
     if (un) {
       if constexpr (sizeof(T) == 4) {
         if (d.u16) {  // the difference from the u it replaces, in BF16
-          const Vec16<T> uo = ld16(un + e);
           Vec16<T> du;
 #pragma unroll
           for (int k = 0; k < VW; ++k) du.v[k] = uv.v[k] - uo.v[k];
@@ -1166,28 +1147,41 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
 #pragma unroll
       for (int j = 0; j < H; ++j)
         if (j < nd) {
+          const Vec16<T> x = rhj(j);
           T pj = T(0);
 #pragma unroll
-          for (int k = 0; k < VW; ++k) pj += rv.v[k] * rh[j].v[k];
+          for (int k = 0; k < VW; ++k) pj += rv.v[k] * x.v[k];
           dot[j] += (double)pj;
         }
     }
   };
-  auto unbf = [&](int j, BF4 q) {
-    Vec16<T> x;
-    if constexpr (sizeof(T) == 4) x = un_hist(d, j, q);
-    return x;
-  };
   bool done = false;
-  if constexpr (PREF) {
-    if (pref) {
+  if constexpr (sizeof(T) == 4) {
+    if (r16) {
+      // the FP32 phase, bound by its 30 bytes of streams per point: two
+      // vectors per step, their streams in flight together, the history
+      // kept packed (88 VGPRs at 8 slots, 5 waves per SIMD).  Loading the
+      // streams before the inverse FFT held 139 and, at N0 = 3 2^k, ran out
+      // of threads: 377 us at 192^3 with 5 sites, this way 246 (4.3 TB/s).
+      for (int e0 = threadIdx.x * VW; e0 < vrows * N0; e0 += 2 * NT * VW) {
+        Vec16<T> tv[2], f[2];
+        BF4 rb[2][H];
 #pragma unroll
-      for (int it = 0; it < ITP; ++it) {
-        Vec16<T> rh[H];
+        for (int q = 0; q < 2; ++q) {
+          const int e = e0 + q * NT * VW;
+          if (e >= vrows * N0) continue;
+          tv[q] = ld16(t + e);
+          if (mode == 5) f[q] = ld16(static_cast<const T*>(d.fb) + off + e);
 #pragma unroll
-        for (int j = 0; j < H; ++j)
-          if (j < nd) rh[j] = unbf(j, prh[it][j]);
-        point(threadIdx.x * VW + it * NT * VW, ptv[it], pfb[it], rh);
+          for (int j = 0; j < H; ++j)
+            if (j < nd) rb[q][j] = ld_hist(d, d.rh[j], off + e);
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int e = e0 + q * NT * VW;
+          if (e >= vrows * N0) continue;
+          point(e, tv[q], f[q], [&](int j) { return un_hist(d, j, rb[q][j]); });
+        }
       }
       done = true;
     }
@@ -1200,16 +1194,8 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
       Vec16<T> rh[H];
 #pragma unroll
       for (int j = 0; j < H; ++j)
-        if (j < nd) {
-          if constexpr (sizeof(T) == 4) {
-            if (r16) {
-              rh[j] = unbf(j, ld_hist(d, d.rh[j], off + e));
-              continue;
-            }
-          }
-          rh[j] = ld16(static_cast<const T*>(d.rh[j]) + off + e);
-        }
-      point(e, tv, f, rh);
+        if (j < nd) rh[j] = ld16(static_cast<const T*>(d.rh[j]) + off + e);
+      point(e, tv, f, [&](int j) { return rh[j]; });
     }
   }
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
