@@ -834,7 +834,8 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
   const T* chit = nyq ? chi3 + NTAB * g.K : chi3;
   const T* taut = nyq ? tau3 + MS * g.K : tau3;
   const int tbase = nyq ? y : base, tz = nyq ? g.N1 : zs;
-  const int nl = nyq ? min(LINES, g.N1 - y) : min(LINES, g.NX - kx0);  // valid lines
+  const int nl = nyq ? min(LINES, g.N1 - y)  // valid lines
+                     : min(LINES, (g.nyqb ? g.NX - 1 : g.NX) - kx0);
   const int tid = threadIdx.x;
   cpx<T> c[MS][PPT];
   // every site's loads first, staged in its registers of c (its FFT result
@@ -1226,10 +1227,13 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
 // of the five-launch chain costs no HBM traffic.  Rows of the plane are at
 // stride LS = N0/2 + 1 in LDS; the row FFTs run on the first N0/2 points of
 // each row, the column FFTs on all N0/2 + 1 columns.
-// Threads of a plane workgroup.
+// Threads of a plane workgroup: two or more vectors each, so that a small
+// plane's workgroup leaves room for others (24 x 48^3 in FP32 208 us per pass
+// with 512 threads, 184 with 256; 24 x 32^3 84 and 61 with 128).
 template <typename T, int N0, int N1>
 constexpr int plane_threads() {
-  return 512;
+  constexpr int vectors = N0 * N1 * (int)sizeof(T) / 16;
+  return vectors >= 1024 ? 512 : vectors >= 512 ? 256 : 128;
 }
 
 // t, c = closure(beta v, t) as closure_r2c_x over the plane, the N0-point

@@ -47,7 +47,10 @@ inline bool use_zreg(const GridArgs& g) {
 // The residual of B solutes on xy planes (closure_r2c_xy, zstar,
 // c2r_xy_resid: three launches, the y transforms inside the plane kernels)
 // when the planes are square, otherwise (and with RISM3D_PLANES=0) the
-// five-launch chain.  FP32: 64, 96 or 128 points per side.  FP64: up to 64
+// five-launch chain.  FP32: up to 128 points per side, at 48 from four solutes
+// on (us per pass, rows against planes: 48^3 50 and 48 but 68 and 72 with the
+// host's part for one solute, 195 and 184 for 24; 32^3 48 and 37, 86 and 61;
+// 192^2 planes would fill a CU's LDS: 800 and 800, 481 and 552).  FP64: up to 64
 // points always; planes of 96 and 128 points take 75 and 133 KB of LDS, two
 // and one workgroup per CU, and need about four workgroups per CU to fill
 // the chip (us per FP64 pass, rows against planes: 32^3 47 and 30, 64^3 72
@@ -57,7 +60,9 @@ inline bool use_zreg(const GridArgs& g) {
 // apart (GridArgs::ylay), which only zstar_reg reads.
 inline bool use_planes(const GridArgs& g, int B, bool fp32, int on) {
   if (!on || g.N0 != g.N1 || !use_zreg(g)) return false;
-  if (fp32) return g.N0 == 64 || g.N0 == 96 || g.N0 == 128;
+  if (fp32)
+    return g.N0 == 32 || g.N0 == 64 || g.N0 == 96 || g.N0 == 128 ||
+           (g.N0 == 48 && (int64_t)g.m * g.N2 * B >= 512);
   if (g.N0 <= 64) return true;
   return (g.N0 == 96 || g.N0 == 128) && (int64_t)g.m * g.N2 * B >= 1024;
 }

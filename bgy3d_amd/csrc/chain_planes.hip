@@ -27,11 +27,9 @@ template <typename T>
 void launch_planes(bool inv, int B, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
                    const cpx<T>* twh, const cpx<T>* twf, const cpx<T>* twy, int hist) {
   const dim3 grid(g.N2, g.m, B);
-  if constexpr (sizeof(T) == 8) {
-    if (g.N0 == 32) return launch_planes_n<T, 32>(inv, grid, s, sd, g, twh, twf, twy, hist);
-    if (g.N0 == 48) return launch_planes_n<T, 48>(inv, grid, s, sd, g, twh, twf, twy, hist);
-  }
   switch (g.N0) {
+    case 32: launch_planes_n<T, 32>(inv, grid, s, sd, g, twh, twf, twy, hist); break;
+    case 48: launch_planes_n<T, 48>(inv, grid, s, sd, g, twh, twf, twy, hist); break;
     case 64: launch_planes_n<T, 64>(inv, grid, s, sd, g, twh, twf, twy, hist); break;
     case 96: launch_planes_n<T, 96>(inv, grid, s, sd, g, twh, twf, twy, hist); break;
     case 128: launch_planes_n<T, 128>(inv, grid, s, sd, g, twh, twf, twy, hist); break;

@@ -1,6 +1,4 @@
 // The z pass of the residual chain.
-#include <cstdio>
-
 #include "chain_launch.hpp"
 
 #ifndef RISM_T
@@ -30,13 +28,9 @@ void launch_zreg_n(int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd, c
   // tile that holds it alone (one workgroup in five at N0 = 128): 1.19 ->
   // 1.08 ms per pass at 64 x 128^3.  In FP64 in rows, and in the y passes,
   // that cost more than the tile it replaced.  RISM3D_NYQ=0 keeps it in the
-  // last tile (g.nyq).
-  const bool split = g.nyq && (sizeof(T) == 4 || g.ylay) && NX > 1 && (NX - 1) % L == 0;
-  if (g.ylay && !split) {  // evaluate forces the split for the plane chain
-    std::fprintf(stderr, "rism3d: y-major spectra need the Nyquist launch\n");
-    throw HipFailure{hipErrorInvalidValue};
-  }
-  const int tiles = split ? (NX - 1) / L : (NX + L - 1) / L;
+  // last tile (g.nyq).  Y-major spectra (g.ylay) always have it apart.
+  const bool split = g.ylay || (g.nyq && sizeof(T) == 4 && NX > 1 && (NX - 1) % L == 0);
+  const int tiles = (split ? NX - 1 + L - 1 : NX + L - 1) / L;
   GridArgs gz = g;
   if (gz.zorder == 2 && (tiles * N1) % 8 != 0) gz.zorder = 1;  // whole tiles per XCD
   if (gz.zorder == 3 && N1 % 8 != 0) gz.zorder = 1;             // whole rows per XCD
