@@ -93,7 +93,11 @@ nyq_tables(GridArgs g, T* __restrict__ tab) {
 
 // Fixed-order reduction of the residual-workgroup partials of each solute.
 // Grid: x = quantity (2 + the history width of the pass at least), y =
-// solute.  out[b * NPART + q]: max|r|, ||r||^2, <r, r_j>.  One workgroup per
+// solute.  out[b * NPART + q]: max|r|, ||r||^2, <r, r_j>; with hout instead
+// the bits of the value at hout[2 (b * NPART + q)] and those bits ^ the
+// solute's key behind them, in pinned host memory, where the host polls for
+// the pair (each word tells the other's arrival, so no order between the two
+// stores is needed, nor the end of the kernel).  One workgroup per
 // quantity, whose partials lie together: latency bound (a partial per
 // thread or a few), so the quantities run side by side and each thread keeps
 // four sums in flight.  One workgroup per solute over rows of NPART took
@@ -101,7 +105,8 @@ nyq_tables(GridArgs g, T* __restrict__ tab) {
 // 10% and 15% of a pass; this way 4.1 and 12.8 us.
 constexpr int NTR = 1024;
 __global__ void __launch_bounds__(NTR)
-reduce_resid(const SoluteDesc* __restrict__ sd, int nparts, double* __restrict__ out) {
+reduce_resid(const SoluteDesc* __restrict__ sd, int nparts, double* __restrict__ out,
+             uint64_t* __restrict__ hout) {
   __shared__ double red[NTR / 64];
   const SoluteDesc& d = sd[blockIdx.y];
   const int q = blockIdx.x;
@@ -125,8 +130,29 @@ reduce_resid(const SoluteDesc* __restrict__ sd, int nparts, double* __restrict__
   if (w == 0) {
     const double v = lane < NTR / 64 ? red[lane] : 0.0;
     const double r = q == 0 ? warp_max(v) : warp_sum(v);
-    if (lane == 0) out[blockIdx.y * NPART + q] = r;
+    if (lane == 0) {
+      const size_t i = (size_t)blockIdx.y * NPART + q;
+      if (hout) {
+        const uint64_t bits = (uint64_t)__double_as_longlong(r);
+        __hip_atomic_store(hout + 2 * i, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(hout + 2 * i + 1, bits ^ d.key, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+      } else {
+        out[i] = r;
+      }
+    }
   }
+}
+
+// The descriptors of a pass from pinned host memory to the device, as the
+// first kernel of the pass's graph.  Grid: x = solute.
+constexpr int NTL = 128;
+__global__ void __launch_bounds__(NTL)
+load_sd(const SoluteDesc* __restrict__ src, SoluteDesc* __restrict__ dst) {
+  constexpr int W = sizeof(SoluteDesc) / 8;
+  const uint64_t* s = reinterpret_cast<const uint64_t*>(src + blockIdx.x);
+  uint64_t* d = reinterpret_cast<uint64_t*>(dst + blockIdx.x);
+  for (int i = threadIdx.x; i < W; i += NTL) d[i] = s[i];
 }
 
 // v from lane `lane` (the same in every lane of the wavefront) to all lanes.

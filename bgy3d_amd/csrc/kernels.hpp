@@ -54,6 +54,8 @@ struct SoluteDesc {
                              //   BF16, each entry scaled into the e4m3 range
   float rsc;                 // r8: the new r is stored as r * rsc
   float rhinv[MAX_DIIS];     // r8: 1 / the scale of rh[j]
+  uint64_t key;              // of this pass, never 0, where the norms go to the
+                             //   host's memory (reduce_resid)
 };
 static_assert(sizeof(SoluteDesc) % 8 == 0, "SoluteDesc is copied in 8-byte words");
 constexpr int NPART = 2 + MAX_DIIS;   // doubles per residual workgroup

@@ -415,8 +415,24 @@ struct Problem {
   DevBuf<int> d_cmask;
   int nparts = 0;  // partials per quantity: workgroups of the residual kernel at most
   std::vector<SoluteState> st;
-  PinnedRing up;    // descriptor uploads
-  PinnedRing down;  // norms and Gram rows
+  PinnedRing up;    // descriptor uploads outside the chain's graphs
+  PinnedRing down;  // device MDIIS state
+  // A pass's traffic with the host, in pinned memory that the pass's own
+  // kernels read and write: load_sd takes the descriptors from sd and
+  // reduce_resid leaves the norms and Gram rows in out, which the host polls.
+  // A copy each way and a wait for the stream took 15 to 20 us more a pass
+  // (FP64, one solute: 50 -> 36 us at 32^3, 184 -> 165 us at 96^3).
+  struct PassIO {
+    SoluteDesc* sd = nullptr;
+    uint64_t* out = nullptr;  // [B][NPART][2]
+    uint64_t key = 0;         // of the last pass
+    bool open = false;        // a pass is launched whose results nobody took
+    std::vector<int> nq;      // its quantities per solute
+    ~PassIO() {
+      if (sd) (void)hipHostFree(sd);
+      if (out) (void)hipHostFree(out);
+    }
+  } io;
   // The residual chain (five kernels + the norm reduction) as HIP graphs,
   // one per working precision and history width, captured on first use and
   // replayed every iteration (the descriptors they read are uploaded
@@ -483,15 +499,41 @@ void upload_sd(Problem& pb, const std::vector<SoluteDesc>& sd, SoluteDesc* dst) 
   HIPCHK(hipMemcpyAsync(dst, h, bytes, hipMemcpyHostToDevice, pb.s));
   pb.up.mark(k, pb.s);
 }
-// pb.d_out to out[], synchronising the stream.
+// The norms and Gram rows of the pass just launched (evaluate) to out[].
 void download_out(Problem& pb, std::vector<double>& out) {
-  const size_t bytes = out.size() * sizeof(double);
-  int k = 0;
-  void* h = pb.down.slot(bytes, &k);
-  HIPCHK(hipMemcpyAsync(h, pb.d_out.p, bytes, hipMemcpyDeviceToHost, pb.s));
-  pb.down.mark(k, pb.s);
-  HIPCHK(hipStreamSynchronize(pb.s));
-  std::memcpy(out.data(), h, bytes);
+  if (pb.noalloc) {
+    HIPCHK(hipMemcpyAsync(out.data(), pb.d_out.p, out.size() * sizeof(double),
+                          hipMemcpyDeviceToHost, pb.s));
+    HIPCHK(hipStreamSynchronize(pb.s));
+    return;
+  }
+  auto& io = pb.io;
+  auto taken = [&](size_t i) {
+    const uint64_t v = __atomic_load_n(io.out + 2 * i, __ATOMIC_RELAXED);
+    const uint64_t w = __atomic_load_n(io.out + 2 * i + 1, __ATOMIC_RELAXED);
+    if ((v ^ w) != io.key) return false;
+    std::memcpy(&out[i], &v, 8);
+    return true;
+  };
+  long spin = 0;
+  bool ended = false;
+  for (int b = 0; b < pb.B; ++b)
+    for (int q = 0; q < io.nq[b]; ++q)
+      while (!taken((size_t)b * NPART + q)) {
+        // the stream is asked only now and then (a failed pass ends the wait
+        // within milliseconds): its lock is shared with the launches of other
+        // threads, such as the size classes of rism3d_batch_solve_grids
+        __builtin_ia32_pause();
+        if (++spin % 16384 != 0) continue;
+        if (ended) {
+          std::fprintf(stderr, "rism3d: the pass ended without its norms\n");
+          throw HipFailure{hipErrorUnknown};
+        }
+        const hipError_t e = hipStreamQuery(pb.s);
+        if (e == hipSuccess) ended = true;  // everything it wrote arrives by the next look
+        else if (e != hipErrorNotReady) HIPCHK(e);
+      }
+  io.open = false;
 }
 
 // Per-kernel HIP-event timing of the residual chain (rism3d_profile_*).
@@ -541,9 +583,26 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
   g.zwide = kn.zwide;
   g.nyq = kn.nyq;
   SoluteDesc* dsd = step ? pb.d_sd32.p : pb.d_sd.p;
+  const bool pinned = !step && !pb.noalloc;  // this pass's host traffic through pb.io
   Profile& pf = g_prof;
   std::vector<SoluteDesc> sdp;  // profiling, step 2: the descriptors on the device
-  if (!step) {
+  if (pinned) {
+    auto& io = pb.io;
+    if (!io.sd) {
+      HIPCHK(hipHostMalloc((void**)&io.sd, pb.B * sizeof(SoluteDesc), hipHostMallocCoherent));
+      HIPCHK(hipHostMalloc((void**)&io.out, (size_t)pb.B * NPART * 16, hipHostMallocCoherent));
+      std::memset(io.out, 0, (size_t)pb.B * NPART * 16);
+    }
+    if (io.open) HIPCHK(hipStreamSynchronize(pb.s));  // its load_sd may not have run yet
+    io.open = true;
+    io.key += 0x9E3779B97F4A7C15ull;  // odd: 0 again only after 2^64 passes
+    io.nq.assign(pb.B, 0);
+    for (int b = 0; b < pb.B; ++b) {
+      sd[b].key = io.key;
+      if (sd[b].active) io.nq[b] = 2 + sd[b].ndot;
+    }
+    std::memcpy(io.sd, sd.data(), sd.size() * sizeof(SoluteDesc));
+  } else if (!step) {
     upload_sd(pb, sd, dsd);
   } else if (pf.on) {
     sdp.resize(sd.size());
@@ -567,6 +626,8 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
   }
   const int nparts = planes ? g.m * g.N2 : resid_grid_x(g) * g.m;  // partials per quantity
   auto chain = [&]() {
+    if (pinned)
+      hipLaunchKernelGGL(load_sd, dim3(pb.B), dim3(NTL), 0, pb.s, (const SoluteDesc*)pb.io.sd, dsd);
     if (planes && fp32) {
       using T = float;
       mark(0, 0); launch_planes<T>(false, pb.B, pb.s, dsd, g, pb.tw.f[1].p, pb.tw.f[0].p, pb.tw.f[2].p, hist); mark(0, 1);
@@ -598,7 +659,8 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
     }
     // 2 + the history width this launch (or graph, captured per width) serves
     const int nq = 2 + (hist <= 8 ? 8 : (hist <= 10 ? 10 : MAX_DIIS));
-    hipLaunchKernelGGL(reduce_resid, dim3(nq, pb.B), dim3(NTR), 0, pb.s, dsd, nparts, pb.d_out.p);
+    hipLaunchKernelGGL(reduce_resid, dim3(nq, pb.B), dim3(NTR), 0, pb.s, dsd, nparts, pb.d_out.p,
+                       pinned ? pb.io.out : (uint64_t*)nullptr);
     if (step)
       hipLaunchKernelGGL(mdiis_step, dim3(pb.B), dim3(64), 0, pb.s, pb.d_out.p, pb.d_mdiis.p, dsd,
                          pb.h_status.p);
