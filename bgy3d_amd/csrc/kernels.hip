@@ -49,7 +49,7 @@ __device__ __forceinline__ double interp_eval(const Interp& a, const double* __r
 // chi_ij(|k|) - delta_ij and tau_i(|k|) on the 3D k grid, once per batch
 // (solute independent; solvent_kernel_rism hnc3d.c:1443-1566 tabulates
 // them the same way with vec_ktab).  Grid: x = chunks of K.  Writes FP64
-// and FP32 copies, [npairs][K] and [m][K].
+// and, unless null, FP32 copies, [npairs][K] and [m][K].
 __global__ void __launch_bounds__(NT)
 ktab3(GridArgs g, const double* __restrict__ chi_tab, const double* __restrict__ tau_tab,
       double* __restrict__ chi3, float* __restrict__ chi3f, double* __restrict__ tau3,
@@ -68,12 +68,12 @@ ktab3(GridArgs g, const double* __restrict__ chi_tab, const double* __restrict__
     for (int p = 0; p < np; ++p) {
       const double v = interp_eval(ip, chi_tab + (int64_t)p * g.nrad);
       chi3[p * g.K + e] = v;
-      chi3f[p * g.K + e] = (float)v;
+      if (chi3f) chi3f[p * g.K + e] = (float)v;
     }
     for (int i = 0; i < g.m; ++i) {
       const double v = interp_eval(ip, tau_tab + (int64_t)i * g.nrad);
       tau3[i * g.K + e] = v;
-      tau3f[i * g.K + e] = (float)v;
+      if (tau3f) tau3f[i * g.K + e] = (float)v;
     }
   }
 }

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -31,18 +32,20 @@
 // itself is not a device address on the host.
 static __device__ __align__(256) unsigned char scratch[(size_t)RISM3D_NOALLOC_SCRATCH_MB << 20];
 
-namespace rism {
-namespace {
-
 #define HIPCHK(x)                                                                        \
   do {                                                                                   \
     hipError_t e_ = (x);                                                                 \
     if (e_ != hipSuccess) {                                                              \
       std::fprintf(stderr, "rism3d: %s failed: %s (%s:%d)\n", #x, hipGetErrorString(e_), \
                    __FILE__, __LINE__);                                                  \
-      throw HipFailure{e_};                                                              \
+      throw rism::HipFailure{e_};                                                              \
     }                                                                                    \
   } while (0)
+
+#include "host_io.hpp"
+
+namespace rism {
+namespace {
 
 bool supported_n(int n) {
   switch (n) {
@@ -234,32 +237,34 @@ struct PinnedRing {
   }
 };
 
-template <typename T>
-std::vector<cpx<T>> twiddles(int n) {
-  std::vector<cpx<T>> w(n);
-  for (int j = 0; j < n; ++j) {
-    const long double a = -2.0L * 3.14159265358979323846264338327950288L * j / n;
-    w[j] = cpx<T>{(T)std::cos(a), (T)std::sin(a)};
-  }
-  return w;
-}
-
 struct Twiddles {
-  DevBuf<cpx<double>> d[4];  // N0, N0/2, N1, N2
-  DevBuf<cpx<float>> f[4];
+  struct { cpx<double>* p; } d[4];  // N0, N0/2, N1, N2
+  struct { cpx<float>* p; } f[4];
+  DevBuf<cpx<double>> own_d[4];     // the allocation-free path's, in its arena
+  DevBuf<cpx<float>> own_f[4];
 };
 
-void make_twiddles(Twiddles& tw, const int N[3], hipStream_t s) {
+void make_twiddles(Twiddles& tw, const int N[3], hipStream_t s, bool own) {
   const int len[4] = {N[0], N[0] / 2, N[1], N[2]};
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
   for (int i = 0; i < 4; ++i) {
+    if (!own) {
+      const auto t = twiddles_on(dev, len[i]);
+      tw.d[i].p = t.first;
+      tw.f[i].p = t.second;
+      continue;
+    }
     auto wd = twiddles<double>(len[i]);
     auto wf = twiddles<float>(len[i]);
-    tw.d[i] = DevBuf<cpx<double>>(len[i]);
-    tw.f[i] = DevBuf<cpx<float>>(len[i]);
+    tw.own_d[i] = DevBuf<cpx<double>>(len[i]);
+    tw.own_f[i] = DevBuf<cpx<float>>(len[i]);
+    tw.d[i].p = tw.own_d[i].p;
+    tw.f[i].p = tw.own_f[i].p;
     HIPCHK(hipMemcpyAsync(tw.d[i].p, wd.data(), wd.size() * sizeof(cpx<double>), hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(tw.f[i].p, wf.data(), wf.size() * sizeof(cpx<float>), hipMemcpyHostToDevice, s));
+    HIPCHK(hipStreamSynchronize(s));
   }
-  HIPCHK(hipStreamSynchronize(s));
 }
 
 // ------------------------------------------------------------ DIIS solve
@@ -350,7 +355,6 @@ struct SoluteState {
   DevBuf<cpx<double>> fs64;
   DevBuf<cpx<float>> fs32;  // y-major with the Nyquist column apart (fs_index)
   DevBuf<double> part;     // residual-workgroup partials, NPART each
-  DevBuf<double> sites;    // n * 6
   DevBuf<double> Dt, gmu;  // adjoint: dc/dt and dmu/dt at the converged t
   DevBuf<double> r64;      // mixed: F(t_b) at a rebase, FP64
   DevBuf<float> fb32;      // mixed: F(t_b) for the FP32 correction passes
@@ -405,11 +409,10 @@ struct Problem {
   int64_t mP;
   hipStream_t s;
   Twiddles tw;
-  DevBuf<double> chi_tab, tau_tab;      // 1D tables [pairs][nrad], [m][nrad]
   DevBuf<double> chi3, tau3;            // on the 3D k grid, FP64
   DevBuf<float> chi3f, tau3f;           // and FP32
   DevBuf<SoluteDesc> d_sd;
-  DevBuf<SitesDesc> d_sites;
+  SitesDesc* d_sites = nullptr;         // in setup
   DevBuf<double> d_out;                 // B * NPART
   DevBuf<void*> d_cdst, d_csrc;         // precision hand-over copies
   DevBuf<int> d_cmask;
@@ -423,16 +426,16 @@ struct Problem {
   // A copy each way and a wait for the stream took 15 to 20 us more a pass
   // (FP64, one solute: 50 -> 36 us at 32^3, 184 -> 165 us at 96^3).
   struct PassIO {
+    Pinned mem;               // sd and out
     SoluteDesc* sd = nullptr;
     uint64_t* out = nullptr;  // [B][NPART][2]
     uint64_t key = 0;         // of the last pass
     bool open = false;        // a pass is launched whose results nobody took
     std::vector<int> nq;      // its quantities per solute
-    ~PassIO() {
-      if (sd) (void)hipHostFree(sd);
-      if (out) (void)hipHostFree(out);
-    }
   } io;
+  // The small arrays of the setup (1D tables, sites, pointers), one upload.
+  DevBuf<char> setup;
+  Pinned setup_host;
   // The residual chain (five kernels + the norm reduction) as HIP graphs,
   // one per working precision and history width, captured on first use and
   // replayed every iteration (the descriptors they read are uploaded
@@ -589,13 +592,18 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
   if (pinned) {
     auto& io = pb.io;
     if (!io.sd) {
-      HIPCHK(hipHostMalloc((void**)&io.sd, pb.B * sizeof(SoluteDesc), hipHostMallocCoherent));
-      HIPCHK(hipHostMalloc((void**)&io.out, (size_t)pb.B * NPART * 16, hipHostMallocCoherent));
-      std::memset(io.out, 0, (size_t)pb.B * NPART * 16);
+      const size_t out_bytes = (size_t)pb.B * NPART * 16;
+      io.mem = Pinned(out_bytes + pb.B * sizeof(SoluteDesc));
+      io.out = io.mem.as<uint64_t>();
+      io.sd = io.mem.as<SoluteDesc>(out_bytes);
+      std::memset(io.out, 0, out_bytes);
+      // any start will do whose pairs no earlier pass of this memory wrote
+      static std::atomic<uint64_t> calls{0};
+      io.key = ++calls << 40;
     }
     if (io.open) HIPCHK(hipStreamSynchronize(pb.s));  // its load_sd may not have run yet
     io.open = true;
-    io.key += 0x9E3779B97F4A7C15ull;  // odd: 0 again only after 2^64 passes
+    ++io.key;
     io.nq.assign(pb.B, 0);
     for (int b = 0; b < pb.B; ++b) {
       sd[b].key = io.key;
@@ -1615,7 +1623,7 @@ void newton_solve(Problem& pb, const Config& cf, int b, int max_newton) {
       for (int i = 0; i < nv; ++i) res[i] += hp[(size_t)c * nv + i];
   };
   auto axpy_many = [&](double* wv, const double* Vb, const std::vector<double>& h, int nv) {
-    HIPCHK(hipMemcpy(hdev.p, h.data(), nv * 8, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpyWithStream(hdev.p, h.data(), nv * 8, hipMemcpyHostToDevice, pb.s));
     hipLaunchKernelGGL(maxpy, dim3(ch), dim3(NT), 0, pb.s, wv, Vb, hdev.p, nv, n);
   };
   auto [rinf, r2] = os.F(s.t64.p, nullptr, 0.0, r.p);
@@ -1928,9 +1936,8 @@ void info_observables(Problem& pb, const Inputs& in, int b, const SitesDesc& sit
   std::vector<double> hp((size_t)cp * INFO_NSUM), hi((size_t)n * ck);
   HIPCHK(hipMemcpyAsync(hp.data(), part.p, hp.size() * 8, hipMemcpyDeviceToHost, pb.s));
   HIPCHK(hipMemcpyAsync(hi.data(), ipart.p, hi.size() * 8, hipMemcpyDeviceToHost, pb.s));
-  if (out->potential)
-    HIPCHK(hipMemcpyAsync(out->potential, ve.p, P * 8, hipMemcpyDeviceToHost, pb.s));
   HIPCHK(hipStreamSynchronize(pb.s));
+  if (out->potential) host_copies({{out->potential, ve.p, (size_t)P * 8}}, true);
   HIPCHK(hipGetLastError());
   double acc[INFO_NSUM];
   for (int q = 0; q < INFO_NSUM; ++q) {
@@ -2210,12 +2217,13 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
   g.pse_order = pd->closure == RISM3D_CLOSURE_KH ? 1 : (pd->closure >= RISM3D_CLOSURE_PSE0 ? pd->closure - RISM3D_CLOSURE_PSE0 : 0);
   for (int i = 0; i < m; ++i) g.q[i] = solvent[i].charge;
   pb.mP = (int64_t)np * g.P;
-  HIPCHK(hipStreamCreateWithFlags(&pb.s, hipStreamNonBlocking));
+  pb.s = stream_take(opt.device);
   struct StreamGuard {  // idle before its buffers return to the cache
+    int dev;
     hipStream_t s;
-    ~StreamGuard() { (void)hipStreamSynchronize(s); (void)hipStreamDestroy(s); }
-  } sg{pb.s};
-  make_twiddles(pb.tw, pb.N, pb.s);
+    ~StreamGuard() { stream_give(dev, s); }
+  } sg{opt.device, pb.s};
+  make_twiddles(pb.tw, pb.N, pb.s, false);
 
   // omega_ij(k) in the chi3 slots of the pairs
   pb.chi3 = DevBuf<double>((size_t)np * w_points(g));
@@ -2228,7 +2236,7 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
         rij[i * (i + 1) / 2 + j] = std::sqrt(d2);
       }
     DevBuf<double> d_rij(np);
-    HIPCHK(hipMemcpy(d_rij.p, rij.data(), np * 8, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpyWithStream(d_rij.p, rij.data(), np * 8, hipMemcpyHostToDevice, pb.s));
     const int ck = (int)std::min<int64_t>(4096, (g.K + NT - 1) / NT);
     hipLaunchKernelGGL(omega3, dim3(ck, np), dim3(NT), 0, pb.s, g, pd->L[0], d_rij.p, pb.chi3.p);
     hipLaunchKernelGGL(nyq_tables<double>, nyq_grid(g, np), dim3(NT), 0, pb.s, g, pb.chi3.p);
@@ -2246,7 +2254,7 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
   pb.d_sd = DevBuf<SoluteDesc>(1);
   pb.d_out = DevBuf<double>(NPART);
   if (t_init)
-    HIPCHK(hipMemcpyAsync(s0.t64.p, t_init, pb.mP * 8, hipMemcpyHostToDevice, pb.s));
+    host_copies({{const_cast<double*>(t_init), s0.t64.p, (size_t)pb.mP * 8}}, false);
   else
     HIPCHK(hipMemsetAsync(s0.t64.p, 0, pb.mP * 8, pb.s));
   {
@@ -2257,7 +2265,7 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
       sse[3 * i + 2] = solvent[i].charge;
     }
     DevBuf<double> d_sse(sse.size());
-    HIPCHK(hipMemcpy(d_sse.p, sse.data(), sse.size() * 8, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpyWithStream(d_sse.p, sse.data(), sse.size() * 8, hipMemcpyHostToDevice, pb.s));
     const int cp = (int)std::min<int64_t>(4096, (g.P + NT - 1) / NT);
     hipLaunchKernelGGL(pair_field, dim3(cp, np), dim3(NT), 0, pb.s, g, d_sse.p, pd->L[0],
                        pd->L[1], pd->L[2], pb.h[0], pb.h[1], pb.h[2], s0.bv64.p);
@@ -2305,9 +2313,11 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
                        s0.R.p, g_out ? gbuf.p : (double*)nullptr, part.p);
     std::vector<double> hp((size_t)cp * 4);
     HIPCHK(hipMemcpyAsync(hp.data(), part.p, hp.size() * 8, hipMemcpyDeviceToHost, pb.s));
-    if (g_out) HIPCHK(hipMemcpyAsync(g_out, gbuf.p, pb.mP * 8, hipMemcpyDeviceToHost, pb.s));
-    if (t_out) HIPCHK(hipMemcpyAsync(t_out, s0.t64.p, pb.mP * 8, hipMemcpyDeviceToHost, pb.s));
     HIPCHK(hipStreamSynchronize(pb.s));
+    std::vector<HostCopy> down;
+    if (g_out) down.push_back({g_out, gbuf.p, (size_t)pb.mP * 8});
+    if (t_out) down.push_back({t_out, s0.t64.p, (size_t)pb.mP * 8});
+    host_copies(down, true);
     double acc[4] = {0, 0, 0, 0};
     for (int c = 0; c < cp; ++c)
       for (int q = 0; q < 4; ++q) acc[q] += hp[(size_t)c * 4 + q];
@@ -2337,8 +2347,8 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
     const int ck = (int)std::min<int64_t>(4096, (g.K + NT - 1) / NT);
     hipLaunchKernelGGL(chi_from_h, dim3(ck, np), dim3(NT), 0, pb.s, g,
                        (const cpx<double>*)s0.W.p, pb.chi3.p, cbuf.p);
-    HIPCHK(hipMemcpyAsync(chi_out, cbuf.p, cbuf.n * 8, hipMemcpyDeviceToHost, pb.s));
     HIPCHK(hipStreamSynchronize(pb.s));
+    host_copies({{chi_out, cbuf.p, cbuf.n * 8}}, true);
   }
   HIPCHK(hipGetLastError());
   return res->status;
@@ -2367,7 +2377,7 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
   pb.D = (in.opt.solver == RISM3D_SOLVER_MDIIS && !in.t_eval) ? in.opt.diis_depth : 1;
   pb.mixed = in.opt.precision != RISM3D_FP64;
   pb.noalloc = in.noalloc;
-  if (in.noalloc) pb.use_graphs = 0;
+  if (in.noalloc || in.t_eval) pb.use_graphs = 0;  // t_eval: one pass, no replay
   // BF16 residual history with defect correction only: the FP32-only study
   // iterates t itself to its floor, where the Gram rounding would show
   if (in.opt.precision != RISM3D_MIXED) pb.r16 = 0;
@@ -2411,71 +2421,42 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
   if (in.stream)
     pb.s = in.stream;
   else
-    HIPCHK(hipStreamCreateWithFlags(&pb.s, hipStreamNonBlocking));
+    pb.s = stream_take(in.opt.device);
   struct StreamGuard {  // idle before its buffers return to the cache
+    int dev;
     hipStream_t s;
     bool own;
     ~StreamGuard() {
-      (void)hipStreamSynchronize(s);
-      if (own) (void)hipStreamDestroy(s);
+      if (own) stream_give(dev, s);
+      else (void)hipStreamSynchronize(s);
     }
-  } sg{pb.s, in.stream == nullptr};
-  make_twiddles(pb.tw, pb.N, pb.s);
+  } sg{in.opt.device, pb.s, in.stream == nullptr};
+  make_twiddles(pb.tw, pb.N, pb.s, in.noalloc != 0);
 
   // Solvent kernel: chi - delta and the renormalisation tables
   // (solvent_kernel_rism, hnc3d.c:1499-1566; rism_solvent_renorm,
   // rism.f90:141-208).  chi_k is C layout [m][m][nrad].
   const int m = in.m, nrad = pd.nrad;
+  const size_t np = (size_t)m * (m + 1) / 2;
+  const bool f32 = pb.mixed != 0;  // the FP32 chain's copies
+  pb.chi3 = DevBuf<double>(np * w_points(g));
+  pb.tau3 = DevBuf<double>((size_t)m * w_points(g));
+  if (f32) {
+    pb.chi3f = DevBuf<float>(np * w_points(g));
+    pb.tau3f = DevBuf<float>((size_t)m * w_points(g));
+  }
   if (in.opt.chi3d) {
     // --solvent-3d: chi - 1 of a 3D solvent solve on this grid
     // (solvent_kernel_file, hnc3d.c:1434-1437, 1572-1590), no tau
-    const size_t np = (size_t)m * (m + 1) / 2;
-    pb.chi3 = DevBuf<double>(np * w_points(g));
-    pb.chi3f = DevBuf<float>(np * w_points(g));
-    pb.tau3 = DevBuf<double>((size_t)m * w_points(g));
-    pb.tau3f = DevBuf<float>((size_t)m * w_points(g));
     HIPCHK(hipMemcpy2DAsync(pb.chi3.p, g.NH * 8, in.opt.chi3d, g.NX * 8, g.NX * 8,
                             np * g.N1 * g.N2, hipMemcpyHostToDevice, pb.s));
     const int ck = (int)std::min<int64_t>(4096, (np * g.K + NT - 1) / NT);
-    hipLaunchKernelGGL(to_f32, dim3(ck), dim3(NT), 0, pb.s, pb.chi3f.p, pb.chi3.p,
-                       (int64_t)(np * g.K));
+    if (f32)
+      hipLaunchKernelGGL(to_f32, dim3(ck), dim3(NT), 0, pb.s, pb.chi3f.p, pb.chi3.p,
+                         (int64_t)(np * g.K));
     HIPCHK(hipMemsetAsync(pb.tau3.p, 0, pb.tau3.n * 8, pb.s));
-    HIPCHK(hipMemsetAsync(pb.tau3f.p, 0, pb.tau3f.n * 4, pb.s));
-  } else {
-  std::vector<double> chi_tab((size_t)m * (m + 1) / 2 * nrad), tau_tab((size_t)m * nrad);
-  for (int i = 0; i < m; ++i)
-    for (int j = 0; j <= i; ++j)
-      for (int k = 0; k < nrad; ++k)
-        chi_tab[((size_t)i * (i + 1) / 2 + j) * nrad + k] =  // S_ij = chi_ij sig_j / sig_i
-            in.chi_k[((size_t)i * m + j) * nrad + k] * (g.sig[j] / g.sig[i]) -
-            (i == j ? 1.0 : 0.0);
-  for (int i = 0; i < m; ++i)
-    for (int k = 0; k < nrad; ++k) {
-      const double kk = (2 * k + 1) * g.dk_tab / 2;
-      const double v = 4 * M_PI * std::exp(-kk * kk / (4 * G_COULOMB * G_COULOMB)) / (kk * kk);
-      double x = 0.0;
-      for (int j = 0; j < m; ++j) x += in.chi_k[((size_t)j * m + i) * nrad + k] * in.solvent[j].charge;
-      tau_tab[(size_t)i * nrad + k] = x * v;
-    }
-  pb.chi_tab = DevBuf<double>(chi_tab.size());
-  pb.tau_tab = DevBuf<double>(tau_tab.size());
-  HIPCHK(hipMemcpyAsync(pb.chi_tab.p, chi_tab.data(), chi_tab.size() * 8, hipMemcpyHostToDevice, pb.s));
-  HIPCHK(hipMemcpyAsync(pb.tau_tab.p, tau_tab.data(), tau_tab.size() * 8, hipMemcpyHostToDevice, pb.s));
-  {
-    const size_t np = (size_t)m * (m + 1) / 2;
-    pb.chi3 = DevBuf<double>(np * w_points(g));
-    pb.chi3f = DevBuf<float>(np * w_points(g));
-    pb.tau3 = DevBuf<double>((size_t)m * w_points(g));
-    pb.tau3f = DevBuf<float>((size_t)m * w_points(g));
-    const int ck = (int)std::min<int64_t>(4096, (g.K + NT - 1) / NT);
-    hipLaunchKernelGGL(ktab3, dim3(ck), dim3(NT), 0, pb.s, g, pb.chi_tab.p, pb.tau_tab.p,
-                       pb.chi3.p, pb.chi3f.p, pb.tau3.p, pb.tau3f.p);
-    hipLaunchKernelGGL(nyq_tables<double>, nyq_grid(g, m), dim3(NT), 0, pb.s, g, pb.tau3.p);
-    hipLaunchKernelGGL(nyq_tables<float>, nyq_grid(g, m), dim3(NT), 0, pb.s, g, pb.tau3f.p);
+    if (f32) HIPCHK(hipMemsetAsync(pb.tau3f.p, 0, pb.tau3f.n * 4, pb.s));
   }
-  }
-  hipLaunchKernelGGL(nyq_tables<double>, nyq_grid(g, m * (m + 1) / 2), dim3(NT), 0, pb.s, g, pb.chi3.p);
-  hipLaunchKernelGGL(nyq_tables<float>, nyq_grid(g, m * (m + 1) / 2), dim3(NT), 0, pb.s, g, pb.chi3f.p);
 
   // per-solute buffers
   const int B = in.B;
@@ -2483,11 +2464,7 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
   pb.nparts = m * std::max(resid_grid_x(g), g.N2);
   const int64_t mK = (int64_t)m * w_points(g);
   std::vector<SitesDesc> sites(B);
-  std::vector<double*> bv64p(B), tp(B), gp(B);
-  std::vector<float*> bv32p(B);
-  std::vector<cpx<double>*> fs64p(B);
-  std::vector<cpx<float>*> fs32p(B);
-  std::vector<std::vector<double>> site_host(B);
+  std::vector<double*> bv64p(B);
   for (int b = 0; b < B; ++b) {
     auto& s = pb.st[b];
     s.U = DevBuf<double>((size_t)pb.D * pb.mP);
@@ -2506,61 +2483,109 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
     if (pb.mixed) s.fs32 = DevBuf<cpx<float>>(w_points(g));  // fs_index
     s.part = DevBuf<double>((size_t)pb.nparts * NPART);
     s.n_sites = in.n_sites[b];
-    auto& sh = site_host[b];
-    sh.resize((size_t)s.n_sites * 6);
-    for (int a = 0; a < s.n_sites; ++a) {
-      const rism3d_site& st = in.solutes[b][a];
-      sh[6 * a + 0] = st.x[0]; sh[6 * a + 1] = st.x[1]; sh[6 * a + 2] = st.x[2];
-      sh[6 * a + 3] = st.sigma; sh[6 * a + 4] = st.epsilon; sh[6 * a + 5] = st.charge;
-    }
-    s.sites = DevBuf<double>(sh.size());
-    HIPCHK(hipMemcpyAsync(s.sites.p, sh.data(), sh.size() * 8, hipMemcpyHostToDevice, pb.s));
-    sites[b].xyz_s_e_q = s.sites.p;
-    sites[b].n = s.n_sites;
     bv64p[b] = s.bv64.p;
-    bv32p[b] = pb.mixed ? s.bv32.p : nullptr;
-    fs64p[b] = s.fs64.p;
-    fs32p[b] = pb.mixed ? s.fs32.p : nullptr;
-    // initial iterate: zero (hnc3d.c:1845) or the restart token
+    // initial iterate: zero (hnc3d.c:1845), the restart token, or the t of a
+    // single evaluation (copied where it is evaluated)
     if (t_init && b == 0)
       HIPCHK(hipMemcpyAsync(s.t64.p, t_init->data(), pb.mP * 8, hipMemcpyHostToDevice, pb.s));
-    else
+    else if (!in.t_eval)
       HIPCHK(hipMemsetAsync(s.t64.p, 0, pb.mP * 8, pb.s));
   }
   pb.d_sd = DevBuf<SoluteDesc>(B);
-  pb.d_sites = DevBuf<SitesDesc>(B);
   pb.d_out = DevBuf<double>((size_t)B * NPART);
   pb.d_cdst = DevBuf<void*>(B);
   pb.d_csrc = DevBuf<void*>(B);
   pb.d_cmask = DevBuf<int>(B);
-  HIPCHK(hipMemcpyAsync(pb.d_sites.p, sites.data(), B * sizeof(SitesDesc), hipMemcpyHostToDevice, pb.s));
 
-  // setup: beta v (field0) and F(k) s(k)
+  // setup: the tables chi - delta and tau, beta v (field0) and F(k) s(k),
+  // from small arrays that go up together
   {
-    std::vector<double> sse(3 * m);
-    for (int i = 0; i < m; ++i) {
-      sse[3 * i] = in.solvent[i].sigma;
-      sse[3 * i + 1] = in.solvent[i].epsilon;
-      sse[3 * i + 2] = in.solvent[i].charge;
+    size_t bytes = 0;
+    auto place = [&](size_t n) {
+      const size_t o = bytes;
+      bytes += (n + 255) & ~(size_t)255;
+      return o;
+    };
+    const bool tabs = !in.opt.chi3d;
+    const size_t o_chi = place(tabs ? np * nrad * 8 : 0), o_tau = place(tabs ? m * nrad * 8 : 0),
+                 o_sse = place(3 * m * 8), o_sd = place(B * sizeof(SitesDesc)),
+                 o_bv64 = place(B * 8), o_bv32 = place(B * 8), o_fs64 = place(B * 8),
+                 o_fs32 = place(B * 8);
+    std::vector<size_t> o_site(B);
+    for (int b = 0; b < B; ++b) o_site[b] = place((size_t)in.n_sites[b] * 6 * 8);
+    pb.setup = DevBuf<char>(bytes);
+    std::vector<char> pageable;
+    if (pb.noalloc) pageable.resize(bytes);
+    else pb.setup_host = Pinned(bytes);
+    char* const host = pb.noalloc ? pageable.data() : pb.setup_host.as<char>();
+    auto put = [&](size_t o) { return reinterpret_cast<double*>(host + o); };
+    auto ptr = [&](size_t o) { return reinterpret_cast<void**>(host + o); };
+    if (tabs) {
+      // chi_k is C layout [m][m][nrad]; S_ij = chi_ij sig_j / sig_i
+      double* chi_tab = put(o_chi);
+      for (int i = 0; i < m; ++i)
+        for (int j = 0; j <= i; ++j)
+          for (int k = 0; k < nrad; ++k)
+            chi_tab[((size_t)i * (i + 1) / 2 + j) * nrad + k] =
+                in.chi_k[((size_t)i * m + j) * nrad + k] * (g.sig[j] / g.sig[i]) -
+                (i == j ? 1.0 : 0.0);
+      double* tau_tab = put(o_tau);
+      for (int k = 0; k < nrad; ++k) {
+        const double kk = (2 * k + 1) * g.dk_tab / 2;
+        const double v = 4 * M_PI * std::exp(-kk * kk / (4 * G_COULOMB * G_COULOMB)) / (kk * kk);
+        for (int i = 0; i < m; ++i) {
+          double x = 0.0;
+          for (int j = 0; j < m; ++j)
+            x += in.chi_k[((size_t)j * m + i) * nrad + k] * in.solvent[j].charge;
+          tau_tab[(size_t)i * nrad + k] = x * v;
+        }
+      }
     }
-    DevBuf<double> d_sse(sse.size());
-    DevBuf<double*> d_bv64(B);
-    DevBuf<float*> d_bv32(B);
-    DevBuf<cpx<double>*> d_fs64(B);
-    DevBuf<cpx<float>*> d_fs32(B);
-    HIPCHK(hipMemcpyAsync(d_sse.p, sse.data(), sse.size() * 8, hipMemcpyHostToDevice, pb.s));
-    HIPCHK(hipMemcpyAsync(d_bv64.p, bv64p.data(), B * sizeof(double*), hipMemcpyHostToDevice, pb.s));
-    HIPCHK(hipMemcpyAsync(d_bv32.p, bv32p.data(), B * sizeof(float*), hipMemcpyHostToDevice, pb.s));
-    HIPCHK(hipMemcpyAsync(d_fs64.p, fs64p.data(), B * sizeof(void*), hipMemcpyHostToDevice, pb.s));
-    HIPCHK(hipMemcpyAsync(d_fs32.p, fs32p.data(), B * sizeof(void*), hipMemcpyHostToDevice, pb.s));
+    for (int i = 0; i < m; ++i) {
+      put(o_sse)[3 * i] = in.solvent[i].sigma;
+      put(o_sse)[3 * i + 1] = in.solvent[i].epsilon;
+      put(o_sse)[3 * i + 2] = in.solvent[i].charge;
+    }
+    for (int b = 0; b < B; ++b) {
+      auto& s = pb.st[b];
+      double* sh = put(o_site[b]);
+      for (int a = 0; a < s.n_sites; ++a) {
+        const rism3d_site& st = in.solutes[b][a];
+        sh[6 * a + 0] = st.x[0]; sh[6 * a + 1] = st.x[1]; sh[6 * a + 2] = st.x[2];
+        sh[6 * a + 3] = st.sigma; sh[6 * a + 4] = st.epsilon; sh[6 * a + 5] = st.charge;
+      }
+      sites[b].xyz_s_e_q = reinterpret_cast<const double*>(pb.setup.p + o_site[b]);
+      sites[b].n = s.n_sites;
+      sites[b].pad_ = 0;
+      ptr(o_bv64)[b] = s.bv64.p;
+      ptr(o_bv32)[b] = s.bv32.p;
+      ptr(o_fs64)[b] = s.fs64.p;
+      ptr(o_fs32)[b] = s.fs32.p;
+    }
+    std::memcpy(host + o_sd, sites.data(), B * sizeof(SitesDesc));
+    HIPCHK(hipMemcpyAsync(pb.setup.p, host, bytes, hipMemcpyHostToDevice, pb.s));
+    if (pb.noalloc) HIPCHK(hipStreamSynchronize(pb.s));  // host goes out of scope
+    auto at = [&](size_t o) { return reinterpret_cast<double*>(pb.setup.p + o); };
+    auto at_ptr = [&](size_t o) { return reinterpret_cast<void**>(pb.setup.p + o); };
+    pb.d_sites = reinterpret_cast<SitesDesc*>(pb.setup.p + o_sd);
     const int cp = (int)std::min<int64_t>(4096, (g.P + NT - 1) / NT);
     const int ck = (int)std::min<int64_t>(4096, (g.K + NT - 1) / NT);
-    hipLaunchKernelGGL(g.m <= 3 ? field_bv<3> : field_bv<MAX_SITES>, dim3(cp, B), dim3(NT), 0, pb.s, pb.d_sites.p, g, d_sse.p,
-                       pd.L[0], pd.L[1], pd.L[2], pb.h[0], pb.h[1], pb.h[2], d_bv64.p,
-                       pb.mixed ? d_bv32.p : (float* const*)nullptr);
-    hipLaunchKernelGGL(form_factor, dim3(ck, B), dim3(NT), 0, pb.s, pb.d_sites.p, g, d_fs64.p,
-                       pb.mixed ? d_fs32.p : (cpx<float>* const*)nullptr);
-    HIPCHK(hipStreamSynchronize(pb.s));
+    if (tabs) {
+      hipLaunchKernelGGL(ktab3, dim3(ck), dim3(NT), 0, pb.s, g, at(o_chi), at(o_tau), pb.chi3.p,
+                         pb.chi3f.p, pb.tau3.p, pb.tau3f.p);
+      hipLaunchKernelGGL(nyq_tables<double>, nyq_grid(g, m), dim3(NT), 0, pb.s, g, pb.tau3.p);
+      if (f32) hipLaunchKernelGGL(nyq_tables<float>, nyq_grid(g, m), dim3(NT), 0, pb.s, g, pb.tau3f.p);
+    }
+    hipLaunchKernelGGL(nyq_tables<double>, nyq_grid(g, (int)np), dim3(NT), 0, pb.s, g, pb.chi3.p);
+    if (f32)
+      hipLaunchKernelGGL(nyq_tables<float>, nyq_grid(g, (int)np), dim3(NT), 0, pb.s, g, pb.chi3f.p);
+    hipLaunchKernelGGL(g.m <= 3 ? field_bv<3> : field_bv<MAX_SITES>, dim3(cp, B), dim3(NT), 0, pb.s,
+                       pb.d_sites, g, at(o_sse), pd.L[0], pd.L[1], pd.L[2], pb.h[0], pb.h[1],
+                       pb.h[2], (double* const*)at_ptr(o_bv64),
+                       pb.mixed ? (float* const*)at_ptr(o_bv32) : (float* const*)nullptr);
+    hipLaunchKernelGGL(form_factor, dim3(ck, B), dim3(NT), 0, pb.s, pb.d_sites, g,
+                       (cpx<double>* const*)at_ptr(o_fs64),
+                       pb.mixed ? (cpx<float>* const*)at_ptr(o_fs32) : (cpx<float>* const*)nullptr);
     HIPCHK(hipGetLastError());
   }
 
@@ -2634,8 +2659,8 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
     const int64_t mP = pb.mP;
     const int ch = (int)std::min<int64_t>(2048, (mP + NT - 1) / NT);
     DevBuf<double> D(mP), v(mP), jv(mP);
-    HIPCHK(hipMemcpyAsync(s0.t64.p, in.t_eval, mP * 8, hipMemcpyHostToDevice, pb.s));
-    HIPCHK(hipMemcpyAsync(v.p, in.j_dt, mP * 8, hipMemcpyHostToDevice, pb.s));
+    host_copies({{const_cast<double*>(in.t_eval), s0.t64.p, (size_t)mP * 8},
+                 {const_cast<double*>(in.j_dt), v.p, (size_t)mP * 8}}, false);
     hipLaunchKernelGGL(closure_dcdt, dim3(ch), dim3(NT), 0, pb.s, g, s0.t64.p, s0.bv64.p, D.p, mP);
     std::vector<SoluteDesc> sd(1);
     std::memset(sd.data(), 0, sizeof(SoluteDesc));
@@ -2649,8 +2674,8 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
     sd[0].mode = in.j_flag ? 7 : 6;
     sd[0].active = 1;
     evaluate(pb, false, sd);
-    HIPCHK(hipMemcpyAsync(in.r_out, jv.p, mP * 8, hipMemcpyDeviceToHost, pb.s));
     HIPCHK(hipStreamSynchronize(pb.s));
+    host_copies({{in.r_out, jv.p, (size_t)mP * 8}}, true);
     HIPCHK(hipGetLastError());
     res[0].status = RISM3D_OK;
     return RISM3D_OK;
@@ -2659,7 +2684,10 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
   if (in.t_eval) {
     // one residual evaluation F(t) = T(t) - t (iterate_t1, hnc3d.c:1184)
     auto& s0 = pb.st[0];
-    HIPCHK(hipMemcpyAsync(s0.t64.p, in.t_eval, pb.mP * 8, hipMemcpyHostToDevice, pb.s));
+    if (pb.noalloc)
+      HIPCHK(hipMemcpyAsync(s0.t64.p, in.t_eval, pb.mP * 8, hipMemcpyHostToDevice, pb.s));
+    else
+      host_copies({{const_cast<double*>(in.t_eval), s0.t64.p, (size_t)pb.mP * 8}}, false);
     if (pb.mixed) convert_iterates(pb, std::vector<int>(1, 1), false);
     std::vector<SoluteDesc> sd(1);
     std::memset(sd.data(), 0, sizeof(SoluteDesc));
@@ -2672,15 +2700,16 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
     sd[0].part = s0.part.p;
     sd[0].active = 1;
     evaluate(pb, pb.mixed != 0, sd);
+    const double* r = s0.R.p;
     if (pb.mixed) {
       // FP32 residual to FP64 through the (now free) iterate buffers
       HIPCHK(hipMemcpyAsync(s0.t32.p, s0.R.p, pb.mP * 4, hipMemcpyDeviceToDevice, pb.s));
       convert_iterates(pb, std::vector<int>(1, 1), true);
-      HIPCHK(hipMemcpyAsync(in.r_out, s0.t64.p, pb.mP * 8, hipMemcpyDeviceToHost, pb.s));
-    } else {
-      HIPCHK(hipMemcpyAsync(in.r_out, s0.R.p, pb.mP * 8, hipMemcpyDeviceToHost, pb.s));
+      r = s0.t64.p;
     }
+    if (pb.noalloc) HIPCHK(hipMemcpyAsync(in.r_out, r, pb.mP * 8, hipMemcpyDeviceToHost, pb.s));
     HIPCHK(hipStreamSynchronize(pb.s));
+    if (!pb.noalloc) host_copies({{in.r_out, const_cast<double*>(r), (size_t)pb.mP * 8}}, true);
     HIPCHK(hipGetLastError());
     res[0].status = RISM3D_OK;
     return RISM3D_OK;
@@ -2729,22 +2758,28 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
         want_g = true;
       }
     }
-    DevBuf<const double*> d_tt(B);
-    DevBuf<double*> d_gg(B);
-    DevBuf<const double*> d_bv(B);
-    std::vector<const double*> bvc(bv64p.begin(), bv64p.end());
-    HIPCHK(hipMemcpyAsync(d_tt.p, tt.data(), B * sizeof(void*), hipMemcpyHostToDevice, pb.s));
-    HIPCHK(hipMemcpyAsync(d_gg.p, gg.data(), B * sizeof(void*), hipMemcpyHostToDevice, pb.s));
-    HIPCHK(hipMemcpyAsync(d_bv.p, bvc.data(), B * sizeof(void*), hipMemcpyHostToDevice, pb.s));
+    // their pointers up in one copy, the sums of the chunks down in another
+    Pinned up(3 * B * sizeof(void*));
+    DevBuf<void*> d_up(3 * B);
+    for (int b = 0; b < B; ++b) {
+      up.as<const void*>()[b] = tt[b];
+      up.as<const void*>()[B + b] = gg[b];
+      up.as<const void*>()[2 * B + b] = bv64p[b];
+    }
+    HIPCHK(hipMemcpyAsync(d_up.p, up.as<void>(), 3 * B * sizeof(void*), hipMemcpyHostToDevice, pb.s));
+    double* const* d_up64 = reinterpret_cast<double* const*>(d_up.p);
     const int cp = (int)std::min<int64_t>(2048, (g.P + NT - 1) / NT);
     DevBuf<double> d_mu((size_t)B * cp * 5);
-    hipLaunchKernelGGL(mu_density, dim3(cp, B), dim3(NT), 0, pb.s, pb.d_sites.p, g, d_tt.p, d_bv.p,
+    hipLaunchKernelGGL(mu_density, dim3(cp, B), dim3(NT), 0, pb.s, pb.d_sites, g,
+                       (const double* const*)d_up64, (const double* const*)(d_up64 + 2 * B),
                        pd.L[0], pd.L[1], pd.L[2], pb.h[0], pb.h[1], pb.h[2],
-                       want_g ? d_gg.p : (double* const*)nullptr, d_mu.p);
-    std::vector<double> mu((size_t)B * cp * 5);
-    HIPCHK(hipMemcpyAsync(mu.data(), d_mu.p, mu.size() * 8, hipMemcpyDeviceToHost, pb.s));
+                       want_g ? d_up64 + B : (double* const*)nullptr, d_mu.p);
+    Pinned mu_host(d_mu.n * 8);
+    const double* mu = mu_host.as<double>();
+    HIPCHK(hipMemcpyAsync(mu_host.as<void>(), d_mu.p, d_mu.n * 8, hipMemcpyDeviceToHost, pb.s));
     HIPCHK(hipStreamSynchronize(pb.s));
     HIPCHK(hipGetLastError());
+    std::vector<HostCopy> down;
     for (int b = 0; b < B; ++b) {
       double acc[5] = {0, 0, 0, 0, 0}, comp[5] = {0, 0, 0, 0, 0};
       for (int c = 0; c < cp; ++c)
@@ -2766,15 +2801,14 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
       res[b].iterations = s.iters;
       res[b].iterations_fp32 = s.iters32;
       res[b].status = s.status;
-      if (res[b].g)
-        HIPCHK(hipMemcpy(res[b].g, gg[b], pb.mP * 8, hipMemcpyDeviceToHost));
-      if (res[b].t)
-        HIPCHK(hipMemcpy(res[b].t, tt[b], pb.mP * 8, hipMemcpyDeviceToHost));
+      if (res[b].g) down.push_back({res[b].g, gg[b], (size_t)pb.mP * 8});
+      if (res[b].t) down.push_back({res[b].t, const_cast<double*>(tt[b]), (size_t)pb.mP * 8});
       if (t_final && b == 0) {
         t_final->resize(pb.mP);
-        HIPCHK(hipMemcpy(t_final->data(), tt[b], pb.mP * 8, hipMemcpyDeviceToHost));
+        down.push_back({t_final->data(), const_cast<double*>(tt[b]), (size_t)pb.mP * 8});
       }
     }
+    host_copies(down, true);
   }
   if (spec_out) {
     // forward spectrum of each converged t (closure pass with c = t, y,
@@ -3192,6 +3226,8 @@ int rism3d_solvent_chi(const rism3d_problem* pd, int m, const rism3d_site* solve
 int rism3d_cache_release(void) {
   std::lock_guard<std::mutex> lock(rism::g_mutex);
   rism::cache_empty(-1);
+  rism::host_pool_empty();
+  rism::twiddles_empty();
   return RISM3D_OK;
 }
 

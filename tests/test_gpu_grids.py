@@ -66,3 +66,26 @@ def test_tuner_records_choices_and_keeps_results(chi_w, tmp_path, monkeypatch):
     print("  " + "\n  ".join(lines), flush=True)
     keys = [ln.split()[0] for ln in lines if ln.strip()]
     assert "64x64x64,m3,B4,fp64" in keys and "64x64x64,m3,B4,fp32" in keys
+
+
+def test_size_classes_from_an_empty_cache(chi_w):
+    """The first calls of a process: every size class allocates, makes its
+    twiddle tables and records its graphs beside the others.  Nothing that
+    one class does may touch the default stream, which would void another's
+    recording.  Three classes, three times from an empty cache, mu as from a
+    warm one (the same kernels in the same order: bit-identical)."""
+    print("case grids from an empty cache", flush=True)
+    from bgy3d_amd import rism3d as R
+    from bgy3d_amd import synthetic as S
+    sols = [S.solute(s, n=4, net=0) for s in range(6)]
+    sets = [dict(README, N=N, L=0.15 * N, rmax=40.0, nrad=1536, closure="KH",
+                 **{"norm-tol": 1e-7, "max-iter": 500})
+            for N in (32, 48, 64, 32, 48, 64)]
+    got = []
+    for k in range(4):
+        if k < 3:
+            R.cache_release()
+        out = R.batch_solve_grids(sols, W, sets, chi_w, want_g=True)
+        assert all(o["status"] == "OK" for o in out)
+        got.append([o["free-energy"] for o in out])
+    assert all(g == got[-1] for g in got)
