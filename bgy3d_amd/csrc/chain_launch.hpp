@@ -3,6 +3,7 @@
 // chain_zpass.hip, chain_planes.hip, once with RISM_T double and once with
 // float), so that the instantiations build in parallel.
 #pragma once
+#include <algorithm>
 #include <cstdlib>
 
 #include "chain.hpp"
@@ -79,6 +80,16 @@ void launch_fft_y(int N1, dim3 grid, hipStream_t s, const SoluteDesc* sd, const 
 template <typename T>
 void launch_zstar(int N2, int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd,
                   const GridArgs& g, const cpx<T>* tw, const T* chi, const T* tau);
+// Workgroups of gram_rows per solute: 4 points or more a thread, 2048 at most
+// (a workgroup's own reduction is worth about 30 points a thread), and 8192 in
+// all: in a batch only the solutes at an extrapolation work, a third of them.
+// 24 x 64^3 in FP64: 139 us per pass with 85 workgroups a solute, 117 with 341.
+inline int gram_blocks(int64_t mP, int B) {
+  const int64_t most = std::max(64, std::min(2048, 8192 / B)), fit = mP / (NT * 4);
+  return (int)std::max<int64_t>(1, std::min(most, fit));
+}
+template <typename T>
+void launch_gram(dim3 grid, hipStream_t s, const SoluteDesc* sd, int64_t mP, int n);
 template <typename T>
 void launch_planes(bool inv, int B, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
                    const cpx<T>* twh, const cpx<T>* twf, const cpx<T>* twy, int hist);

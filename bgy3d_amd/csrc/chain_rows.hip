@@ -1,4 +1,4 @@
-// The x and y passes of the residual chain on rows.
+// The x and y passes of the residual chain on rows, and the Gram rows.
 #include "chain_launch.hpp"
 
 #ifndef RISM_T
@@ -74,6 +74,15 @@ void launch_fft_y(int N1, dim3 grid, hipStream_t s, const SoluteDesc* sd, const 
   }
 }
 
+// n: entries of the solute with the most.
+template <typename T>
+void launch_gram(dim3 grid, hipStream_t s, const SoluteDesc* sd, int64_t mP, int n) {
+  if (n <= 8) hipLaunchKernelGGL((gram_rows<T, 8>), grid, dim3(NT), 0, s, sd, mP);
+  else if (n <= 10) hipLaunchKernelGGL((gram_rows<T, 10>), grid, dim3(NT), 0, s, sd, mP);
+  else hipLaunchKernelGGL((gram_rows<T, MAX_DIIS>), grid, dim3(NT), 0, s, sd, mP);
+}
+
+template void launch_gram<RISM_T>(dim3, hipStream_t, const SoluteDesc*, int64_t, int);
 template void launch_closure_r2c<RISM_T>(int, dim3, hipStream_t, const SoluteDesc*, const GridArgs&,
                                          const cpx<RISM_T>*, const cpx<RISM_T>*, int);
 template void launch_c2r_resid<RISM_T>(int, dim3, hipStream_t, const SoluteDesc*, const GridArgs&,

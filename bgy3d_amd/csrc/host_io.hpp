@@ -149,9 +149,10 @@ void host_pool_empty() {
 // every page of a fresh array for the first time: 10 GB/s into a new 50 MB
 // array and 27 GB/s from one, of the link's 57.  Here several threads each
 // take every n-th chunk through two pinned slots and a stream of their own, so
-// that page faults, host copies and the link overlap: COPY_RATES.  One such
-// transfer at a time (the link is shared); arrays under COPY_MIN go through
-// the runtime (0.1 ms of thread starts is not paid back).
+// that page faults, host copies and the link overlap: 35 GB/s into a new 50 MB
+// array, 46 into 170 MB.  One such transfer at a time (the link is shared);
+// arrays under COPY_MIN go through the runtime (0.1 ms of thread starts is not
+// paid back).
 constexpr size_t COPY_CHUNK = (size_t)2 << 20;
 constexpr size_t COPY_MIN = (size_t)4 << 20;
 constexpr int COPY_THREADS = 8;

@@ -92,9 +92,10 @@ nyq_tables(GridArgs g, T* __restrict__ tab) {
 }
 
 // Fixed-order reduction of the residual-workgroup partials of each solute.
-// Grid: x = quantity (2 + the history width of the pass at least), y =
-// solute.  out[b * NPART + q]: max|r|, ||r||^2, <r, r_j>; with hout instead
-// the bits of the value at hout[2 (b * NPART + q)] and those bits ^ the
+// Grid: x = quantity (2 + the history width of the pass at least, or NOUT
+// where gram_rows ran, with ngparts partials), y = solute.  out[b * NOUT + q]:
+// max|r|, ||r||^2, <r, r_j> or the Gram rows (NOUT); with hout instead
+// the bits of the value at hout[2 (b * NOUT + q)] and those bits ^ the
 // solute's key behind them, in pinned host memory, where the host polls for
 // the pair (each word tells the other's arrival, so no order between the two
 // stores is needed, nor the end of the kernel).  One workgroup per
@@ -105,13 +106,21 @@ nyq_tables(GridArgs g, T* __restrict__ tab) {
 // 10% and 15% of a pass; this way 4.1 and 12.8 us.
 constexpr int NTR = 1024;
 __global__ void __launch_bounds__(NTR)
-reduce_resid(const SoluteDesc* __restrict__ sd, int nparts, double* __restrict__ out,
+reduce_resid(const SoluteDesc* __restrict__ sd, int nparts, int ngparts, double* __restrict__ out,
              uint64_t* __restrict__ hout) {
   __shared__ double red[NTR / 64];
   const SoluteDesc& d = sd[blockIdx.y];
   const int q = blockIdx.x;
-  if (!d.active || q >= 2 + d.ndot) return;
+  if (!d.active) return;
   const double* p = d.part + (int64_t)q * nparts;
+  if (q >= 2 && d.ngram) {
+    const int i = (q - 2) / MAX_DIIS, j = (q - 2) - i * MAX_DIIS;
+    if (i >= d.nrow || j <= i || j >= d.ngram) return;
+    p = d.gpart + (int64_t)(q - 2) * ngparts;
+    nparts = ngparts;
+  } else if (q >= 2 + d.ndot) {
+    return;
+  }
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
   for (int i = threadIdx.x; i < nparts; i += 4 * NTR) {
 #pragma unroll
@@ -131,7 +140,7 @@ reduce_resid(const SoluteDesc* __restrict__ sd, int nparts, double* __restrict__
     const double v = lane < NTR / 64 ? red[lane] : 0.0;
     const double r = q == 0 ? warp_max(v) : warp_sum(v);
     if (lane == 0) {
-      const size_t i = (size_t)blockIdx.y * NPART + q;
+      const size_t i = (size_t)blockIdx.y * NOUT + q;
       if (hout) {
         const uint64_t bits = (uint64_t)__double_as_longlong(r);
         __hip_atomic_store(hout + 2 * i, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -185,7 +194,7 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
   constexpr int NM = MAX_DIIS + 1;
   constexpr int MD = MAX_DIIS;
   __shared__ MdiisDev s;
-  __shared__ double o[NPART];
+  __shared__ double o[NOUT];
   __shared__ double pcol[NM];  // |column| by row position, for the pivot scan
   __shared__ int plane[NM];    // lane holding the row at each position
   __shared__ int ctl[4];       // flag, -, -, LU ok
@@ -196,7 +205,7 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
     const uint64_t* src = reinterpret_cast<const uint64_t*>(mst + b);
     uint64_t* dst = reinterpret_cast<uint64_t*>(&s);
     for (int i = l; i < (int)(sizeof(MdiisDev) / 8); i += 64) dst[i] = src[i];
-    if (l < NPART) o[l] = out[(size_t)b * NPART + l];
+    if (l < NOUT) o[l] = out[(size_t)b * NOUT + l];
     if (!act) return;
   }
   __syncthreads();
@@ -206,13 +215,24 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
   if (fin && l < nd0) {  // the new entry after the ones it was dotted with, its Gram row
     const int q = s.dotted[l];
     s.order[l] = q;
-    s.gram[sn * MD + q] = o[2 + l];
-    s.gram[q * MD + sn] = o[2 + l];
+    if (s.rows == 1) {
+      s.gram[sn * MD + q] = o[2 + l];
+      s.gram[q * MD + sn] = o[2 + l];
+    }
   }
+  if (fin && s.rows == 2 && l <= nd0) {  // or the rows of gram_rows, the newest entry first
+    auto entry = [&](int k) { return k == 0 ? sn : s.dotted[nd0 - k]; };
+    for (int i = 0; i <= s.pend && i < l; ++i) {
+      s.gram[entry(i) * MD + entry(l)] = o[2 + i * MD + l];
+      s.gram[entry(l) * MD + entry(i)] = o[2 + i * MD + l];
+    }
+  }
+  __syncthreads();  // rows and pend are read above, written below
   if (l == 0) {
     s.iters++;
     s.iters32++;
     s.resid = rinf;
+    if (rinf < s.low) s.low = rinf;
     int flag = 0;
     if (!fin) {
       flag = 2;
@@ -222,7 +242,7 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
       // with hold: the 1e3 drop only marks the solute ready, and one that
       // reached the phase's tolerance waits without iterating (parked)
       const bool drop = !s.only32 && rinf <= 1e-3 * s.rb_rinf, conv = rinf <= s.tol_half;
-      if (s.stall32 >= 12 || s.iters32 >= s.max_iter || (!s.hold && (drop || conv)) ||
+      if (s.stall32 >= stall_passes(s.period, s.low) || s.iters32 >= s.max_iter || (!s.hold && (drop || conv)) ||
           (s.only32 && conv))
         flag = 1;
       else if (conv)
@@ -235,19 +255,24 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
       s.gram[sn * MD + sn] = r2;
       // restart when the residual blows up against the best one, or stalls
       if (r2 < s.best) { s.best = r2; s.since_best = 0; } else { s.since_best++; }
-      if (r2 > 100.0 * s.best || s.since_best > 3 * s.D) {
+      const bool extrap = s.rows != 0;
+      s.pend = extrap ? 0 : s.pend + 1;
+      s.skipped = extrap ? 0 : s.skipped + 1;
+      if (r2 > (extrap ? RESTART_EXTRAP : RESTART_PLAIN) * s.best || s.since_best > 3 * s.D) {
         s.order[0] = sn;
         s.n = 1;
         s.best = r2;
         s.since_best = 0;
+        s.pend = s.skipped = 0;
       }
+      s.picard = !extrap || s.n == 1;
     }
     ctl[0] = flag;
     ctl[3] = 0;
   }
   __syncthreads();
   const int flag = ctl[0];
-  if (flag != 2 && s.n > 1) {
+  if (flag != 2 && !s.picard) {
     // bordered system [G/sc -1; -1 0] [c; l] = [0; -1], sc = max diag G
     const int nh = s.n, n = nh + 1;
     double sc = 0.0;
@@ -369,10 +394,10 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
     }
   }
   __syncthreads();
-  if (flag != 2 && (s.n == 1 || !ctl[3]) && l == 0) {  // one entry, or no usable solution: restart
+  if (flag != 2 && !s.picard && !ctl[3] && l == 0) {  // no usable solution: restart
     s.order[0] = s.slot_new;
     s.n = 1;
-    s.coef[0] = 1.0;
+    s.picard = 1;
   }
   __syncthreads();
   if (flag == 0 || flag == 4) {
@@ -385,7 +410,10 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
     const bool fresh = n < D;
     const int q = fresh ? __ffsll(~busy) - 1 : s.order[0];
     const int nd = fresh ? n : n - 1;
-    if (l + 1 < n) {
+    // the rows of the next pass (the host's make_desc)
+    const int period = s.low <= PULAY_BELOW ? s.period : 1;
+    const int rows = s.skipped + 1 >= period ? (s.pend ? 2 : 1) : 0;
+    if (!s.picard && l + 1 < n) {
       double cum = 0.0;
       for (int i = 0; i <= l; ++i) cum += s.coef[i];
       d.u[1 + l] = s.U + (size_t)s.order[l + 1] * s.mP;
@@ -395,19 +423,28 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
     if (l < nd) {
       const int qq = s.order[fresh ? l : l + 1];
       s.dotted[l] = qq;
-      d.rh[l] = s.R + (size_t)qq * s.mP;
-      d.rhinv[l] = 1.0f / s.rsc[qq];
+      const int at = rows == 2 ? nd - l : l;  // gram_rows: the newest first
+      d.rh[at] = s.R + (size_t)qq * s.mP * s.rbytes;
+      d.rhinv[at] = 1.0f / s.rsc[qq];
     }
     if (l == 0) {
-      d.ncomb = n;
+      if (rows == 2) {
+        d.rh[0] = s.R + (size_t)q * s.mP * s.rbytes;
+        d.rhinv[0] = 1.0f / rsc;
+      }
+      d.ngram = rows == 2 ? nd + 1 : 0;
+      d.nrow = s.pend + 1;
+      s.rows = rows;
+      d.ncomb = s.picard ? 1 : n;
+      d.plain = s.picard;
       d.u[0] = s.ucur;
       d.coef[0] = 1.0;
       s.slot_new = q;
       s.ndot = nd;
-      d.ndot = nd;
+      d.ndot = rows == 1 ? nd : 0;
       s.rsc[q] = rsc;
       d.rsc = rsc;
-      d.r = s.R + (size_t)q * s.mP;
+      d.r = s.R + (size_t)q * s.mP * s.rbytes;
       d.dnew = s.U + (size_t)q * s.mP;
     }
   } else if (l == 0) {
@@ -419,7 +456,7 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
     MdiisStatus& st = status[b];
     st.flag = flag;
     st.iters32 = s.iters32;
-    st.hist = (flag == 0 || flag == 4) ? (s.n > s.ndot ? s.n : s.ndot) : 0;
+    st.hist = (flag == 0 || flag == 4) ? (d.ncomb > d.ndot ? d.ncomb : d.ndot) : 0;
     st.resid = rinf;
     st.r2 = r2;
     __threadfence_system();

@@ -56,12 +56,42 @@ struct SoluteDesc {
   float rhinv[MAX_DIIS];     // r8: 1 / the scale of rh[j]
   uint64_t key;              // of this pass, never 0, where the norms go to the
                              //   host's memory (reduce_resid)
+  int plain;                 // u16: t is the u that the new one replaces (u[0])
+  int pad_plain_;
+  int ngram;                 // 0, or (with ndot = 0) the residuals rh[0..ngram-1],
+                             //   the new one first and older ones behind, whose
+  int nrow;                  //   products <rh[i], rh[j]>, i < nrow, j > i, the pass
+                             //   forms after it (gram_rows): several Gram rows from
+  double* gpart;             //   one reading of the history; its partials
 };
 static_assert(sizeof(SoluteDesc) % 8 == 0, "SoluteDesc is copied in 8-byte words");
 constexpr int NPART = 2 + MAX_DIIS;   // doubles per residual workgroup
+constexpr int MAX_ROWS = 3;           // Gram rows of one gram_rows pass
+// A pass's results per solute: max|r|, ||r||^2, then <r, r_j> (ndot) or
+// <rh[i], rh[j]> at 2 + i MAX_DIIS + j (ngram).
+constexpr int NOUT = 2 + MAX_ROWS * MAX_DIIS;
+
+// Periodic Pulay mixing.  Between two MDIIS extrapolations the iteration takes
+// PULAY_PERIOD - 1 plain steps t = u, whose entries join the history without
+// a reading of it (Banerjee, Suryanarayana and Pask, Chem. Phys. Lett. 647,
+// 31 (2016)); their Gram rows are formed together at the next extrapolation.
+// It begins once max|F| fell to PULAY_BELOW, where the closure is close to
+// linear (above, a plain step can overshoot: with period 3 from the start
+// Cl- with PSE-3 took 78 passes instead of 45, and Na+ with HNC could
+// overflow), at once for the linear adjoint, and with at least PULAY_DEPTH
+// entries.  Passes to 1e-10, MDIIS each pass and period 3: 227 and 215, 322
+// and 263, 425 and 233 (14-site solutes, KH, 64^3), 393 and 315 (PSE-3), 375
+// and 268 (saline), 45 and 55 (Cl-, PSE-3, the worst seen), adjoint 604 and
+// 190.  Not for the 3D solvent: 82 and 122.
+constexpr int PULAY_PERIOD = 3;
+constexpr int PULAY_DEPTH = 5;
+constexpr double PULAY_BELOW = 1.0;
+// Restart limits on ||F||^2 over its best: at an extrapolation, after a plain
+// step.
+constexpr double RESTART_EXTRAP = 100.0, RESTART_PLAIN = 1e4;
 
 // MDIIS state of one solute in the FP32 defect-correction phase with the
-// difference-form u history and the FP8 residual history, kept on the
+// difference-form u history and the BF16 or FP8 residual history, kept on the
 // device between passes (mdiis_step): the history bookkeeping the host loop
 // would otherwise do between two residual passes.  The host takes a
 // solute's state back when it asks for a rebase or fails.  gram is indexed
@@ -70,7 +100,7 @@ struct MdiisDev {
   // fixed while the solute stays on the device
   float* ucur;            // the newest u (FP32)
   uint16_t* U;            // BF16 difference slots, mP each
-  uint8_t* R;             // FP8 residual slots, mP each
+  uint8_t* R;             // residual slots, mP each, BF16 or FP8
   int64_t mP;
   double rb_rinf;         // max|F(t_b)| of the current base
   double tol_half;        // half the FP64-checked tolerance of the phase
@@ -83,6 +113,12 @@ struct MdiisDev {
   int slot_new;           // slot receiving the pending r and u
   int ndot;               // entries the pending r is dotted with (dotted)
   int since_best, stall32, iters, iters32;
+  int rbytes;             // of a residual: 2 (BF16) or 1 (FP8)
+  int period;             // PULAY_PERIOD, or 1: every pass extrapolates
+  int skipped;            // plain steps since the last extrapolation
+  int pend;               // newest entries without Gram rows
+  int rows;               // of the pending pass: 0 none, 1 its dots, 2 gram_rows
+  int picard;             // the next pass takes t = the newest u
   int hold;               // the 1e3 drop only marks the solute ready (flag 4),
                           // the phase's tolerance parks it (flag 5)
   int order[MAX_DIIS];
@@ -91,6 +127,7 @@ struct MdiisDev {
   float rsc[MAX_DIIS];    // FP8 scale of each slot's residual
   double coef[MAX_DIIS];  // t = sum coef_j u_{order_j} for the next pass
   double resid, best, best32;
+  double low;             // lowest max|F| of the iteration
   double gram[MAX_DIIS * MAX_DIIS];
 };
 static_assert(sizeof(MdiisDev) % 8 == 0, "MdiisDev is copied in 8-byte words");
@@ -104,6 +141,12 @@ struct MdiisStatus {
   int hist;               // flag 0: history slots of the next pass, max(ncomb, ndot)
   double resid, r2;       // max|F|, ||F||^2 of the pass
 };
+
+// Passes of the FP32 phase without a 30% gain on its best residual that ask
+// for a rebase: plain steps do not gain by themselves.
+__host__ __device__ inline int stall_passes(int period, double low) {
+  return period > 1 && low <= PULAY_BELOW ? 18 : 12;
+}
 
 // FP8 residual history: the scale that puts max|r| = rinf at 240 (the
 // largest e4m3 value is 448; the next pass's residual may grow 1.8x before

@@ -355,6 +355,7 @@ struct SoluteState {
   DevBuf<cpx<double>> fs64;
   DevBuf<cpx<float>> fs32;  // y-major with the Nyquist column apart (fs_index)
   DevBuf<double> part;     // residual-workgroup partials, NPART each
+  DevBuf<double> gpart;    // gram_rows partials, MAX_ROWS * MAX_DIIS each
   DevBuf<double> Dt, gmu;  // adjoint: dc/dt and dmu/dt at the converged t
   DevBuf<double> r64;      // mixed: F(t_b) at a rebase, FP64
   DevBuf<float> fb32;      // mixed: F(t_b) for the FP32 correction passes
@@ -388,6 +389,13 @@ struct SoluteState {
   int polish = 0;             // FP64 steps taken after the FP32 phase
   double resid = INFINITY, best = INFINITY;
   int since_best = 0;
+  // periodic Pulay mixing (kernels.hpp)
+  double low = INFINITY;      // lowest max|F| of the iteration
+  int skipped = 0;            // plain steps since the last extrapolation
+  int pend = 0;               // newest entries without Gram rows
+  int rows = 0;               // of the pending pass: 0 none, 1 its dots, 2 gram_rows
+  int picard = 0;             // the next pass takes t = the newest u
+  int talias = -1;            // FP64: the u slot the last pass read as its t
 };
 
 struct Problem {
@@ -395,6 +403,7 @@ struct Problem {
   int N[3];
   double L[3], h[3];
   int D;          // DIIS depth (1 = Picard)
+  int period = 1; // of the running iteration: PULAY_PERIOD or 1 (kernels.hpp)
   int mixed;
   int r16 = env_int("RISM3D_R_BF16", 1);  // FP32 phase: residual history in BF16
   int D32 = env_int("RISM3D_DEPTH32", 0);   // FP32 phase: MDIIS depth (0: D)
@@ -403,8 +412,12 @@ struct Problem {
   // in FP32 and the differences of consecutive entries in BF16
   int u16 = env_int("RISM3D_U_DIFF", 1);
   // FP32 phase (with r16): the residual history in FP8 e4m3, each entry
-  // scaled by 240 / (max|r| of the previous pass) into the e4m3 range
-  int r8 = env_int("RISM3D_R_FP8", 1);
+  // scaled by 240 / (max|r| of the previous pass) into the e4m3 range; -1:
+  // where every pass extrapolates.  Periodic mixing reads the history once in
+  // three passes and tells nearly parallel residuals apart, for which FP8 is
+  // too coarse: 253 passes to 1e-10 with FP8 each pass, 249 with BF16 and
+  // period 3, 395 with FP8 and period 3 (12-site solutes, 64^3, depth 10).
+  int r8 = env_int("RISM3D_R_FP8", -1);
   int B;
   int64_t mP;
   hipStream_t s;
@@ -413,7 +426,7 @@ struct Problem {
   DevBuf<float> chi3f, tau3f;           // and FP32
   DevBuf<SoluteDesc> d_sd;
   SitesDesc* d_sites = nullptr;         // in setup
-  DevBuf<double> d_out;                 // B * NPART
+  DevBuf<double> d_out;                 // B * NOUT
   DevBuf<void*> d_cdst, d_csrc;         // precision hand-over copies
   DevBuf<int> d_cmask;
   int nparts = 0;  // partials per quantity: workgroups of the residual kernel at most
@@ -428,10 +441,10 @@ struct Problem {
   struct PassIO {
     Pinned mem;               // sd and out
     SoluteDesc* sd = nullptr;
-    uint64_t* out = nullptr;  // [B][NPART][2]
+    uint64_t* out = nullptr;  // [B][NOUT][2]
     uint64_t key = 0;         // of the last pass
     bool open = false;        // a pass is launched whose results nobody took
-    std::vector<int> nq;      // its quantities per solute
+    std::vector<std::vector<int>> q;  // its quantities per solute
   } io;
   // The small arrays of the setup (1D tables, sites, pointers), one upload.
   DevBuf<char> setup;
@@ -443,20 +456,21 @@ struct Problem {
   // RISM3D_GRAPHS=0 launches the kernels one by one instead.
   struct Graphs {
     // [FP64 / FP32 / FP32 with the device MDIIS step][history width 8 / 10 / 16]
-    hipGraph_t graph[3][3] = {};
-    hipGraphExec_t exec[3][3] = {};
-    GridArgs key[3][3];
-    ~Graphs() {
-      for (int a = 0; a < 3; ++a)
-        for (int b = 0; b < 3; ++b) {
-          if (exec[a][b]) (void)hipGraphExecDestroy(exec[a][b]);
-          if (graph[a][b]) (void)hipGraphDestroy(graph[a][b]);
-        }
-    }
+    // [gram_rows: none / width 8 / 10 / 16]
+    struct One {
+      hipGraph_t graph = nullptr;
+      hipGraphExec_t exec = nullptr;
+      GridArgs key;
+      ~One() {
+        if (exec) (void)hipGraphExecDestroy(exec);
+        if (graph) (void)hipGraphDestroy(graph);
+      }
+    } one[3][3][4];
   } graphs;
   int use_graphs = env_int("RISM3D_GRAPHS", 1);
+  int pulay = std::min(MAX_ROWS, std::max(1, env_int("RISM3D_PULAY", PULAY_PERIOD)));
   // RISM3D_DEVICE_MDIIS=1: the FP32 phase's MDIIS step on the device
-  // (mdiis_step, with the difference-form u and FP8 r histories): its own
+  // (mdiis_step, with the difference-form u and 16 or 8 bit r histories): its own
   // descriptors, which the step rewrites, the solutes' history state and
   // the pinned status array the host polls after each pass.  Off by
   // default: the same step on the host measured about 1% faster, on the
@@ -521,8 +535,8 @@ void download_out(Problem& pb, std::vector<double>& out) {
   long spin = 0;
   bool ended = false;
   for (int b = 0; b < pb.B; ++b)
-    for (int q = 0; q < io.nq[b]; ++q)
-      while (!taken((size_t)b * NPART + q)) {
+    for (int q : io.q[b])
+      while (!taken((size_t)b * NOUT + q)) {
         // the stream is asked only now and then (a failed pass ends the wait
         // within milliseconds): its lock is shared with the launches of other
         // threads, such as the size classes of rism3d_batch_solve_grids
@@ -533,8 +547,10 @@ void download_out(Problem& pb, std::vector<double>& out) {
           throw HipFailure{hipErrorUnknown};
         }
         const hipError_t e = hipStreamQuery(pb.s);
-        if (e == hipSuccess) ended = true;  // everything it wrote arrives by the next look
-        else if (e != hipErrorNotReady) HIPCHK(e);
+        if (e == hipErrorNotReady) continue;
+        HIPCHK(e);
+        HIPCHK(hipStreamSynchronize(pb.s));
+        ended = true;  // everything it wrote arrives by the next look
       }
   io.open = false;
 }
@@ -575,6 +591,14 @@ int hist_of(const std::vector<SoluteDesc>& sd) {
   return h;
 }
 
+// Entries of the largest gram_rows pass of this batch (0: none).
+int gram_of(const std::vector<SoluteDesc>& sd) {
+  int n = 0;
+  for (const auto& d : sd)
+    if (d.active) n = std::max(n, d.ngram);
+  return n;
+}
+
 // One residual pass over the batch.  step 0: the host's descriptors sd.
 // step 1 (FP32): the descriptors already in pb.d_sd32, with hist2 history
 // slots at most; the device MDIIS step (mdiis_step) follows the pass and
@@ -592,7 +616,7 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
   if (pinned) {
     auto& io = pb.io;
     if (!io.sd) {
-      const size_t out_bytes = (size_t)pb.B * NPART * 16;
+      const size_t out_bytes = (size_t)pb.B * NOUT * 16;
       io.mem = Pinned(out_bytes + pb.B * sizeof(SoluteDesc));
       io.out = io.mem.as<uint64_t>();
       io.sd = io.mem.as<SoluteDesc>(out_bytes);
@@ -604,10 +628,16 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
     if (io.open) HIPCHK(hipStreamSynchronize(pb.s));  // its load_sd may not have run yet
     io.open = true;
     ++io.key;
-    io.nq.assign(pb.B, 0);
+    io.q.resize(pb.B);
     for (int b = 0; b < pb.B; ++b) {
-      sd[b].key = io.key;
-      if (sd[b].active) io.nq[b] = 2 + sd[b].ndot;
+      SoluteDesc& d = sd[b];
+      auto& q = io.q[b];
+      d.key = io.key;
+      q.clear();
+      if (!d.active) continue;
+      for (int k = 0; k < 2 + d.ndot; ++k) q.push_back(k);
+      for (int i = 0; d.ngram && i < d.nrow; ++i)
+        for (int j = i + 1; j < d.ngram; ++j) q.push_back(2 + i * MAX_DIIS + j);
     }
     std::memcpy(io.sd, sd.data(), sd.size() * sizeof(SoluteDesc));
   } else if (!step) {
@@ -633,6 +663,8 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
     if (g.zwide && (g.NX - 1) % 32 != 0) g.zwide = 0;
   }
   const int nparts = planes ? g.m * g.N2 : resid_grid_x(g) * g.m;  // partials per quantity
+  const int ngram = step ? (pb.period > 1 ? pb.D : 0) : gram_of(sd);
+  const int ngparts = gram_blocks((int64_t)g.m * g.P, pb.B);
   auto chain = [&]() {
     if (pinned)
       hipLaunchKernelGGL(load_sd, dim3(pb.B), dim3(NTL), 0, pb.s, (const SoluteDesc*)pb.io.sd, dsd);
@@ -665,29 +697,38 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
       mark(3, 0); launch_fft_y<T, true>(g.N1, gy, pb.s, dsd, g, pb.tw.d[2].p); mark(3, 1);
       mark(4, 0); launch_c2r_resid<T>(g.N0, gx, pb.s, dsd, g, pb.tw.d[1].p, pb.tw.d[0].p, hist); mark(4, 1);
     }
+    if (ngram && fp32)
+      launch_gram<float>(dim3(ngparts, pb.B), pb.s, dsd, (int64_t)g.m * g.P, ngram);
+    else if (ngram)
+      launch_gram<double>(dim3(ngparts, pb.B), pb.s, dsd, (int64_t)g.m * g.P, ngram);
     // 2 + the history width this launch (or graph, captured per width) serves
-    const int nq = 2 + (hist <= 8 ? 8 : (hist <= 10 ? 10 : MAX_DIIS));
-    hipLaunchKernelGGL(reduce_resid, dim3(nq, pb.B), dim3(NTR), 0, pb.s, dsd, nparts, pb.d_out.p,
+    const int nq = ngram ? NOUT : 2 + (hist <= 8 ? 8 : (hist <= 10 ? 10 : MAX_DIIS));
+    hipLaunchKernelGGL(reduce_resid, dim3(nq, pb.B), dim3(NTR), 0, pb.s, dsd, nparts, ngparts, pb.d_out.p,
                        pinned ? pb.io.out : (uint64_t*)nullptr);
     if (step)
       hipLaunchKernelGGL(mdiis_step, dim3(pb.B), dim3(64), 0, pb.s, pb.d_out.p, pb.d_mdiis.p, dsd,
                          pb.h_status.p);
   };
   if (pb.use_graphs && !pf.on) {
-    auto& G = pb.graphs;
     const int a = step ? 2 : (fp32 ? 1 : 0), b = hist <= 8 ? 0 : (hist <= 10 ? 1 : 2);
-    if (!G.exec[a][b] || std::memcmp(&G.key[a][b], &g, sizeof g) != 0) {
-      if (G.exec[a][b]) HIPCHK(hipGraphExecDestroy(G.exec[a][b]));
-      if (G.graph[a][b]) HIPCHK(hipGraphDestroy(G.graph[a][b]));
-      G.exec[a][b] = nullptr;
-      G.graph[a][b] = nullptr;
+    auto& G = pb.graphs.one[a][b][ngram == 0 ? 0 : ngram <= 8 ? 1 : ngram <= 10 ? 2 : 3];
+    if (!G.exec || std::memcmp(&G.key, &g, sizeof g) != 0) {
+      if (G.exec) HIPCHK(hipGraphExecDestroy(G.exec));
+      G.exec = nullptr;
+      if (G.graph) HIPCHK(hipGraphDestroy(G.graph));
+      G.graph = nullptr;
       HIPCHK(hipStreamBeginCapture(pb.s, hipStreamCaptureModeThreadLocal));
       chain();
-      HIPCHK(hipStreamEndCapture(pb.s, &G.graph[a][b]));
-      HIPCHK(hipGraphInstantiate(&G.exec[a][b], G.graph[a][b], nullptr, nullptr, 0));
-      std::memcpy(&G.key[a][b], &g, sizeof g);
+      if (hipStreamEndCapture(pb.s, &G.graph) == hipSuccess && G.graph) {
+        HIPCHK(hipGraphInstantiate(&G.exec, G.graph, nullptr, nullptr, 0));
+        std::memcpy(&G.key, &g, sizeof g);
+      } else {  // voided by another thread's use of the default stream
+        (void)hipGetLastError();
+        G.graph = nullptr;
+      }
     }
-    HIPCHK(hipGraphLaunch(G.exec[a][b], pb.s));
+    if (G.exec) HIPCHK(hipGraphLaunch(G.exec, pb.s));
+    else chain();
   } else {
     chain();
   }
@@ -922,15 +963,15 @@ void rebase(Problem& pb, const Config& cf, const std::vector<int>& mask, bool ad
     }
   }
   evaluate(pb, false, sd);
-  std::vector<double> out((size_t)B * NPART);
+  std::vector<double> out((size_t)B * NOUT);
   download_out(pb, out);
   HIPCHK(hipGetLastError());
   rinf.assign(B, 0.0);
   r2.assign(B, 0.0);
   for (int b = 0; b < B; ++b) {
     if (!mask[b]) continue;
-    rinf[b] = out[(size_t)b * NPART];
-    r2[b] = out[(size_t)b * NPART + 1];
+    rinf[b] = out[(size_t)b * NOUT];
+    r2[b] = out[(size_t)b * NOUT + 1];
   }
 }
 
@@ -982,12 +1023,16 @@ void rebase_start(Problem& pb, const Config& cf, int b, double r2, bool seed) {
     s.gram[0] = r2;
     s.best = r2;
     s.since_best = 0;
+    s.picard = 1;
+    s.pend = s.skipped = 0;
     return;
   }
   std::vector<int> keep;
   for (int q : s.order)
     if (s.sbase[q] == s.base) keep.push_back(q);
-  if (keep.size() != s.order.size()) {
+  if (keep.size() != s.order.size() && s.picard) {
+    s.order = keep;  // a plain step: no coefficients to refit, Gram rows pending
+  } else if (keep.size() != s.order.size()) {
     s.order = keep;
     const int nh = (int)s.order.size();
     std::vector<double> G(nh * nh);
@@ -996,6 +1041,7 @@ void rebase_start(Problem& pb, const Config& cf, int b, double r2, bool seed) {
     if (nh == 1 || !diis_coefficients(G, nh, s.coef)) {
       s.order.assign(1, s.order.back());
       s.coef.assign(1, 1.0);
+      s.picard = 1;
     }
   }
   std::swap(s.dcur, s.dshift);
@@ -1017,10 +1063,16 @@ void iterate_batch(Problem& pb, const Config& cf) {
   const int64_t mP = pb.mP;
   const int D = pb.D;
   std::vector<SoluteDesc> sd(B);
-  std::vector<double> out((size_t)B * NPART);
+  std::vector<double> out((size_t)B * NOUT);
   std::vector<int> act(B, 0);
+  pb.period = D >= PULAY_DEPTH && pb.g.special == 0 ? pb.pulay : 1;
   for (int b = 0; b < B; ++b) {
     auto& s = pb.st[b];
+    s.low = cf.mode == 1 ? 0.0 : INFINITY;  // the adjoint is linear throughout
+    s.skipped = s.pend = s.rows = s.picard = 0;
+    s.talias = -1;
+    if (s.active && pb.period > 1 && !s.gpart.p)
+      s.gpart = DevBuf<double>((size_t)MAX_ROWS * MAX_DIIS * gram_blocks(mP, B));
     act[b] = s.active != 0;
     s.phase32 = s.active && cf.precision != RISM3D_FP64;
     s.gram.assign(D * D, 0.0);
@@ -1050,6 +1102,8 @@ void iterate_batch(Problem& pb, const Config& cf) {
     s.gram[0] = r2;
     s.best = r2;
     s.since_best = 0;
+    s.picard = 1;
+    s.pend = s.skipped = 0;
   };
   auto after_rebase = [&](const std::vector<int>& mask, const std::vector<double>& rinf,
                           const std::vector<double>& r2, bool seed) {
@@ -1060,6 +1114,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
       s.ready_at = -1;
       s.iters++;
       s.resid = rinf[b];
+      s.low = std::min(s.low, rinf[b]);
       if (cf.verbose)
         std::fprintf(stderr, "rism3d: solute %d iter %d fp64 rebase |F|inf = %.3e\n", b, s.iters,
                      rinf[b]);
@@ -1100,8 +1155,8 @@ void iterate_batch(Problem& pb, const Config& cf) {
     after_rebase(act, rinf, r2, true);
   }
   // the FP32 phase's MDIIS step on the device (mdiis_step): the history in
-  // difference form with FP8 residuals, the library's own allocations
-  const bool dev_ok = pb.dev_mdiis && pb.u16 && pb.r8 && pb.r16 && !pb.noalloc &&
+  // difference form with BF16 or FP8 residuals, the library's own allocations
+  const bool dev_ok = pb.dev_mdiis && pb.u16 && pb.r16 && !pb.noalloc &&
                       cf.precision != RISM3D_FP64;
   bool dev_on = false;          // the FP32 solutes' state is on the device
   std::vector<int> dev_dirty;   // solutes whose host state goes up before the next pass
@@ -1130,14 +1185,21 @@ void iterate_batch(Problem& pb, const Config& cf) {
     m.iters = s.iters;
     m.iters32 = s.iters32;
     m.hold = pb.rebase_wait > 0;
+    m.rbytes = pb.r8 ? 1 : 2;
+    m.period = pb.period;
+    m.skipped = s.skipped;
+    m.pend = s.pend;
+    m.rows = s.rows;
+    m.picard = s.picard;
+    m.low = s.low;
     for (int i = 0; i < m.n; ++i) {
       m.order[i] = s.order[i];
-      m.coef[i] = s.coef[i];
+      m.coef[i] = s.picard ? 0.0 : s.coef[i];
     }
     for (int i = 0; i < m.ndot; ++i) m.dotted[i] = s.dotted[i];
     for (int q = 0; q < D; ++q) {
       m.sbase[q] = s.sbase[q];
-      m.rsc[q] = s.rsc[q];
+      m.rsc[q] = pb.r8 ? s.rsc[q] : 1.f;
       for (int j = 0; j < D; ++j) m.gram[q * MAX_DIIS + j] = s.gram[q * D + j];
     }
     m.resid = s.resid;
@@ -1148,11 +1210,16 @@ void iterate_batch(Problem& pb, const Config& cf) {
     auto& s = pb.st[b];
     s.order.assign(m.order, m.order + m.n);
     s.coef.assign(m.coef, m.coef + m.n);
+    s.skipped = m.skipped;
+    s.pend = m.pend;
+    s.rows = m.rows;
+    s.picard = m.picard;
+    s.low = m.low;
     s.dotted.assign(m.dotted, m.dotted + m.ndot);
     s.slot_new = m.slot_new;
     for (int q = 0; q < D; ++q) {
       s.sbase[q] = m.sbase[q];
-      s.rsc[q] = m.rsc[q];
+      if (pb.r8) s.rsc[q] = m.rsc[q];
       for (int j = 0; j < D; ++j) s.gram[q * D + j] = m.gram[q * MAX_DIIS + j];
     }
     s.since_best = m.since_best;
@@ -1261,7 +1328,19 @@ void iterate_batch(Problem& pb, const Config& cf) {
       d.ncomb = (int)s.coef.size();
       const bool u16 = fp32 && pb.u16;
       auto slotD = [&](int q) { return (void*)((uint16_t*)s.U.p + (size_t)q * mP); };
-      if (u16) {
+      s.talias = -1;
+      if (s.picard && !fp32) {  // t = the newest u, read where it is
+        d.ncomb = 0;
+        s.talias = s.order.back();
+        d.t = slotU(s.talias);
+      } else if (s.picard) {
+        const int q = s.order.back();
+        d.ncomb = 1;
+        d.u16 = d.plain = u16;
+        d.u[0] = u16 ? (void*)s.ucur : slotU(q);
+        d.coef[0] = 1.0;
+        if (!u16 && s.sbase[q] != s.base) d.shift_w = 1.0;
+      } else if (u16) {
         // t = sum_j c_j u_j = u_newest - sum_i (c_0 + .. + c_i) (u_i+1 - u_i),
         // the difference u_i+1 - u_i in the BF16 slot of entry i + 1
         d.u16 = 1;
@@ -1291,14 +1370,28 @@ void iterate_batch(Problem& pb, const Config& cf) {
         s.slot_new = s.order.front();
         s.dotted.erase(s.dotted.begin());
       }
-      d.ndot = (int)s.dotted.size();
-      for (int j = 0; j < d.ndot; ++j) d.rh[j] = slotR(s.dotted[j]);
+      // the Gram rows this pass forms: none at a plain step; its own with the
+      // history; or, after plain steps, theirs and its own by gram_rows.  The
+      // polish after an FP32 phase extrapolates at every pass (few passes).
+      const bool polish = !fp32 && cf.precision != RISM3D_FP64;
+      const int period = s.low <= PULAY_BELOW && !polish ? pb.period : 1;
+      s.rows = s.skipped + 1 >= period ? (s.pend ? 2 : 1) : 0;
+      const int nh = (int)s.dotted.size();
+      d.ndot = s.rows == 1 ? nh : 0;
+      d.ngram = s.rows == 2 ? nh + 1 : 0;
+      d.nrow = s.pend + 1;
+      d.gpart = s.gpart.p;
       if (fp32 && pb.r8) {
         d.r8 = 1;
         d.rsc = fp8_scale(s.resid);
         s.rsc[s.slot_new] = d.rsc;
-        for (int j = 0; j < d.ndot; ++j) d.rhinv[j] = 1.0f / s.rsc[s.dotted[j]];
       }
+      auto hist_entry = [&](int at, int q) {
+        d.rh[at] = slotR(q);
+        if (d.r8) d.rhinv[at] = 1.0f / s.rsc[q];
+      };
+      if (s.rows == 2) hist_entry(0, s.slot_new);
+      for (int j = 0; j < nh; ++j) hist_entry(s.rows == 2 ? nh - j : j, s.dotted[j]);
       d.r = slotR(s.slot_new);
       d.unew = u16 ? (void*)s.ucur : slotU(s.slot_new);
       d.dnew = u16 ? slotD(s.slot_new) : nullptr;
@@ -1403,11 +1496,12 @@ void iterate_batch(Problem& pb, const Config& cf) {
     for (int b = 0; b < B; ++b) {
       auto& s = pb.st[b];
       if (!sd[b].active) continue;
-      const double* o = out.data() + (size_t)b * NPART;
+      const double* o = out.data() + (size_t)b * NOUT;
       const double rinf = o[0], r2 = o[1];
       s.iters++;
       if (fp32) s.iters32++;
       s.resid = rinf;
+      s.low = std::min(s.low, rinf);
       if (cf.verbose)
         std::fprintf(stderr, "rism3d: solute %d iter %d %s |F|inf = %.3e |F|2 = %.3e\n", b, s.iters,
                      fp32 ? "fp32" : "fp64", rinf, std::sqrt(r2));
@@ -1429,7 +1523,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
         // The new entry still enters the history (the rebase moves it).
         // ready (with a rebase wait): the 1e3 drop, or mixed_tol / 2 reached
         const bool drop = !only32 && rinf <= 1e-3 * s.rb_rinf, conv = rinf <= 0.5 * s.tol_mixed;
-        if (s.stall32 >= 12 || s.iters32 >= cf.max_iter || (pb.rebase_wait <= 0 && (drop || conv)) ||
+        if (s.stall32 >= stall_passes(pb.period, s.low) || s.iters32 >= cf.max_iter || (pb.rebase_wait <= 0 && (drop || conv)) ||
             (only32 && conv)) {
           rebase_mask[b] = 1;
           any_rebase = true;
@@ -1463,28 +1557,40 @@ void iterate_batch(Problem& pb, const Config& cf) {
           continue;
         }
       }
-      // enter the new entry, refresh its Gram row
+      // enter the new entry, refresh the Gram rows this pass formed
       s.order = s.dotted;
       s.order.push_back(s.slot_new);
-      for (int j = 0; j < (int)s.dotted.size(); ++j) {
-        s.gram[s.slot_new * D + s.dotted[j]] = o[2 + j];
-        s.gram[s.dotted[j] * D + s.slot_new] = o[2 + j];
-      }
+      const int nd = (int)s.dotted.size();
+      auto pair = [&](int p, int q, double v) { s.gram[p * D + q] = s.gram[q * D + p] = v; };
+      auto entry = [&](int k) { return k == 0 ? s.slot_new : s.dotted[nd - k]; };
+      if (s.rows == 1)
+        for (int j = 0; j < nd; ++j) pair(s.slot_new, s.dotted[j], o[2 + j]);
+      if (s.rows == 2)
+        for (int i = 0; i <= s.pend; ++i)
+          for (int j = i + 1; j <= nd; ++j) pair(entry(i), entry(j), o[2 + i * MAX_DIIS + j]);
       s.gram[s.slot_new * D + s.slot_new] = r2;
       // restart when the residual blows up against the best one, or stalls
       if (r2 < s.best) { s.best = r2; s.since_best = 0; } else { s.since_best++; }
-      if (r2 > 100.0 * s.best || s.since_best > 3 * Dp) {
+      const bool extrap = s.rows != 0;
+      s.pend = extrap ? 0 : s.pend + 1;
+      s.skipped = extrap ? 0 : s.skipped + 1;
+      if (r2 > (extrap ? RESTART_EXTRAP : RESTART_PLAIN) * s.best || s.since_best > 3 * Dp) {
         s.order.assign(1, s.slot_new);
         s.best = r2;
         s.since_best = 0;
+        s.pend = s.skipped = 0;
       }
       const int nh = (int)s.order.size();
+      s.picard = !extrap || nh == 1;
+      s.coef.assign(1, 1.0);
+      if (s.picard) continue;
       std::vector<double> G(nh * nh);
       for (int i = 0; i < nh; ++i)
         for (int j = 0; j < nh; ++j) G[i * nh + j] = s.gram[s.order[i] * D + s.order[j]];
-      if (nh == 1 || !diis_coefficients(G, nh, s.coef)) {
+      if (!diis_coefficients(G, nh, s.coef)) {
         s.order.assign(1, s.slot_new);
         s.coef.assign(1, 1.0);
+        s.picard = 1;
       }
     }
     if (fp32) {
@@ -1496,6 +1602,14 @@ void iterate_batch(Problem& pb, const Config& cf) {
       rebase(pb, cf, rebase_mask, true, rinf, r2);
       after_rebase(rebase_mask, rinf, r2, false);
     }
+  }
+  // solutes whose last pass read t in the history
+  for (int b = 0; b < B; ++b) {
+    auto& s = pb.st[b];
+    if (s.talias >= 0)
+      HIPCHK(hipMemcpyAsync(s.t64.p, s.U.p + (size_t)s.talias * mP, mP * 8,
+                            hipMemcpyDeviceToDevice, pb.s));
+    s.talias = -1;
   }
   // solutes that stopped inside the FP32 phase (NaN): t = t_b + delta
   for (int b = 0; b < B; ++b)
@@ -1517,7 +1631,7 @@ struct OneSolute {
   int b;
   std::vector<SoluteDesc> sd;
   std::vector<double> out;
-  OneSolute(Problem& p, int bb) : pb(p), b(bb), sd(p.B), out((size_t)p.B * NPART) {}
+  OneSolute(Problem& p, int bb) : pb(p), b(bb), sd(p.B), out((size_t)p.B * NOUT) {}
   SoluteDesc& desc() {
     for (auto& d : sd) std::memset(&d, 0, sizeof d);
     auto& s = pb.st[b];
@@ -1535,7 +1649,7 @@ struct OneSolute {
     download_out(pb, out);
     HIPCHK(hipGetLastError());
     pb.st[b].iters++;
-    return {out[(size_t)b * NPART], out[(size_t)b * NPART + 1]};
+    return {out[(size_t)b * NOUT], out[(size_t)b * NOUT + 1]};
   }
   // F at t = u0 + a u1 (ncomb 2) or at t itself (u1 == nullptr) into r;
   // t64 receives the point
@@ -2252,7 +2366,7 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
   s0.W = DevBuf<cpx<double>>((size_t)np * w_points(g));
   s0.part = DevBuf<double>((size_t)pb.nparts * NPART);
   pb.d_sd = DevBuf<SoluteDesc>(1);
-  pb.d_out = DevBuf<double>(NPART);
+  pb.d_out = DevBuf<double>(NOUT);
   if (t_init)
     host_copies({{const_cast<double*>(t_init), s0.t64.p, (size_t)pb.mP * 8}}, false);
   else
@@ -2382,6 +2496,7 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
   // iterates t itself to its floor, where the Gram rounding would show
   if (in.opt.precision != RISM3D_MIXED) pb.r16 = 0;
   if (!pb.r16) pb.u16 = 0;
+  if (pb.r8 < 0) pb.r8 = pb.pulay > 1 && pb.D >= PULAY_DEPTH ? 0 : 1;
   if (!pb.r16) pb.r8 = 0;
   for (int d = 0; d < 3; ++d) { pb.N[d] = pd.N[d]; pb.L[d] = pd.L[d]; pb.h[d] = pd.L[d] / pd.N[d]; }
   GridArgs& g = pb.g;
@@ -2492,7 +2607,7 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
       HIPCHK(hipMemsetAsync(s.t64.p, 0, pb.mP * 8, pb.s));
   }
   pb.d_sd = DevBuf<SoluteDesc>(B);
-  pb.d_out = DevBuf<double>((size_t)B * NPART);
+  pb.d_out = DevBuf<double>((size_t)B * NOUT);
   pb.d_cdst = DevBuf<void*>(B);
   pb.d_csrc = DevBuf<void*>(B);
   pb.d_cmask = DevBuf<int>(B);
@@ -2879,7 +2994,7 @@ size_t noalloc_bytes(const rism3d_problem& pd, int m, int n, bool mixed) {
   b += 4 * al(mP * 8) + al(m * Kw * 16) + al(Kw * 16);  // U, R, t, beta v; W; F s
   if (mixed) b += 4 * al(mP * 4) + al(mP * 8) + al(Kw * 8);
   b += al(N1 * N2 * m * NPART * 8) + al((size_t)std::max(n, 0) * 6 * 8);
-  b += al(sizeof(SoluteDesc)) + al(sizeof(SitesDesc)) + al(NPART * 8) + 3 * al(8);
+  b += al(sizeof(SoluteDesc)) + al(sizeof(SitesDesc)) + al(NOUT * 8) + 3 * al(8);
   b += al(3 * (size_t)m * 8) + 4 * al(8);  // setup descriptors
   return b;
 }

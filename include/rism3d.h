@@ -102,7 +102,8 @@ enum rism3d_precision {
                                every rebase, then polish_iters FP64 steps;
                                no FP32 floor.  The FP32 MDIIS history is
                                kept as the newest u in FP32, BF16
-                               differences of u and FP8 residuals;
+                               differences of u and BF16 residuals (FP8
+                               where every pass extrapolates: depth < 5);
                                solutes ready for a rebase wait for one
                                another (grouped FP64 passes)             */
   RISM3D_FP32 = 2           /* FP32 passes only, around the starting
