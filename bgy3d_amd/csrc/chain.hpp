@@ -405,7 +405,7 @@ __device__ void oz_pairs(cpx<T>* __restrict__ lds, const GridArgs& g, const T* _
       const double im = (double)c.im * g.h3 * sgn;
       Cr[i][j] = Cr[j][i] = re;
       Ci[i][j] = Ci[j][i] = im;
-      Wm[i][j] = Wm[j][i] = (i == j) ? 1.0 : (double)chi3[p * g.K + kk];
+      Wm[i][j] = Wm[j][i] = (i == j) ? 1.0 : (double)chi3[p * g.KT + kk];
     }
   // WC, A = 1 - rho WC, B = WC W
   double WCr[MSX][MSX], WCi[MSX][MSX], Ar[MSX][MSX], Ai[MSX][MSX], Br[MSX][MSX],
@@ -486,8 +486,8 @@ __device__ void oz_pairs(cpx<T>* __restrict__ lds, const GridArgs& g, const T* _
 // tile), y = ceil(NH / LINES), z = ky row; zorder 1: x = kx tile, y = ky
 // row, z = solute (concurrent workgroups stream contiguous planes of one
 // solute).  Dynamic LDS:
-// m * LINES * lstride_for(N2) complex.  chi3: [m(m+1)/2][K] chi_ij - delta_ij;
-// tau3: [m][K] s_i(|k|), both on the k grid, in the working type.
+// m * LINES * lstride_for(N2) complex.  chi3: [m(m+1)/2][KT] chi_ij - delta_ij;
+// tau3: [m][KT] s_i(|k|), both on the k grid (table_index), in the working type.
 template <typename T, int N2, int LINES>
 __global__ void __launch_bounds__(NT)
 zstar(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ tw,
@@ -536,7 +536,7 @@ zstar(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ 
     for (int e = threadIdx.x; e < N2 * LINES; e += NT) {
       const int z = e / LINES, l = e - z * LINES;
       if (kx0 + l >= g.NX) continue;
-      const int64_t kk = base + z * zs + l;
+      const int64_t kk = table_index(g, z, y, kx0 + l);
       const int iz = (z <= N2 / 2) ? z : z - N2;
       const int ix = kx0 + l;
       const double sgn = ((ix + iy + iz) & 1) ? -1.0 : 1.0;
@@ -571,7 +571,7 @@ zstar(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ 
   for (int e = threadIdx.x; e < N2 * LINES; e += NT) {
     const int z = e / LINES, l = e - z * LINES;
     if (kx0 + l >= g.NX) continue;
-    const int64_t kk = base + z * zs + l;   // k-grid index of this point
+    const int64_t kk = table_index(g, z, y, kx0 + l);  // this point in the tables
     const cpx<T> fs = Fs[fs_index<T>(g, z, y, kx0 + l)];
     cpx<T> c[MAX_SITES];
     for (int s = 0; s < m; ++s) c[s] = lds[(s * LINES + l) * LS + lpos(z)];
@@ -593,7 +593,7 @@ zstar(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ 
       cpx<T> acc = {T(0), T(0)};
       for (int j = 0; j < m; ++j) {  // sum_j S_ij sig_j c_j / sig_i (sig = 1: one density)
         const int pi_ = (i >= j) ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i;
-        const T chi = chi3[pi_ * g.K + kk] * T(g.sig[j]);
+        const T chi = chi3[pi_ * g.KT + kk] * T(g.sig[j]);
         acc.re += chi * c[j].re;
         acc.im += chi * c[j].im;
       }
@@ -603,7 +603,7 @@ zstar(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ 
         out = cscale(acc, T(g.a_scale));
       } else if (g.renorm) {
         // (h^3/L^3) sum_j chi_ij C_j - (beta/eps0/L^3) tau_i F s  (hnc3d.c:1245-1268)
-        const T tau = tau3[i * g.K + kk] * T(g.tau_scale);
+        const T tau = tau3[i * g.KT + kk] * T(g.tau_scale);
         out = csub(cscale(acc, T(g.a_scale)), cscale(fs, tau));
       } else {
         out = cscale(csub(acc, cscale(uc, T(g.beta * g.q[i]))), T(g.inv_L3));
@@ -764,12 +764,14 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
   // zorder 2: consecutive blocks go to the XCDs in
   // turn, and each XCD walks all solutes of one (ky, kx tile) before the
   // next, so the tile's chi and tau stay in that XCD's L2 for every solute.
-  // zorder 3: XCD x owns the rows ky = x (mod 8) and walks every
+  // zorder 3: XCD x owns the row pairs ky, N1 - ky with ky = x (mod 8), which
+  // share their tables (143 -> 141 us at 192^3 with 5 sites, 26 -> 25.4 at 96^3
+  // in FP64, against rows in order), and walks every
   // solute of a row, the row's kx tiles back to back, so each z line's
   // columns are read by neighbouring workgroups at once (whole rows of the
   // z planes instead of one tile's 128 bytes) and the row's chi and tau
   // stay in the XCD's L2 across solutes.
-  // zorder 1: kx tile fastest, then ky, then the solute; zorder 0: solute
+  // zorder 1: kx tile fastest, then ky (in the same pairs), then the solute; zorder 0: solute
   // fastest, then the kx tile.
   int b, tile, ky;
   const int nnyq = g.nyqb * g.zB;
@@ -783,7 +785,8 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
     if (g.zorder == 3) {
       tile = slot % g.ztiles;
       b = (slot / g.ztiles) % g.zB;
-      ky = (slot / (g.ztiles * g.zB)) * 8 + xcd;
+      const int q = slot / (g.ztiles * g.zB), p = (q >> 1) * 8 + xcd;
+      ky = q & 1 ? (p ? g.N1 - p : g.N1 / 2) : p;
     } else if (g.zorder == 2) {
       const int gt = (slot / g.zB) * 8 + xcd;  // global tile, ky-major
       b = slot - (slot / g.zB) * g.zB;
@@ -791,7 +794,8 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
       ky = gt / g.ztiles;
     } else if (g.zorder == 1) {
       tile = lin % g.ztiles;
-      ky = (lin / g.ztiles) % g.N1;
+      const int q = (lin / g.ztiles) % g.N1;
+      ky = q & 1 ? g.N1 - (q + 1) / 2 : q / 2;
       b = lin / (g.ztiles * g.N1);
     } else {
       b = lin % g.zB;
@@ -807,7 +811,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
   const int kx0 = nyq ? g.NX - 1 : tile * LINES;
   // element offsets below 2^32 bytes from per-workgroup bases (at32): the
   // tables and Fs from their starts, W from its site's
-  const int zs = g.N1 * g.NH;         // z stride (Fs, chi, tau)
+  const int zs = g.N1 * g.NH;         // z stride
   const int ls = nyq ? g.NH : 1;      // line stride
   const int base = y * g.NH + kx0;
   // W: the same index unless ylay (y-major rows, compact Nyquist column)
@@ -826,14 +830,18 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
     }
   }
   // the tables: z-major rows, and the Nyquist column of each compact behind
-  // them all, (z, ky) at z N1 + ky, where a Nyquist block's lines are
+  // them all, (z, ky) at z TN1 + ky, where a Nyquist block's lines are
   // contiguous (8 bytes of each 128-byte line otherwise: at B = 1 such a
   // block was the pass's last, 50 us against 33 for the rows at 96^3 in FP64)
   constexpr int NTAB = OZ > 0 ? MS : MS * (MS + 1) / 2;  // chi3's tables
-  const int64_t tsite = nyq ? (int64_t)g.N1 * g.N2 : g.K;
-  const T* chit = nyq ? chi3 + NTAB * g.K : chi3;
-  const T* taut = nyq ? tau3 + MS * g.K : tau3;
-  const int tbase = nyq ? y : base, tz = nyq ? g.N1 : zs;
+  const int64_t tsite = nyq ? (int64_t)g.TN1 * g.TN2 : g.KT;
+  const T* chit = nyq ? chi3 + NTAB * g.KT : chi3;
+  const T* taut = nyq ? tau3 + MS * g.KT : tau3;
+  const int tbase = nyq ? 0 : table_row(g, y) * g.NH + kx0, tz = nyq ? g.TN1 : g.TN1 * g.NH;
+  // point (z, l) of the tile in the tables
+  auto tpoint = [&](int z, int l) {
+    return (uint32_t)(tbase + table_plane(g, z) * tz + (nyq ? table_row(g, y + l) : l));
+  };
   const int nl = nyq ? min(LINES, g.N1 - y)  // valid lines
                      : min(LINES, (g.nyqb ? g.NX - 1 : g.NX) - kx0);
   const int tid = threadIdx.x;
@@ -906,7 +914,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
       const int e = tid + p * NTZ;
       const int z = e / LINES, l = e - z * LINES;
       if (d.mode == 4 || !(PPT * NTZ == PTS || e < PTS) || l >= nl) continue;
-      const uint32_t kk = (uint32_t)(tbase + z * tz + l);
+      const uint32_t kk = tpoint(z, l);
       const int iz = (z <= N2 / 2) ? z : z - N2, ix = nyq ? kx0 : kx0 + l;
       const int yl = nyq ? y + l : y;
       const int iy = (yl <= g.N1 / 2) ? yl : yl - g.N1;
@@ -937,7 +945,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
     if (d.mode == 4 || !(PPT * NTZ == PTS || e < PTS)) continue;
     const int z = e / LINES, l = e - z * LINES;
     if (l >= nl) continue;
-    const uint32_t kk = (uint32_t)(tbase + z * tz + l);  // this point in the tables
+    const uint32_t kk = tpoint(z, l);  // this point in the tables
     cpx<T> fs = {T(0), T(0)};
     if (!linear)
       fs = ldc(at32(Fs, nyq ? (uint32_t)(g.K + z * g.N1 + y + l)

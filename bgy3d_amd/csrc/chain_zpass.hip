@@ -33,7 +33,7 @@ void launch_zreg_n(int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd, c
   const int tiles = (split ? NX - 1 + L - 1 : NX + L - 1) / L;
   GridArgs gz = g;
   if (gz.zorder == 2 && (tiles * N1) % 8 != 0) gz.zorder = 1;  // whole tiles per XCD
-  if (gz.zorder == 3 && N1 % 8 != 0) gz.zorder = 1;             // whole rows per XCD
+  if (gz.zorder == 3 && N1 % 16 != 0) gz.zorder = 1;            // whole row pairs per XCD
   gz.zB = B;
   gz.ztiles = tiles;
   gz.nyqb = split ? (N1 + L - 1) / L : 0;

@@ -48,45 +48,44 @@ __device__ __forceinline__ double interp_eval(const Interp& a, const double* __r
 
 // chi_ij(|k|) - delta_ij and tau_i(|k|) on the 3D k grid, once per batch
 // (solute independent; solvent_kernel_rism hnc3d.c:1443-1566 tabulates
-// them the same way with vec_ktab).  Grid: x = chunks of K.  Writes FP64
-// and, unless null, FP32 copies, [npairs][K] and [m][K].
+// them the same way with vec_ktab), at ky <= N1/2, kz <= N2/2 (table_index).
+// Grid: x = chunks of KT.  Writes FP64 and, unless null, FP32 copies,
+// [npairs][KT] and [m][KT].
 __global__ void __launch_bounds__(NT)
 ktab3(GridArgs g, const double* __restrict__ chi_tab, const double* __restrict__ tau_tab,
       double* __restrict__ chi3, float* __restrict__ chi3f, double* __restrict__ tau3,
       float* __restrict__ tau3f) {
   const int np = g.m * (g.m + 1) / 2;
   const int64_t stride = (int64_t)gridDim.x * NT;
-  for (int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x; e < g.K; e += stride) {
+  for (int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x; e < g.KT; e += stride) {
     const int x = (int)(e % g.NH);
     if (x >= g.NX) continue;  // row padding
-    const int y = (int)((e / g.NH) % g.N1);
-    const int z = (int)(e / ((int64_t)g.NH * g.N1));
-    const int iy = (y <= g.N1 / 2) ? y : y - g.N1;
-    const int iz = (z <= g.N2 / 2) ? z : z - g.N2;
-    const double k2 = kmag2(x * g.dkx, iy * g.dky, iz * g.dkz);
+    const int y = (int)((e / g.NH) % g.TN1);
+    const int z = (int)(e / ((int64_t)g.NH * g.TN1));
+    const double k2 = kmag2(x * g.dkx, y * g.dky, z * g.dkz);
     const Interp ip = interp_at(sqrt(k2), g.dk_tab, g.nrad);
     for (int p = 0; p < np; ++p) {
       const double v = interp_eval(ip, chi_tab + (int64_t)p * g.nrad);
-      chi3[p * g.K + e] = v;
-      if (chi3f) chi3f[p * g.K + e] = (float)v;
+      chi3[p * g.KT + e] = v;
+      if (chi3f) chi3f[p * g.KT + e] = (float)v;
     }
     for (int i = 0; i < g.m; ++i) {
       const double v = interp_eval(ip, tau_tab + (int64_t)i * g.nrad);
-      tau3[i * g.K + e] = v;
-      if (tau3f) tau3f[i * g.K + e] = (float)v;
+      tau3[i * g.KT + e] = v;
+      if (tau3f) tau3f[i * g.KT + e] = (float)v;
     }
   }
 }
 
-// The Nyquist column kx = N0/2 of n tables [n][K] once more behind them,
-// [n][N2][N1], as the z pass's Nyquist blocks read it.  Grid: x = chunks of
-// N1 N2, y = table.
+// The Nyquist column kx = N0/2 of n tables [n][KT] once more behind them,
+// [n][TN2][TN1], as the z pass's Nyquist blocks read it.  Grid: x = chunks of
+// TN1 TN2, y = table.
 template <typename T>
 __global__ void __launch_bounds__(NT)
 nyq_tables(GridArgs g, T* __restrict__ tab) {
-  const int64_t n12 = (int64_t)g.N1 * g.N2;
-  const T* src = tab + blockIdx.y * g.K + (g.NX - 1);
-  T* dst = tab + gridDim.y * g.K + blockIdx.y * n12;
+  const int64_t n12 = (int64_t)g.TN1 * g.TN2;
+  const T* src = tab + blockIdx.y * g.KT + (g.NX - 1);
+  T* dst = tab + gridDim.y * g.KT + blockIdx.y * n12;
   for (int64_t j = blockIdx.x * (int64_t)NT + threadIdx.x; j < n12; j += (int64_t)gridDim.x * NT)
     dst[j] = src[j * g.NH];
 }
@@ -1043,11 +1042,12 @@ grad_tau(GridArgs g, SitesDesc sd, const cpx<double>* __restrict__ Lam,
       const cpx<double> L = Lam[i * g.K + e];
       double ti;
       if (g.renorm) {
-        ti = tau3[i * g.K + e];
+        ti = tau3[i * g.KT + table_index(g, z, y, x)];
       } else {
         double w = g.q[i];
         for (int j = 0; j < g.m; ++j)
-          w += chi3[(int64_t)((i >= j) ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i) * g.K + e] *
+          w += chi3[(int64_t)((i >= j) ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i) * g.KT +
+                    table_index(g, z, y, x)] *
                g.q[j];
         ti = shape * w;
       }
@@ -1192,16 +1192,14 @@ __global__ void __launch_bounds__(NT)
 omega3(GridArgs g, double L0, const double* __restrict__ rij, double* __restrict__ w) {
   const int p = blockIdx.y;
   const int64_t stride = (int64_t)gridDim.x * NT;
-  for (int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x; e < g.K; e += stride) {
+  for (int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x; e < g.KT; e += stride) {
     const int x = (int)(e % g.NH);
     if (x >= g.NX) continue;
-    const int y = (int)((e / g.NH) % g.N1);
-    const int z = (int)(e / ((int64_t)g.NH * g.N1));
-    const int iy = (y <= g.N1 / 2) ? y : y - g.N1;
-    const int iz = (z <= g.N2 / 2) ? z : z - g.N2;
-    const int k2 = iz * iz + iy * iy + x * x;
+    const int y = (int)((e / g.NH) % g.TN1);
+    const int z = (int)(e / ((int64_t)g.NH * g.TN1));
+    const int k2 = z * z + y * y + x * x;
     const double kr = (2.0 * M_PI * rij[p] / L0) * sqrt((double)k2);
-    w[p * g.K + e] = (kr == 0.0) ? 1.0 : sin(kr) / kr;
+    w[p * g.KT + e] = (kr == 0.0) ? 1.0 : sin(kr) / kr;
   }
 }
 
@@ -1278,7 +1276,7 @@ chi_from_h(GridArgs g, const cpx<double>* __restrict__ W, const double* __restri
     const double sgn = ((x + iy + iz) & 1) ? -1.0 : 1.0;
     const cpx<double> wv = W[p * g.K + e];
     double re = wv.re * g.h3 * sgn, im = wv.im * g.h3 * sgn;
-    if (i != j) re += omega[p * g.K + e];
+    if (i != j) re += omega[p * g.KT + table_index(g, z, y, x)];
     const int64_t o = p * Kv + ((int64_t)z * g.N1 + y) * g.NX + x;
     out[2 * o] = re;
     out[2 * o + 1] = im;

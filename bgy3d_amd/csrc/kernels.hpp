@@ -188,6 +188,17 @@ struct GridArgs {
   // units).  0: W is z-major like the tables, [site][z][ky][NH].
   int ylay;
   int nyqb;            // z pass: Nyquist blocks per solute (0: in the last tile)
+  // The k tables (chi - delta, tau, omega): functions of |k|, held for ky <=
+  // N1/2 and kz <= N2/2 only, [TN2][TN1][NH] of KT points each, the point of
+  // row y and plane z at min(y, mir1 - y), min(z, mir2 - z).  For one solute
+  // the whole tables were up to half of the z pass's traffic (290 of 610 MB at
+  // 192^3 with 5 sites in FP32); now each entry serves two planes from L1 and
+  // two rows from L2 (zstar_reg walks y and N1 - y together): 182 -> 141 us
+  // there, 28 -> 25 at 96^3 in FP64 with 3 sites, 306 -> 282 for 24 x 128^3.
+  // A 3D table from outside need not be even in ky and kz: it is held whole
+  // (TN = N, mir far beyond).
+  int TN1, TN2, mir1, mir2;
+  int64_t KT;
   double q[MAX_SITES]; // solvent charges
   // zstar variants (0 solute residual): 1 solvent-solvent OZ on site-site
   // pairs (msol sites, pair p = i(i+1)/2 + j), 2 Poisson potential of a
@@ -201,6 +212,19 @@ struct GridArgs {
   double sig[MAX_SITES];
   double rw[MAX_SITES];
 };
+
+__host__ __device__ inline void set_tables(GridArgs& g, bool whole) {
+  g.TN1 = whole ? g.N1 : g.N1 / 2 + 1;
+  g.TN2 = whole ? g.N2 : g.N2 / 2 + 1;
+  g.mir1 = whole ? 1 << 30 : g.N1;
+  g.mir2 = whole ? 1 << 30 : g.N2;
+  g.KT = (int64_t)g.NH * g.TN1 * g.TN2;
+}
+__device__ __forceinline__ int table_row(const GridArgs& g, int y) { return min(y, g.mir1 - y); }
+__device__ __forceinline__ int table_plane(const GridArgs& g, int z) { return min(z, g.mir2 - z); }
+__device__ __forceinline__ int64_t table_index(const GridArgs& g, int z, int y, int x) {
+  return ((int64_t)table_plane(g, z) * g.TN1 + table_row(g, y)) * g.NH + x;
+}
 
 // Solute sites for the setup and mu kernels, per solute.
 struct SitesDesc {

@@ -579,8 +579,10 @@ int resid_grid_x(const GridArgs& g) {
 // Points of a spectrum or table with the Nyquist column apart: the rows and
 // that column, compact.
 int64_t w_points(const GridArgs& g) { return g.K + (int64_t)g.N1 * g.N2; }
+// Points of a k table: KT and its Nyquist column once more (nyq_tables)
+int64_t t_points(const GridArgs& g) { return g.KT + (int64_t)g.TN1 * g.TN2; }
 dim3 nyq_grid(const GridArgs& g, int tables) {
-  return dim3((unsigned)std::min<int64_t>(1024, ((int64_t)g.N1 * g.N2 + NT - 1) / NT), tables);
+  return dim3((unsigned)std::min<int64_t>(1024, ((int64_t)g.TN1 * g.TN2 + NT - 1) / NT), tables);
 }
 
 // History slots the closure and residual kernels must unroll for this batch.
@@ -2317,6 +2319,7 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
   g.msol = m;
   g.P = (int64_t)g.N0 * g.N1 * g.N2;
   g.K = (int64_t)g.NH * g.N1 * g.N2;
+  set_tables(g, false);
   g.dkx = 2 * M_PI / pd->L[0]; g.dky = 2 * M_PI / pd->L[1]; g.dkz = 2 * M_PI / pd->L[2];
   const double h3 = pb.h[0] * pb.h[1] * pb.h[2];
   const double L3 = pd->L[0] * pd->L[1] * pd->L[2];
@@ -2340,7 +2343,7 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
   make_twiddles(pb.tw, pb.N, pb.s, false);
 
   // omega_ij(k) in the chi3 slots of the pairs
-  pb.chi3 = DevBuf<double>((size_t)np * w_points(g));
+  pb.chi3 = DevBuf<double>((size_t)np * t_points(g));
   {
     std::vector<double> rij(np, 0.0);
     for (int i = 0; i < m; ++i)
@@ -2351,7 +2354,7 @@ int solvent_run(const rism3d_problem* pd, int m, const rism3d_site* solvent,
       }
     DevBuf<double> d_rij(np);
     HIPCHK(hipMemcpyWithStream(d_rij.p, rij.data(), np * 8, hipMemcpyHostToDevice, pb.s));
-    const int ck = (int)std::min<int64_t>(4096, (g.K + NT - 1) / NT);
+    const int ck = (int)std::min<int64_t>(4096, (g.KT + NT - 1) / NT);
     hipLaunchKernelGGL(omega3, dim3(ck, np), dim3(NT), 0, pb.s, g, pd->L[0], d_rij.p, pb.chi3.p);
     hipLaunchKernelGGL(nyq_tables<double>, nyq_grid(g, np), dim3(NT), 0, pb.s, g, pb.chi3.p);
     HIPCHK(hipStreamSynchronize(pb.s));
@@ -2517,6 +2520,7 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
   g.nrad = pd.nrad;
   g.P = (int64_t)g.N0 * g.N1 * g.N2;
   g.K = (int64_t)g.NH * g.N1 * g.N2;
+  set_tables(g, in.opt.chi3d != nullptr);
   g.dkx = 2 * M_PI / pd.L[0]; g.dky = 2 * M_PI / pd.L[1]; g.dkz = 2 * M_PI / pd.L[2];
   g.dk_tab = M_PI / pd.rmax;
   const double h3 = pb.h[0] * pb.h[1] * pb.h[2];
@@ -2554,11 +2558,11 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
   const int m = in.m, nrad = pd.nrad;
   const size_t np = (size_t)m * (m + 1) / 2;
   const bool f32 = pb.mixed != 0;  // the FP32 chain's copies
-  pb.chi3 = DevBuf<double>(np * w_points(g));
-  pb.tau3 = DevBuf<double>((size_t)m * w_points(g));
+  pb.chi3 = DevBuf<double>(np * t_points(g));
+  pb.tau3 = DevBuf<double>((size_t)m * t_points(g));
   if (f32) {
-    pb.chi3f = DevBuf<float>(np * w_points(g));
-    pb.tau3f = DevBuf<float>((size_t)m * w_points(g));
+    pb.chi3f = DevBuf<float>(np * t_points(g));
+    pb.tau3f = DevBuf<float>((size_t)m * t_points(g));
   }
   if (in.opt.chi3d) {
     // --solvent-3d: chi - 1 of a 3D solvent solve on this grid
@@ -2686,7 +2690,8 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
     const int cp = (int)std::min<int64_t>(4096, (g.P + NT - 1) / NT);
     const int ck = (int)std::min<int64_t>(4096, (g.K + NT - 1) / NT);
     if (tabs) {
-      hipLaunchKernelGGL(ktab3, dim3(ck), dim3(NT), 0, pb.s, g, at(o_chi), at(o_tau), pb.chi3.p,
+      const int ckt = (int)std::min<int64_t>(4096, (g.KT + NT - 1) / NT);
+      hipLaunchKernelGGL(ktab3, dim3(ckt), dim3(NT), 0, pb.s, g, at(o_chi), at(o_tau), pb.chi3.p,
                          pb.chi3f.p, pb.tau3.p, pb.tau3f.p);
       hipLaunchKernelGGL(nyq_tables<double>, nyq_grid(g, m), dim3(NT), 0, pb.s, g, pb.tau3.p);
       if (f32) hipLaunchKernelGGL(nyq_tables<float>, nyq_grid(g, m), dim3(NT), 0, pb.s, g, pb.tau3f.p);
