@@ -590,30 +590,37 @@ __device__ __forceinline__ double cl0(double r) {
 // beta v_i(r) for every solvent site (field0, bgy3d-solutes.c:344-377).
 // Grid: x = chunks of P, y = solute.  Writes FP64 and, if bv32 != NULL,
 // an FP32 copy for the mixed-precision bulk iterations.  The solute sites
-// pass through LDS in chunks of FB_CHUNK (position, sigma, sqrt(epsilon),
-// charge / eps0); per point and site one r^2, 1 / r^2, r and the capped
-// erfc(G r) / r (within G r < 6.5), then per solvent site the Lorentz-Berthelot pair
-// (epsilon_ai = sqrt(eps_a) sqrt(eps_i), sigma_ai = (sigma_a + sigma_i) / 2)
-// with (sigma_ai / r)^6 from 1 / r^2: ljcap0(r / sigma_ai) without a
-// division or square root in the pair loop.
-constexpr int FB_CHUNK = 256;
+// pass through LDS in chunks of FB_CHUNK: position, G charge / eps0 and, per
+// solvent site, sigma_ai^2 and 4 epsilon_ai of the Lorentz-Berthelot pair
+// (epsilon_ai = sqrt(eps_a) sqrt(eps_i), sigma_ai = (sigma_a + sigma_i) / 2).
+// Per point and site one r^2, 1 / r^2, r and the capped erfc(G r) / r (within
+// G r < 6.5), then per solvent site (sigma_ai / r)^6 from 1 / r^2:
+// ljcap0(r / sigma_ai) without a division or square root in the pair loop.
+// Bound by FP64 arithmetic and its latencies: a thread takes FB_PTS points
+// side by side in x, whose divisions overlap and which share the site's LDS
+// reads and y, z terms, and one test tells whether any pair is inside its cap.
+// Four waves per SIMD are worth 20 bytes of spill (218 -> 205 us).  One point
+// a thread and pair parameters formed per point took 318 us for 30 sites on
+// 128^3 (now 205) and 2744 us for 5 solvent sites on 192^3 (now 1282).
+constexpr int FB_CHUNK = 128, FB_PTS = 2;
 constexpr double FB_RC2 = (6.5 / G_COULOMB) * (6.5 / G_COULOMB);
 // MS: the solvent-site arrays' size (>= g.m), so that water's three fit
 // in few registers.
 template <int MS>
-__global__ void __launch_bounds__(NT)
+__global__ void __launch_bounds__(NT, 4)
 field_bv(const SitesDesc* __restrict__ sites, GridArgs g, const double* __restrict__ solvent_sse,
          double L0, double L1, double L2, double h0, double h1, double h2,
          double* const* __restrict__ bv64, float* const* __restrict__ bv32) {
-  __shared__ double st[FB_CHUNK][6];
+  struct Site {
+    double x, y, z, qg, top;   // top: the largest sigma_ai^2
+    double sab2[MS], e4[MS];
+  };
+  __shared__ Site st[FB_CHUNK];
   const SitesDesc sd = sites[blockIdx.y];
   const int m = g.m;
-  double ssig[MS], sse[MS], sq[MS];
-  for (int i = 0; i < m; ++i) {
-    ssig[i] = solvent_sse[3 * i];
-    sse[i] = sqrt(solvent_sse[3 * i + 1]);
-    sq[i] = solvent_sse[3 * i + 2];
-  }
+  double sq[MS];
+#pragma unroll
+  for (int i = 0; i < MS; ++i) sq[i] = i < m ? solvent_sse[3 * i + 2] : 0.0;
   // ljcap0 below r = 0.2 sigma: a + b (x^2 - 0.04), x = r / sigma
   const double R = 0.2, cap_a = lj0(R), cap_b = lj1(R) / (2 * R);
   const int nch = (sd.n + FB_CHUNK - 1) / FB_CHUNK;
@@ -622,29 +629,43 @@ field_bv(const SitesDesc* __restrict__ sites, GridArgs g, const double* __restri
       const int a = c * FB_CHUNK + k;
       if (a >= sd.n) break;
       const double* s = sd.xyz_s_e_q + 6 * a;
-      st[k][0] = s[0];
-      st[k][1] = s[1];
-      st[k][2] = s[2];
-      st[k][3] = s[3];
-      st[k][4] = sqrt(s[4]);
-      st[k][5] = s[5] * EPSILON0INV;
+      Site& t = st[k];
+      t.x = s[0];
+      t.y = s[1];
+      t.z = s[2];
+      t.qg = s[5] * EPSILON0INV * G_COULOMB;
+      t.top = 0.0;
+      const double se = sqrt(s[4]);
+#pragma unroll
+      for (int i = 0; i < MS; ++i) {
+        if (i >= m) continue;
+        const double sab = 0.5 * (s[3] + solvent_sse[3 * i]);
+        t.sab2[i] = sab * sab;
+        t.e4[i] = 4 * (se * sqrt(solvent_sse[3 * i + 1]));
+        t.top = fmax(t.top, t.sab2[i]);
+      }
     }
   };
   if (nch == 1) {
     load(0);
     __syncthreads();
   }
-  const int64_t stride = (int64_t)gridDim.x * NT;
-  // rounds of NT points, the same count in every thread (LDS reloads)
-  for (int64_t e0 = blockIdx.x * (int64_t)NT; e0 < g.P; e0 += stride) {
-    const int64_t e = e0 + threadIdx.x;
+  const int64_t stride = (int64_t)gridDim.x * NT, np = g.P / FB_PTS;  // N0 is even
+  // rounds of NT threads, the same count in every thread (LDS reloads)
+  for (int64_t e0 = blockIdx.x * (int64_t)NT; e0 < np; e0 += stride) {
+    const int64_t e = (e0 + threadIdx.x) * FB_PTS;
     const bool ok = e < g.P;
     const int x = (int)(e % g.N0);
     const int y = (int)((e / g.N0) % g.N1);
     const int z = (int)(e / ((int64_t)g.N0 * g.N1));
-    const double rx = x * h0 - L0 / 2, ry = y * h1 - L1 / 2, rz = z * h2 - L2 / 2;
-    double v[MS];
-    for (int i = 0; i < m; ++i) v[i] = 0.0;
+    const double ry = y * h1 - L1 / 2, rz = z * h2 - L2 / 2;
+    double rx[FB_PTS], v[MS][FB_PTS];
+#pragma unroll
+    for (int p = 0; p < FB_PTS; ++p) {
+      rx[p] = (x + p) * h0 - L0 / 2;
+#pragma unroll
+      for (int i = 0; i < MS; ++i) v[i][p] = 0.0;
+    }
     for (int c = 0; c < nch; ++c) {
       if (nch > 1) {
         __syncthreads();
@@ -654,33 +675,48 @@ field_bv(const SitesDesc* __restrict__ sites, GridArgs g, const double* __restri
       const int na = min(FB_CHUNK, sd.n - c * FB_CHUNK);
       if (!ok) continue;
       for (int k = 0; k < na; ++k) {
-        const double dx = rx - st[k][0], dy = ry - st[k][1], dz = rz - st[k][2];
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        const double ir2 = 1.0 / r2;
+        const Site& s = st[k];
+        const double dy = ry - s.y, dz = rz - s.z;
+        const double dyz = dy * dy + dz * dz;
+        double r2[FB_PTS], ir2[FB_PTS], csc[FB_PTS];
+        bool capped = false;
+#pragma unroll
+        for (int p = 0; p < FB_PTS; ++p) {
+          const double dx = rx[p] - s.x;
+          r2[p] = dx * dx + dyz;
+          ir2[p] = 1.0 / r2[p];
+          capped |= !(s.top * ir2[p] <= 25.0);  // r = 0 gives infinity, or NaN with sigma 0
+        }
         // erfc(G r) / r vanishes beyond G r = 6.5 (erfc(6.5) = 3.8e-20: the
         // term is below 2e-18 kcal/mol there, under the rounding of v)
-        const double csc =
-            r2 < FB_RC2 ? st[k][5] * G_COULOMB * cscap0(G_COULOMB * sqrt(r2)) : 0.0;
-        for (int i = 0; i < m; ++i) {
-          const double sab = 0.5 * (st[k][3] + ssig[i]);
-          const double sab2 = sab * sab;
-          const double s2 = sab2 * ir2;  // (sigma_ai / r)^2
-          double lj;
-          if (s2 <= 25.0) {
+#pragma unroll
+        for (int p = 0; p < FB_PTS; ++p)
+          csc[p] = r2[p] < FB_RC2 ? s.qg * cscap0(G_COULOMB * sqrt(r2[p])) : 0.0;
+#pragma unroll
+        for (int i = 0; i < MS; ++i) {
+          if (i >= m) continue;
+#pragma unroll
+          for (int p = 0; p < FB_PTS; ++p) {
+            const double s2 = s.sab2[i] * ir2[p];  // (sigma_ai / r)^2
             const double p6 = s2 * s2 * s2;
-            lj = 4 * p6 * (p6 - 1);
-          } else {
-            lj = cap_a + cap_b * (r2 / sab2 - R * R);
+            double lj = s.e4[i] * (p6 * (p6 - 1));
+            if (capped && !(s2 <= 25.0))
+              lj = 0.25 * s.e4[i] * (cap_a + cap_b * (r2[p] / s.sab2[i] - R * R));
+            v[i][p] += lj + sq[i] * csc[p];
           }
-          v[i] += st[k][4] * sse[i] * lj + sq[i] * csc;
         }
       }
     }
     if (!ok) continue;
-    for (int i = 0; i < m; ++i) {
-      const double b = g.beta * v[i];
-      bv64[blockIdx.y][i * g.P + e] = b;
-      if (bv32) bv32[blockIdx.y][i * g.P + e] = (float)b;
+#pragma unroll
+    for (int i = 0; i < MS; ++i) {
+      if (i >= m) continue;
+#pragma unroll
+      for (int p = 0; p < FB_PTS; ++p) {
+        const double b = g.beta * v[i][p];
+        bv64[blockIdx.y][i * g.P + e + p] = b;
+        if (bv32) bv32[blockIdx.y][i * g.P + e + p] = (float)b;
+      }
     }
   }
 }
@@ -726,34 +762,70 @@ spec_upsample(const cpx<double>* __restrict__ wc, cpx<double>* __restrict__ wf, 
 
 // F(k) s(k) = s(k) sum_a Q_a exp(-i k.x_a), corner k (form_factor,
 // bgy3d-solutes.c:587-600, times bgy3d_vec_fft_trans bgy3d-vec.c:619-646).
-// Grid: x = chunks of K, y = solute.
+// A workgroup takes FF_X columns kx by FF_Y rows ky of one z plane; for
+// FF_SITES sites at a time it puts exp(-i kx x) of the columns and
+// Q exp(-i (ky y + kz z)) of the rows in LDS, so that a point costs one complex
+// product per site instead of a sine and cosine (104 -> 33 us for 30 sites on
+// 128^3, 21 MB to write).
+// Grid: x = column tile, then row tile, then z plane; y = solute.
+constexpr int FF_X = 32, FF_Y = 32, FF_SITES = 16;
+__host__ __device__ inline int ff_tiles(const GridArgs& g) {
+  return ((g.NX + FF_X - 1) / FF_X) * ((g.N1 + FF_Y - 1) / FF_Y) * g.N2;
+}
 __global__ void __launch_bounds__(NT)
 form_factor(const SitesDesc* __restrict__ sites, GridArgs g, cpx<double>* const* __restrict__ fs64,
             cpx<float>* const* __restrict__ fs32) {
+  constexpr int RPT = FF_X * FF_Y / NT;  // rows per thread
+  __shared__ cpx<double> ex[FF_SITES][FF_X], eyz[FF_SITES][FF_Y];
   const SitesDesc sd = sites[blockIdx.y];
-  const int64_t stride = (int64_t)gridDim.x * NT;
-  for (int64_t e = blockIdx.x * (int64_t)NT + threadIdx.x; e < g.K; e += stride) {
-    const int x = (int)(e % g.NH);
-    if (x >= g.NX) continue;  // row padding
-    const int y = (int)((e / g.NH) % g.N1);
-    const int z = (int)(e / ((int64_t)g.NH * g.N1));
-    const int iy = (y <= g.N1 / 2) ? y : y - g.N1;
-    const int iz = (z <= g.N2 / 2) ? z : z - g.N2;
-    const double kx = x * g.dkx, ky = iy * g.dky, kz = iz * g.dkz;
-    double re = 0.0, im = 0.0;
-    for (int a = 0; a < sd.n; ++a) {
-      const double* s = sd.xyz_s_e_q + 6 * a;
+  const int tx = (g.NX + FF_X - 1) / FF_X, ty = (g.N1 + FF_Y - 1) / FF_Y;
+  const int x0 = (int)(blockIdx.x % tx) * FF_X, y0 = (int)(blockIdx.x / tx % ty) * FF_Y;
+  const int z = (int)(blockIdx.x / (tx * ty));
+  const int iz = (z <= g.N2 / 2) ? z : z - g.N2;
+  const int col = threadIdx.x % FF_X, row = threadIdx.x / FF_X * RPT;
+  double re[RPT], im[RPT];
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) re[r] = im[r] = 0.0;
+  for (int a0 = 0; a0 < sd.n; a0 += FF_SITES) {
+    const int na = min(FF_SITES, sd.n - a0);
+    __syncthreads();
+    for (int k = threadIdx.x; k < na * (FF_X + FF_Y); k += NT) {
+      const int a = k / (FF_X + FF_Y), c = k - a * (FF_X + FF_Y);
+      const double* s = sd.xyz_s_e_q + 6 * (a0 + a);
       double sn, cs;
-      sincos(kx * s[0] + ky * s[1] + kz * s[2], &sn, &cs);
-      re += s[5] * cs;
-      im -= s[5] * sn;
+      if (c < FF_X) {
+        sincos((x0 + c) * g.dkx * s[0], &sn, &cs);
+        ex[a][c] = cpx<double>{cs, -sn};
+      } else {
+        const int y = y0 + c - FF_X, iy = (y <= g.N1 / 2) ? y : y - g.N1;
+        sincos(iy * g.dky * s[1] + iz * g.dkz * s[2], &sn, &cs);
+        eyz[a][c - FF_X] = cpx<double>{s[5] * cs, -s[5] * sn};
+      }
     }
+    __syncthreads();
+    for (int a = 0; a < na; ++a) {
+      const cpx<double> u = ex[a][col];
+#pragma unroll
+      for (int r = 0; r < RPT; ++r) {
+        const cpx<double> w = eyz[a][row + r];
+        re[r] += u.re * w.re - u.im * w.im;
+        im[r] += u.re * w.im + u.im * w.re;
+      }
+    }
+  }
+  const int x = x0 + col;
+  if (x >= g.NX) return;
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    const int y = y0 + row + r;
+    if (y >= g.N1) return;
+    const int iy = (y <= g.N1 / 2) ? y : y - g.N1;
     const double sign = ((x + iy + iz) & 1) ? -1.0 : 1.0;
-    fs64[blockIdx.y][e] = cpx<double>{sign * re, sign * im};
-    if (x == g.NX - 1) fs64[blockIdx.y][g.K + (int64_t)z * g.N1 + y] = cpx<double>{sign * re, sign * im};
+    const cpx<double> f = {sign * re[r], sign * im[r]};
+    fs64[blockIdx.y][((int64_t)z * g.N1 + y) * g.NH + x] = f;
+    if (x == g.NX - 1) fs64[blockIdx.y][g.K + (int64_t)z * g.N1 + y] = f;
     if (fs32)
-      fs32[blockIdx.y][fs_index<float>(g, z, y, x)] =
-          cpx<float>{(float)(sign * re), (float)(sign * im)};
+      fs32[blockIdx.y][fs_index<float>(g, z, y, x)] = cpx<float>{(float)f.re, (float)f.im};
   }
 }
 

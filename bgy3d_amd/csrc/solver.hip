@@ -2687,8 +2687,7 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
     auto at = [&](size_t o) { return reinterpret_cast<double*>(pb.setup.p + o); };
     auto at_ptr = [&](size_t o) { return reinterpret_cast<void**>(pb.setup.p + o); };
     pb.d_sites = reinterpret_cast<SitesDesc*>(pb.setup.p + o_sd);
-    const int cp = (int)std::min<int64_t>(4096, (g.P + NT - 1) / NT);
-    const int ck = (int)std::min<int64_t>(4096, (g.K + NT - 1) / NT);
+    const int cp = (int)std::min<int64_t>(4096, (g.P / FB_PTS + NT - 1) / NT);
     if (tabs) {
       const int ckt = (int)std::min<int64_t>(4096, (g.KT + NT - 1) / NT);
       hipLaunchKernelGGL(ktab3, dim3(ckt), dim3(NT), 0, pb.s, g, at(o_chi), at(o_tau), pb.chi3.p,
@@ -2703,7 +2702,7 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
                        pb.d_sites, g, at(o_sse), pd.L[0], pd.L[1], pd.L[2], pb.h[0], pb.h[1],
                        pb.h[2], (double* const*)at_ptr(o_bv64),
                        pb.mixed ? (float* const*)at_ptr(o_bv32) : (float* const*)nullptr);
-    hipLaunchKernelGGL(form_factor, dim3(ck, B), dim3(NT), 0, pb.s, pb.d_sites, g,
+    hipLaunchKernelGGL(form_factor, dim3(ff_tiles(g), B), dim3(NT), 0, pb.s, pb.d_sites, g,
                        (cpx<double>* const*)at_ptr(o_fs64),
                        pb.mixed ? (cpx<float>* const*)at_ptr(o_fs32) : (cpx<float>* const*)nullptr);
     HIPCHK(hipGetLastError());
