@@ -1532,19 +1532,53 @@ c2r_xy_resid(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __rest
   }
 }
 
+// The sums of v[0 .. N) over a wavefront.  Halving: at each step a lane keeps
+// half of the values, adds its partner's share of them and hands the other
+// half over, so N values take about N exchanges instead of 6 N.  Returns true
+// in one lane per value, with the value's place in at and its sum in v[0].
+template <int N, int MASK = 32>
+__device__ __forceinline__ bool wave_sums(double* v, int lane, int& at) {
+  static_assert(N <= 2 * MASK || N == 1, "a value per lane at most");
+  if constexpr (N == 1) {
+    at = 0;
+    bool first = true;
+#pragma unroll
+    for (int k = MASK; k > 0; k >>= 1) {  // lanes that hold the same value
+      v[0] += __shfl_xor(v[0], k);
+      first = first && !(lane & k);
+    }
+    return first;
+  } else {
+    constexpr int H = (N + 1) / 2;
+    const bool up = (lane & MASK) != 0;
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+      const double hi = H + k < N ? v[H + k] : 0.0;
+      const double keep = up ? hi : v[k], give = up ? v[k] : hi;
+      v[k] = keep + __shfl_xor(give, MASK);
+    }
+    const bool mine = wave_sums<H, MASK / 2>(v, lane, at);
+    if (up) at += H;
+    return mine && at < N;
+  }
+}
+
 // ------------------------------------------- Gram rows of several entries
 // <rh[i], rh[j]> for i < nrow, j > i over the residual history, per workgroup
 // partials gpart[(i MAX_DIIS + j) * gridDim.x + blockIdx.x].  Bound by its
 // ngram streams: each thread holds one 16-byte vector of every entry at a
 // time, so one reading of the history serves nrow rows (the dots inside the
 // residual kernels read it once per row).  Products of one vector in the
-// working type, sums across vectors in FP64, as there.  96^3, 8 entries in
-// FP64: 49 us (3.5 TB/s); 192^3, 5 sites, 8 entries in BF16: 135 us (4.2 TB/s).
+// working type, sums across vectors in FP64, as there.  With short loops the
+// sums over the workgroup count too: by halving (wave_sums) instead of one
+// value after the other 32^3 took 6.0 instead of 9.8 us, 96^3 with 8 entries in
+// FP64 37 instead of 50 (4.6 TB/s), 192^3 with 5 sites and 8 entries in BF16 122
+// instead of 135 (4.6 TB/s).
 // Grid: x = chunks, y = solute.
 template <typename T, int H>
 __global__ void __launch_bounds__(NT)
 gram_rows(const SoluteDesc* __restrict__ sd, int64_t mP) {
-  __shared__ double red[MAX_ROWS][H][NT / 64];
+  __shared__ double red[MAX_ROWS * H][NT / 64];
   const SoluteDesc& d = sd[blockIdx.y];
   const int n = d.ngram, nrow = d.nrow;
   if (!d.active || n == 0) return;
@@ -1619,22 +1653,23 @@ gram_rows(const SoluteDesc* __restrict__ sd, int64_t mP) {
         if (j < n) v[j] = ld16(static_cast<const T*>(d.rh[j]) + e);
       rows(v);
     }
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // the pairs j > i of all rows side by side: wave sums, then over the waves
+  constexpr int NP = MAX_ROWS * H - MAX_ROWS * (MAX_ROWS + 1) / 2;
+  double pair[NP];
 #pragma unroll
   for (int i = 0; i < MAX_ROWS; ++i)
-    if (i < nrow)
 #pragma unroll
-      for (int j = i + 1; j < H; ++j)
-        if (j < n) {
-          const double s = warp_sum(acc[i][j]);
-          if (lane == 0) red[i][j][w] = s;
-        }
+    for (int j = i + 1; j < H; ++j) pair[i * H - i * (i + 1) / 2 + j - i - 1] = acc[i][j];
+  const int w = threadIdx.x >> 6;
+  int at = 0;
+  if (wave_sums<NP>(pair, threadIdx.x & 63, at)) red[at][w] = pair[0];
   __syncthreads();
   for (int q = threadIdx.x; q < MAX_ROWS * H; q += NT) {
     const int i = q / H, j = q - i * H;
     if (i >= nrow || j <= i || j >= n) continue;
-    double a = red[i][j][0];
-    for (int k = 1; k < NT / 64; ++k) a += red[i][j][k];
+    const double* r = red[i * H - i * (i + 1) / 2 + j - i - 1];
+    double a = r[0];
+    for (int k = 1; k < NT / 64; ++k) a += r[k];
     gst(d.gpart + (int64_t)(i * MAX_DIIS + j) * gridDim.x + blockIdx.x, a);
   }
 }

@@ -81,11 +81,11 @@ template <typename T>
 void launch_zstar(int N2, int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd,
                   const GridArgs& g, const cpx<T>* tw, const T* chi, const T* tau);
 // Workgroups of gram_rows per solute: 4 points or more a thread, 2048 at most
-// (a workgroup's own reduction is worth about 30 points a thread), and 8192 in
-// all: in a batch only the solutes at an extrapolation work, a third of them.
-// 24 x 64^3 in FP64: 139 us per pass with 85 workgroups a solute, 117 with 341.
+// (192^3 with 5 sites: 122 us, 127 with 4096), and 16384 in all: in a batch only
+// the solutes at an extrapolation work, a third of them (us per pass with 8192
+// and with 16384: 24 x 64^3 in FP64 104 and 99, 24 x 128^3 in FP32 178 and 173).
 inline int gram_blocks(int64_t mP, int B) {
-  const int64_t most = std::max(64, std::min(2048, 8192 / B)), fit = mP / (NT * 4);
+  const int64_t most = std::max(64, std::min(2048, 16384 / B)), fit = mP / (NT * 4);
   return (int)std::max<int64_t>(1, std::min(most, fit));
 }
 template <typename T>
