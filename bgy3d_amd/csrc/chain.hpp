@@ -27,6 +27,14 @@ __host__ __device__ constexpr int rows_for(int M) {
   return M <= 16 ? 64 : M <= 32 ? 32 : M <= 64 ? 16 : M <= 128 ? 8 : 4;
 }
 
+// Twiddles: every chain kernel copies its tables to LDS (stw) beside its first
+// loads.  Read from global memory inside the stages they shared the vector
+// cache and its wait counter with the streams, and each stage waited on both (us per
+// launch, from global memory and from LDS: closure and residual of 24 x 128^3
+// in FP32 719 and 667, 597 and 547, its z pass 281 and 241; 192^3 with 5 sites
+// in FP32 closure 203 and 186, y 71 and 56, z 140 and 126; 24 x 64^3 in FP64 closure
+// and residual 193 and 185, 153 and 133, z 91 and 82).
+
 // 16-byte vectors of the working type: the streaming loops of the x-axis
 // kernels move 16 B per lane per array (global_load/store_dwordx4), four
 // times fewer memory instructions than scalar accesses.  Every array is
@@ -291,6 +299,9 @@ closure_r2c_x(const SoluteDesc* __restrict__ sd, GridArgs g,
   __shared__ cpx<T> lds[ROWS * LSM];
   const SoluteDesc& d = sd[blockIdx.z];
   if (!d.active) return;
+  // the twiddles in LDS: [M of the rows][M + 1 of the split]
+  __shared__ cpx<T> stw[2 * M + 1];
+  for (int i = threadIdx.x; i < 2 * M + 1; i += NT) stw[i] = i < M ? tw_half[i] : tw_full[i - M];
   const int site = blockIdx.y;
   const int nrows = g.N1 * g.N2;
   const int row0 = blockIdx.x * ROWS;
@@ -312,7 +323,7 @@ closure_r2c_x(const SoluteDesc* __restrict__ sd, GridArgs g,
     for (int h = 0; h < VW / 2; ++h) zrow[lpos(n0 + h)] = cpx<T>{c.v[2 * h], c.v[2 * h + 1]};
   }
   __syncthreads();
-  fft_lines<T, M, ROWS, NT, false>(lds, LSM, vrows, tw_half);
+  fft_lines<T, M, ROWS, NT, false>(lds, LSM, vrows, stw);
   cpx<T>* W = static_cast<cpx<T>*>(d.W) + site * g.K + (int64_t)row0 * g.NH;
   const int nout = min(ROWS, nrows - row0) * (M + 1);
   for (int e = threadIdx.x; e < nout; e += NT) {
@@ -321,7 +332,7 @@ closure_r2c_x(const SoluteDesc* __restrict__ sd, GridArgs g,
     const cpx<T> zk = lds[row * LSM + lpos(k == M ? 0 : k)];
     const cpx<T> zm = cconj(lds[row * LSM + lpos(k == 0 ? 0 : M - k)]);
     const cpx<T> s = cadd(zk, zm);
-    const cpx<T> dd = rot90<T, false>(cmul(tw_full[k], csub(zk, zm)));  // -i w (Zk - conj Zm)
+    const cpx<T> dd = rot90<T, false>(cmul(stw[M + k], csub(zk, zm)));  // -i w (Zk - conj Zm)
     stc(W + row * g.NH + k, cpx<T>{T(0.5) * (s.re + dd.re), T(0.5) * (s.im + dd.im)});
   }
 }
@@ -332,8 +343,10 @@ template <typename T, int N1, int LINES, bool INV>
 __global__ void __launch_bounds__(NT)
 fft_y(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ tw) {
   __shared__ cpx<T> lds[LINES * N1];  // interleaved: point y of column l at y * LINES + l
+  __shared__ cpx<T> stw[N1];
   const SoluteDesc& d = sd[blockIdx.z];
   if (!d.active) return;
+  for (int i = threadIdx.x; i < N1; i += NT) stw[i] = tw[i];
   const int site = blockIdx.y / g.N2;
   const int z = blockIdx.y - site * g.N2;
   const int kx0 = blockIdx.x * LINES;
@@ -363,7 +376,7 @@ fft_y(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ 
     }
   }
   __syncthreads();
-  fft_lines_il<T, N1, LINES, NT, INV>(lds, min(LINES, g.NX - kx0), tw);
+  fft_lines_il<T, N1, LINES, NT, INV>(lds, min(LINES, g.NX - kx0), stw);
   for (int e = threadIdx.x; e < N1 * LINES; e += NT) {
     const int y = e / LINES, l = e - y * LINES;
     if (kx0 + l < g.NX) stc(W + y * g.NH + l, lds[e]);
@@ -756,6 +769,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
   constexpr int PTS = N2 * LINES;
   constexpr int PPT = (PTS + NTZ - 1) / NTZ;
   __shared__ cpx<T> lds[PTS];  // interleaved: point z of line l at z * LINES + l
+  __shared__ cpx<T> stw[N2];   // the twiddles
   // Block order of the 1D grid.  First the Nyquist blocks of a split launch
   // (nyq: lines are LINES rows ky of the column kx = N0/2), whose scattered
   // accesses then run beside the tiles instead of after them; a launch of
@@ -845,6 +859,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
   const int nl = nyq ? min(LINES, g.N1 - y)  // valid lines
                      : min(LINES, (g.nyqb ? g.NX - 1 : g.NX) - kx0);
   const int tid = threadIdx.x;
+  for (int i = tid; i < N2; i += NTZ) stw[i] = tw[i];
   cpx<T> c[MS][PPT];
   // every site's loads first, staged in its registers of c (its FFT result
   // lands there after its pass), so the later sites' loads overlap the
@@ -871,7 +886,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
     cpx<T>* Ws = W + s * wsite;
     if constexpr (RR) {
       if (d.mode == 4) continue;  // inverse only: the loaded spectrum goes to the inverse pass
-      fft_lines_rr<T, N2, LINES, NTZ, false>(c[s], lds, nl, tw);
+      fft_lines_rr<T, N2, LINES, NTZ, false>(c[s], lds, nl, stw);
       if (d.mode == 3) {  // forward spectrum only
 #pragma unroll
         for (int p = 0; p < PPT; ++p) {
@@ -892,7 +907,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
       }
     }
     __syncthreads();
-    fft_lines_il<T, N2, LINES, NTZ, false>(lds, nl, tw);
+    fft_lines_il<T, N2, LINES, NTZ, false>(lds, nl, stw);
 #pragma unroll
     for (int p = 0; p < PPT; ++p) {
       const int e = tid + p * NTZ;
@@ -996,7 +1011,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
   for (int s = 0; s < MS; ++s) {
     cpx<T>* Ws = W + s * wsite;
     if constexpr (RR) {
-      fft_lines_rr<T, N2, LINES, NTZ, true>(c[s], lds, nl, tw);
+      fft_lines_rr<T, N2, LINES, NTZ, true>(c[s], lds, nl, stw);
 #pragma unroll
       for (int p = 0; p < PPT; ++p) {
         const int e = tid + p * NTZ;
@@ -1011,7 +1026,7 @@ zstar_reg(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restric
       if (PPT * NTZ == PTS || e < PTS) lds[e] = c[s][p];
     }
     __syncthreads();
-    fft_lines_il<T, N2, LINES, NTZ, true>(lds, nl, tw);
+    fft_lines_il<T, N2, LINES, NTZ, true>(lds, nl, stw);
 #pragma unroll
     for (int p = 0; p < PPT; ++p) {
       const int e = tid + p * NTZ;
@@ -1042,6 +1057,9 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
   __shared__ double red[NPART][NT / 64];
   const SoluteDesc& d = sd[blockIdx.z];
   if (!d.active) return;
+  // the twiddles in LDS: [M of the rows][M + 1 of the split]
+  __shared__ cpx<T> stw[2 * M + 1];
+  for (int i = threadIdx.x; i < 2 * M + 1; i += NT) stw[i] = i < M ? tw_half[i] : tw_full[i - M];
   const int site = blockIdx.y;
   const int nrows = g.N1 * g.N2;
   const int row0 = blockIdx.x * ROWS;
@@ -1078,11 +1096,11 @@ c2r_x_resid(const SoluteDesc* __restrict__ sd, GridArgs g,
     if (k == 0) { xk.im = T(0); xm.im = T(0); }  // c2r ignores Im at DC / Nyquist
     const cpx<T> a = cadd(xk, cconj(xm));
     const cpx<T> b = csub(xk, cconj(xm));
-    const cpx<T> ib = rot90<T, true>(cmulc(b, tw_full[k]));  // i e^{+2 pi i k/N} b
+    const cpx<T> ib = rot90<T, true>(cmulc(b, stw[M + k]));  // i e^{+2 pi i k/N} b
     zb[row * LSM + lpos(k)] = cadd(a, ib);
   }
   __syncthreads();
-  fft_lines<T, M, ROWS, NT, true>(zb, LSM, vrows, tw_half);
+  fft_lines<T, M, ROWS, NT, true>(zb, LSM, vrows, stw);
   const T* __restrict__ t = static_cast<const T*>(d.t) + off;
   T* __restrict__ r = static_cast<T*>(d.r) + off;  // (BF16 slots: addressed in e below)
   T* __restrict__ un = d.unew ? static_cast<T*>(d.unew) + off : nullptr;  // null: no u
@@ -1252,7 +1270,7 @@ constexpr int plane_threads() {
 template <typename T, int N0, int N1, int H>
 __global__ void __launch_bounds__((plane_threads<T, N0, N1>()))
 closure_r2c_xy(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ tw_half,
-               const cpx<T>* __restrict__ tw_full, const cpx<T>* __restrict__ tw_y) {
+               const cpx<T>* __restrict__ tw_full) {
   constexpr int NTP = plane_threads<T, N0, N1>();
   constexpr int M = N0 / 2, LS = M + 1, PLANE = N0 * N1, HP = M / 2 + 1;
   constexpr int VW = Vec16<T>::W;
@@ -1265,6 +1283,10 @@ closure_r2c_xy(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __re
   const int64_t off = site * g.P + (int64_t)z * PLANE;
   T* __restrict__ t = static_cast<T*>(d.t) + off;
   const T* __restrict__ bv = static_cast<const T*>(d.bv) + off;
+  // the twiddles in LDS: [N0/2 of the rows][N0 of the split and the columns]
+  static_assert(N0 == N1, "one table for both");
+  __shared__ cpx<T> stw[M + N0];
+  for (int i = threadIdx.x; i < M + N0; i += NTP) stw[i] = i < M ? tw_half[i] : tw_full[i - M];
   // two vectors per step, so that both vectors' streams are in flight together
   for (int e0 = threadIdx.x * VW; e0 < PLANE; e0 += 2 * NTP * VW) {
     Vec16<T> c[2];
@@ -1283,7 +1305,7 @@ closure_r2c_xy(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __re
     }
   }
   __syncthreads();
-  fft_lines<T, M, N1, NTP, false>(lds, LS, N1, tw_half);
+  fft_lines<T, M, N1, NTP, false>(lds, LS, N1, stw);
   for (int e = threadIdx.x; e < N1 * HP; e += NTP) {
     const int row = e / HP, k = e - row * HP;
     cpx<T>* r = lds + row * LS;
@@ -1292,7 +1314,7 @@ closure_r2c_xy(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __re
     auto bin = [&](int kk, cpx<T> zk, cpx<T> zo) {
       const cpx<T> zm = cconj(zo);
       const cpx<T> sm = cadd(zk, zm);
-      const cpx<T> dd = rot90<T, false>(cmul(tw_full[kk], csub(zk, zm)));
+      const cpx<T> dd = rot90<T, false>(cmul(stw[M + kk], csub(zk, zm)));
       return cpx<T>{T(0.5) * (sm.re + dd.re), T(0.5) * (sm.im + dd.im)};
     };
     if (k == 0) {
@@ -1305,7 +1327,7 @@ closure_r2c_xy(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __re
     }
   }
   __syncthreads();
-  fft_cols<T, N1, LS, M + 1, NTP, false>(lds, tw_y);
+  fft_cols<T, N1, LS, M + 1, NTP, false>(lds, stw + M);
   // y-major rows of M bins, then the Nyquist bins of the plane's rows
   cpx<T>* W = static_cast<cpx<T>*>(d.W) + site * g.K + (int64_t)z * g.NH;
   const int64_t ys = (int64_t)g.N2 * g.NH;
@@ -1327,7 +1349,7 @@ closure_r2c_xy(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __re
 template <typename T, int N0, int N1, int H>
 __global__ void __launch_bounds__((plane_threads<T, N0, N1>()))
 c2r_xy_resid(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __restrict__ tw_half,
-             const cpx<T>* __restrict__ tw_full, const cpx<T>* __restrict__ tw_y) {
+             const cpx<T>* __restrict__ tw_full) {
   constexpr int NTP = plane_threads<T, N0, N1>();
   constexpr int M = N0 / 2, LS = M + 1, PLANE = N0 * N1, HP = M / 2 + 1;
   constexpr int VW = Vec16<T>::W;
@@ -1338,6 +1360,10 @@ c2r_xy_resid(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __rest
   const SoluteDesc& d = sd[blockIdx.z];
   if (!d.active) return;
   const int site = blockIdx.y, z = blockIdx.x;
+  // the twiddles in LDS: [N0/2 of the rows][N0 of the split and the columns]
+  static_assert(N0 == N1, "one table for both");
+  __shared__ cpx<T> stw[M + N0];
+  for (int i = threadIdx.x; i < M + N0; i += NTP) stw[i] = i < M ? tw_half[i] : tw_full[i - M];
   // the plane's y-major rows of M bins and its Nyquist bins (closure_r2c_xy)
   const cpx<T>* W = static_cast<const cpx<T>*>(d.W) + site * g.K + (int64_t)z * g.NH;
   const cpx<T>* Q = static_cast<const cpx<T>*>(d.W) + g.m * g.K + ((int64_t)site * g.N2 + z) * N1;
@@ -1374,7 +1400,7 @@ c2r_xy_resid(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __rest
     }
   }
   __syncthreads();
-  fft_cols<T, N1, LS, M + 1, NTP, true>(lds, tw_y);
+  fft_cols<T, N1, LS, M + 1, NTP, true>(lds, stw + M);
   for (int e = threadIdx.x; e < N1 * HP; e += NTP) {
     const int row = e / HP, k = e - row * HP;
     cpx<T>* r = lds + row * LS;
@@ -1383,7 +1409,7 @@ c2r_xy_resid(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __rest
     auto pre = [&](int kk, cpx<T> a0, cpx<T> b0) {
       const cpx<T> a = cadd(a0, cconj(b0));
       const cpx<T> b = csub(a0, cconj(b0));
-      return cadd(a, rot90<T, true>(cmulc(b, tw_full[kk])));
+      return cadd(a, rot90<T, true>(cmulc(b, stw[M + kk])));
     };
     if (k == 0) {
       xk.im = T(0);
@@ -1396,7 +1422,7 @@ c2r_xy_resid(const SoluteDesc* __restrict__ sd, GridArgs g, const cpx<T>* __rest
     }
   }
   __syncthreads();
-  fft_lines<T, M, N1, NTP, true>(lds, LS, N1, tw_half);
+  fft_lines<T, M, N1, NTP, true>(lds, LS, N1, stw);
   const int64_t off = site * g.P + (int64_t)z * PLANE;
   const T* __restrict__ t = static_cast<const T*>(d.t) + off;
   T* __restrict__ r = static_cast<T*>(d.r) + off;  // (BF16 slots: addressed in e below)

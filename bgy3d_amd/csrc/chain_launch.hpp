@@ -92,6 +92,6 @@ template <typename T>
 void launch_gram(dim3 grid, hipStream_t s, const SoluteDesc* sd, int64_t mP, int n);
 template <typename T>
 void launch_planes(bool inv, int B, hipStream_t s, const SoluteDesc* sd, const GridArgs& g,
-                   const cpx<T>* twh, const cpx<T>* twf, const cpx<T>* twy, int hist);
+                   const cpx<T>* twh, const cpx<T>* twf, int hist);
 
 }  // namespace rism

@@ -59,15 +59,17 @@ template <typename T>
 void launch_zstar(int N2, int NX, int N1, int B, hipStream_t s, const SoluteDesc* sd,
                   const GridArgs& g, const cpx<T>* tw, const T* chi, const T* tau) {
   if (use_zreg(g)) {
-    if (g.zwide && sizeof(T) == 4 && N2 <= 128) {  // 512 threads over 32 kx columns
-      switch (N2) {
-        case 32: launch_zreg_n<T, 32, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
-        case 48: launch_zreg_n<T, 48, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
-        case 64: launch_zreg_n<T, 64, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
-        case 96: launch_zreg_n<T, 96, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
-        case 128: launch_zreg_n<T, 128, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
+    if constexpr (sizeof(T) == 4) {
+      if (g.zwide && N2 <= 128) {  // 512 threads over 32 kx columns
+        switch (N2) {
+          case 32: launch_zreg_n<T, 32, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
+          case 48: launch_zreg_n<T, 48, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
+          case 64: launch_zreg_n<T, 64, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
+          case 96: launch_zreg_n<T, 96, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
+          case 128: launch_zreg_n<T, 128, 2 * NT>(NX, N1, B, s, sd, g, tw, chi, tau); break;
+        }
+        return;
       }
-      return;
     }
     switch (N2) {
 #define X(n) case n: launch_zreg_n<T, n>(NX, N1, B, s, sd, g, tw, chi, tau); break;

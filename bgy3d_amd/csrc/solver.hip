@@ -672,14 +672,14 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
       hipLaunchKernelGGL(load_sd, dim3(pb.B), dim3(NTL), 0, pb.s, (const SoluteDesc*)pb.io.sd, dsd);
     if (planes && fp32) {
       using T = float;
-      mark(0, 0); launch_planes<T>(false, pb.B, pb.s, dsd, g, pb.tw.f[1].p, pb.tw.f[0].p, pb.tw.f[2].p, hist); mark(0, 1);
+      mark(0, 0); launch_planes<T>(false, pb.B, pb.s, dsd, g, pb.tw.f[1].p, pb.tw.f[0].p, hist); mark(0, 1);
       mark(2, 0); launch_zstar<T>(g.N2, g.NX, g.N1, pb.B, pb.s, dsd, g, pb.tw.f[3].p, pb.chi3f.p, pb.tau3f.p); mark(2, 1);
-      mark(4, 0); launch_planes<T>(true, pb.B, pb.s, dsd, g, pb.tw.f[1].p, pb.tw.f[0].p, pb.tw.f[2].p, hist); mark(4, 1);
+      mark(4, 0); launch_planes<T>(true, pb.B, pb.s, dsd, g, pb.tw.f[1].p, pb.tw.f[0].p, hist); mark(4, 1);
     } else if (planes) {
       using T = double;
-      mark(0, 0); launch_planes<T>(false, pb.B, pb.s, dsd, g, pb.tw.d[1].p, pb.tw.d[0].p, pb.tw.d[2].p, hist); mark(0, 1);
+      mark(0, 0); launch_planes<T>(false, pb.B, pb.s, dsd, g, pb.tw.d[1].p, pb.tw.d[0].p, hist); mark(0, 1);
       mark(2, 0); launch_zstar<T>(g.N2, g.NX, g.N1, pb.B, pb.s, dsd, g, pb.tw.d[3].p, pb.chi3.p, pb.tau3.p); mark(2, 1);
-      mark(4, 0); launch_planes<T>(true, pb.B, pb.s, dsd, g, pb.tw.d[1].p, pb.tw.d[0].p, pb.tw.d[2].p, hist); mark(4, 1);
+      mark(4, 0); launch_planes<T>(true, pb.B, pb.s, dsd, g, pb.tw.d[1].p, pb.tw.d[0].p, hist); mark(4, 1);
     } else if (fp32) {
       using T = float;
       constexpr int LN = y_lines<T>();
