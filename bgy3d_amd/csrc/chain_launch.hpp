@@ -52,20 +52,21 @@ inline bool use_zreg(const GridArgs& g) {
 // on (us per pass, rows against planes: 48^3 50 and 48 but 68 and 72 with the
 // host's part for one solute, 195 and 184 for 24; 32^3 48 and 37, 86 and 61;
 // 192^2 planes would fill a CU's LDS: 800 and 800, 481 and 552).  FP64: up to 64
-// points always; planes of 96 and 128 points take 75 and 133 KB of LDS, two
-// and one workgroup per CU, and need about four workgroups per CU to fill
-// the chip (us per FP64 pass, rows against planes: 32^3 47 and 30, 64^3 72
-// and 59, 24 x 64^3 1006 and 841; 96^3 157 and 164 for one solute, 519 and
-// 483 for 4, 3355 and 2820 for 24; 128^3 339 and 358, 1188 and 1138, 7932
-// and 6855).  The plane kernels write W y-major with the Nyquist column
-// apart (GridArgs::ylay), which only zstar_reg reads.
+// points always; planes of 96 and 128 points take 78 and 136 KB of LDS, two
+// and one workgroup per CU, and need about two and four workgroups per CU to
+// fill the chip (us per FP64 pass, rows against planes: 32^3 47 and 30, 64^3 72
+// and 59, 24 x 64^3 1006 and 841; 96^3 118 and 123 for one solute, 199 and 195
+// for 2, 287 and 270 for 3; 128^3 234 and 261, 423 and 437, 4 solutes 1188
+// and 1138).  The plane kernels write W y-major with the Nyquist column apart
+// (GridArgs::ylay), which only zstar_reg reads.
 inline bool use_planes(const GridArgs& g, int B, bool fp32, int on) {
   if (!on || g.N0 != g.N1 || !use_zreg(g)) return false;
   if (fp32)
     return g.N0 == 32 || g.N0 == 64 || g.N0 == 96 || g.N0 == 128 ||
            (g.N0 == 48 && (int64_t)g.m * g.N2 * B >= 512);
   if (g.N0 <= 64) return true;
-  return (g.N0 == 96 || g.N0 == 128) && (int64_t)g.m * g.N2 * B >= 1024;
+  const int64_t wgs = (int64_t)g.m * g.N2 * B;
+  return (g.N0 == 96 && wgs >= 512) || (g.N0 == 128 && wgs >= 1024);
 }
 
 template <typename T>

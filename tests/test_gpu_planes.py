@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 W = "water, PR-SPC/E"
 
 
-@pytest.mark.parametrize("N,B", [(96, 4), (128, 3)])
+@pytest.mark.parametrize("N,B", [(96, 2), (96, 4), (128, 3)])
 def test_batch_on_planes_equals_single_on_rows(N, B, chi_w):
     print(f"case planes fp64 {N}^3 batch {B}", flush=True)
     from bgy3d_amd import rism3d as R
