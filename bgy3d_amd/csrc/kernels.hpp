@@ -78,11 +78,12 @@ constexpr int NOUT = 2 + MAX_ROWS * MAX_DIIS;
 // It begins once max|F| fell to PULAY_BELOW, where the closure is close to
 // linear (above, a plain step can overshoot: with period 3 from the start
 // Cl- with PSE-3 took 78 passes instead of 45, and Na+ with HNC could
-// overflow), at once for the linear adjoint, and with at least PULAY_DEPTH
-// entries.  Passes to 1e-10, MDIIS each pass and period 3: 227 and 215, 322
+// overflow), and with at least PULAY_DEPTH entries.  Passes to 1e-10, MDIIS each pass and period 3: 227 and 215, 322
 // and 263, 425 and 233 (14-site solutes, KH, 64^3), 393 and 315 (PSE-3), 375
-// and 268 (saline), 45 and 55 (Cl-, PSE-3, the worst seen), adjoint 604 and
-// 190.  Not for the 3D solvent: 82 and 122.
+// and 268 (saline), 45 and 55 (Cl-, PSE-3, the worst seen).  Not for the 3D
+// solvent: 82 and 122.  Not for the adjoint either, whose stopping test leaves
+// its gradients open by up to 2e-9: 604 and 190 passes, but other gradients
+// within that, while with an extrapolation at every pass they repeat to 1e-10.
 constexpr int PULAY_PERIOD = 3;
 constexpr int PULAY_DEPTH = 5;
 constexpr double PULAY_BELOW = 1.0;

@@ -417,7 +417,8 @@ struct Problem {
   // three passes and tells nearly parallel residuals apart, for which FP8 is
   // too coarse: 253 passes to 1e-10 with FP8 each pass, 249 with BF16 and
   // period 3, 395 with FP8 and period 3 (12-site solutes, 64^3, depth 10).
-  int r8 = env_int("RISM3D_R_FP8", -1);
+  int r8_fixed = env_int("RISM3D_R_FP8", -1);
+  int r8 = 0;  // of the running iteration
   int B;
   int64_t mP;
   hipStream_t s;
@@ -745,13 +746,15 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
       ++na;
       // u_j in (+ the shift of the previous base's entries), t out (or t
       // in), beta v in, C out
-      const double uin = d.u16 ? mP * sc + (d.ncomb - 1) * mP * 2.0 : d.ncomb * mP * sc;
+      const double uin =
+          d.ncomb == 0 ? 0.0 : d.u16 ? mP * sc + (d.ncomb - 1) * mP * 2.0 : d.ncomb * mP * sc;
       b0 += uin + (d.shift_w != 0.0 ? mP * sc : 0) + mP * sc + mP * sc + mK * 2 * sc;
       // W in, t in, r and u out, r_j in (+ F(t_b) in, defect correction);
-      // r and r_j in BF16 with r16
+      // r and r_j in BF16 with r16; difference form: the replaced u in, unless
+      // it is t, and the difference out
       const double sr = d.r8 ? 1.0 : (d.r16 ? 2.0 : sc);
       b4 += mK * 2 * sc + mP * sc + mP * sr + mP * sc + d.ndot * mP * sr +
-            (d.mode == 5 ? mP * sc : 0) + (d.u16 ? mP * sc + mP * 2.0 : 0);
+            (d.mode == 5 ? mP * sc : 0) + (d.u16 ? (d.plain ? 0.0 : mP * sc) + mP * 2.0 : 0);
     }
     const double tables = (double)(g.m * (g.m + 1) / 2 + g.m) * Kv * sc;
     const double per[5] = {b0, na * 2 * mK * 2 * sc,
@@ -1067,10 +1070,11 @@ void iterate_batch(Problem& pb, const Config& cf) {
   std::vector<SoluteDesc> sd(B);
   std::vector<double> out((size_t)B * NOUT);
   std::vector<int> act(B, 0);
-  pb.period = D >= PULAY_DEPTH && pb.g.special == 0 ? pb.pulay : 1;
+  pb.period = D >= PULAY_DEPTH && pb.g.special == 0 && cf.mode == 0 ? pb.pulay : 1;
+  pb.r8 = !pb.r16 ? 0 : pb.r8_fixed >= 0 ? pb.r8_fixed : pb.period == 1;
   for (int b = 0; b < B; ++b) {
     auto& s = pb.st[b];
-    s.low = cf.mode == 1 ? 0.0 : INFINITY;  // the adjoint is linear throughout
+    s.low = INFINITY;
     s.skipped = s.pend = s.rows = s.picard = 0;
     s.talias = -1;
     if (s.active && pb.period > 1 && !s.gpart.p)
@@ -2499,8 +2503,6 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
   // iterates t itself to its floor, where the Gram rounding would show
   if (in.opt.precision != RISM3D_MIXED) pb.r16 = 0;
   if (!pb.r16) pb.u16 = 0;
-  if (pb.r8 < 0) pb.r8 = pb.pulay > 1 && pb.D >= PULAY_DEPTH ? 0 : 1;
-  if (!pb.r16) pb.r8 = 0;
   for (int d = 0; d < 3; ++d) { pb.N[d] = pd.N[d]; pb.L[d] = pd.L[d]; pb.h[d] = pd.L[d] / pd.N[d]; }
   GridArgs& g = pb.g;
   std::memset(&g, 0, sizeof g);
