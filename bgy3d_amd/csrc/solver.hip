@@ -452,7 +452,7 @@ struct Problem {
   // The small arrays of the setup (1D tables, sites, pointers), one upload.
   DevBuf<char> setup;
   Pinned setup_host;
-  // The residual chain (five kernels + the norm reduction) as HIP graphs,
+  // The residual chain (its kernels and the norm reduction) as HIP graphs,
   // one per working precision and history width, captured on first use and
   // replayed every iteration (the descriptors they read are uploaded
   // before each replay).  Re-captured if the grid arguments change.

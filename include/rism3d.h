@@ -84,7 +84,9 @@ enum rism3d_status {
    bgy3d-snes.c:16-35) plus MDIIS.  Every solver stops at max|F| <=
    norm_tol.  NEWTON, JAGER and TRIAL run in FP64 only. */
 enum rism3d_solver {
-  RISM3D_SOLVER_MDIIS = 0,  /* default: MDIIS / Anderson mixing         */
+  RISM3D_SOLVER_MDIIS = 0,  /* default: MDIIS / Anderson mixing, near the
+                               root at every third step, plain steps
+                               between (periodic Pulay)                  */
   RISM3D_SOLVER_PICARD = 1, /* x += lambda F(x) (bgy3d-snes.c:348-384)  */
   RISM3D_SOLVER_NEWTON = 2, /* Newton, GMRES(30) on the matrix-free
                                Jacobian, backtracking line search
