@@ -755,7 +755,7 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
       // r and r_j in BF16 with r16; difference form: the replaced u in, unless
       // it is t, and the difference out
       const double sr = d.r8 ? 1.0 : (d.r16 ? 2.0 : sc);
-      b4 += mK * 2 * sc + mP * sc + mP * sr + mP * sc + d.ndot * mP * sr +
+      b4 += mK * 2 * sc + mP * sc + mP * sr + (d.unew ? mP * sc : 0) + d.ndot * mP * sr +
             (d.mode == 5 ? mP * sc : 0) + (d.u16 ? (d.plain ? 0.0 : mP * sc) + mP * 2.0 : 0);
     }
     const double tables = (double)(g.m * (g.m + 1) / 2 + g.m) * Kv * sc;
