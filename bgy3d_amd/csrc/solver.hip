@@ -1337,7 +1337,9 @@ void iterate_batch(Problem& pb, const Config& cf) {
       const bool u16 = fp32 && pb.u16;
       auto slotD = [&](int q) { return (void*)((uint16_t*)s.U.p + (size_t)q * mP); };
       s.talias = -1;
-      if (s.picard && !fp32) {  // t = the newest u, read where it is
+      if (s.picard && !fp32 && Dp > 1) {
+        // t = the newest u, read where it is; with one slot (Dp = 1) the new u
+        // goes over it, so there t is a copy, which the result keeps
         d.ncomb = 0;
         s.talias = s.order.back();
         d.t = slotU(s.talias);
@@ -1355,7 +1357,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
         d.u16 = d.plain = u16;
         d.u[0] = u16 ? (void*)s.ucur : slotU(q);
         d.coef[0] = 1.0;
-        if (!u16 && s.sbase[q] != s.base) d.shift_w = 1.0;
+        if (fp32 && !u16 && s.sbase[q] != s.base) d.shift_w = 1.0;
       } else if (u16) {
         // t = sum_j c_j u_j = u_newest - sum_i (c_0 + .. + c_i) (u_i+1 - u_i),
         // the difference u_i+1 - u_i in the BF16 slot of entry i + 1
