@@ -2994,10 +2994,14 @@ int run(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
   return run_impl(in, res, t_init, t_final, nullptr);
 }
 
-// Device bytes one residual evaluation takes from the arena (the buffers
-// run_impl creates on the t_eval path with one history slot), each rounded
-// up to the arena's 256-byte alignment; the residual-workgroup partials
-// are bounded by one workgroup per (y, z) row and site.
+// The scratch that a residual evaluation is admitted by: the fields, the
+// spectra and the k tables whole in both precisions, each rounded up to the
+// arena's 256-byte alignment, and a residual workgroup per (y, z) row and site.
+// What run_impl takes on the t_eval path with one history slot is always less:
+// its tables are quarters, and whole only for a chi3d; their Nyquist columns and
+// those of W and F s weigh less than the partials of the rows that a workgroup
+// takes together (53 KB to spare at least, at 384 x 32 x 32 with one site,
+// mixed and a chi3d).
 size_t noalloc_bytes(const rism3d_problem& pd, int m, int n, bool mixed) {
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t N0 = pd.N[0], N1 = pd.N[1], N2 = pd.N[2];
@@ -3007,12 +3011,11 @@ size_t noalloc_bytes(const rism3d_problem& pd, int m, int n, bool mixed) {
   size_t b = 0;
   for (size_t len : {N0, N0 / 2, N1, N2}) b += al(len * 16) + al(len * 8);  // twiddles
   b += al(np * nrad * 8) + al(m * nrad * 8);                       // 1D tables
-  const size_t Kw = K + N1 * N2;  // with the Nyquist column apart
-  b += al(np * Kw * 8) + al(np * Kw * 4) + al(m * Kw * 8) + al(m * Kw * 4);  // 3D tables
-  b += 4 * al(mP * 8) + al(m * Kw * 16) + al(Kw * 16);  // U, R, t, beta v; W; F s
-  if (mixed) b += 4 * al(mP * 4) + al(mP * 8) + al(Kw * 8);
+  b += al(np * K * 8) + al(np * K * 4) + al(m * K * 8) + al(m * K * 4);  // 3D tables
+  b += 4 * al(mP * 8) + al(m * K * 16) + al(K * 16);  // U, R, t, beta v; W; F s
+  if (mixed) b += 4 * al(mP * 4) + al(mP * 8) + al((K + N1 * N2) * 8);
   b += al(N1 * N2 * m * NPART * 8) + al((size_t)std::max(n, 0) * 6 * 8);
-  b += al(sizeof(SoluteDesc)) + al(sizeof(SitesDesc)) + al(NOUT * 8) + 3 * al(8);
+  b += al(sizeof(SoluteDesc)) + al(sizeof(SitesDesc)) + al(NPART * 8) + 3 * al(8);
   b += al(3 * (size_t)m * 8) + 4 * al(8);  // setup descriptors
   return b;
 }
