@@ -248,6 +248,7 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
         flag = 5;
       else if (drop)
         flag = 4;
+      if (s.to16 && s.low <= PULAY_BELOW && (flag == 0 || flag == 4)) flag = flag == 0 ? 6 : 7;
       s.sbase[sn] = s.base;
       s.order[nd0] = sn;
       s.n = nd0 + 1;
@@ -481,6 +482,23 @@ mdiis_load(const uint64_t* __restrict__ rows, SoluteDesc* __restrict__ sd,
   uint64_t* dm = reinterpret_cast<uint64_t*>(mst + b);
   for (int i = threadIdx.x; i < WS; i += 64) ds[i] = row[1 + i];
   for (int i = threadIdx.x; i < WM; i += 64) dm[i] = row[1 + WS + i];
+}
+
+// FP8 residuals to BF16, four points a thread (once per solve, when periodic
+// mixing begins).  Grid: x = chunks, y = entry.
+struct HistMove {
+  const uint8_t* src[MAX_DIIS];
+  uint16_t* dst[MAX_DIIS];
+  float inv[MAX_DIIS];  // 1 / the scale of src
+};
+__global__ void __launch_bounds__(NT)
+hist_to_bf16(HistMove h, int64_t n) {
+  const uint8_t* src = h.src[blockIdx.y];
+  uint16_t* dst = h.dst[blockIdx.y];
+  const float inv = h.inv[blockIdx.y];
+  const int64_t stride = (int64_t)gridDim.x * NT * 4;
+  for (int64_t e = (blockIdx.x * (int64_t)NT + threadIdx.x) * 4; e < n; e += stride)
+    stbf4(dst + e, to_bf4(from_fp8x4(*reinterpret_cast<const uint32_t*>(src + e), inv)));
 }
 
 // FP32 <-> FP64 copies of the iterate at a precision hand-over.

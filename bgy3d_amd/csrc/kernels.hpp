@@ -120,6 +120,8 @@ struct MdiisDev {
   int pend;               // newest entries without Gram rows
   int rows;               // of the pending pass: 0 none, 1 its dots, 2 gram_rows
   int picard;             // the next pass takes t = the newest u
+  int to16;               // stop for the host when periodic mixing begins, which
+                          // moves the FP8 history to BF16 (flags 6, 7)
   int hold;               // the 1e3 drop only marks the solute ready (flag 4),
                           // the phase's tolerance parks it (flag 5)
   int order[MAX_DIIS];
@@ -137,7 +139,9 @@ static_assert(sizeof(MdiisDev) % 8 == 0, "MdiisDev is copied in 8-byte words");
 struct MdiisStatus {
   int flag;               // 0 next pass prepared, 1 rebase wanted, 2 not
                           // finite, 4 ready for a rebase, next pass prepared,
-                          // 5 at the phase's tolerance: parked until a rebase
+                          // 5 at the phase's tolerance: parked until a rebase,
+                          // 6 and 7: as 0 and 4, but the history goes to BF16
+                          // before the next pass
   int iters, iters32;
   int hist;               // flag 0: history slots of the next pass, max(ncomb, ndot)
   double resid, r2;       // max|F|, ||F||^2 of the pass

@@ -398,6 +398,7 @@ struct SoluteState {
   int rows = 0;               // of the pending pass: 0 none, 1 its dots, 2 gram_rows
   int picard = 0;             // the next pass takes t = the newest u
   int talias = -1;            // FP64: the u slot the last pass read as its t
+  int r8 = 0;                 // the FP32 phase's residual history is in FP8 now
 };
 
 struct Problem {
@@ -415,12 +416,17 @@ struct Problem {
   int u16 = env_int("RISM3D_U_DIFF", 1);
   // FP32 phase (with r16): the residual history in FP8 e4m3, each entry
   // scaled by 240 / (max|r| of the previous pass) into the e4m3 range; -1:
-  // where every pass extrapolates.  Periodic mixing reads the history once in
-  // three passes and tells nearly parallel residuals apart, for which FP8 is
+  // as long as every pass extrapolates.  Periodic mixing reads the history once
+  // in three passes and tells nearly parallel residuals apart, for which FP8 is
   // too coarse: 253 passes to 1e-10 with FP8 each pass, 249 with BF16 and
   // period 3, 395 with FP8 and period 3 (12-site solutes, 64^3, depth 10).
+  // Before it, far from the root, the coarse Gram rows hold the extrapolations
+  // back: with BF16 from the start the iterations of most ions with HNC
+  // overflowed and began again along the closures (F-, 48^3: 121 passes
+  // instead of 52).
   int r8_fixed = env_int("RISM3D_R_FP8", -1);
-  int r8 = 0;  // of the running iteration
+  // of the running iteration: 0 BF16, 1 FP8 until periodic mixing begins, 2 FP8
+  int r8 = 0;
   int B;
   int64_t mP;
   hipStream_t s;
@@ -992,6 +998,27 @@ void rebase(Problem& pb, const Config& cf, const std::vector<int>& mask, bool ad
 // The FP32 phase's MDIIS step (RISM3D_STEP32, default the solve's step).
 double lam32(const Problem& pb, const Config& cf) { return pb.lam32 > 0 ? pb.lam32 : cf.lam; }
 
+// The FP8 residual slots, behind the BF16 ones (R holds FP64 slots).
+uint8_t* slots8(const Problem& pb, const SoluteState& s) {
+  return reinterpret_cast<uint8_t*>(s.R.p) + (size_t)pb.D * pb.mP * 2;
+}
+
+// Solute s's residual history from FP8 to BF16, slot by slot.
+void history_to_bf16(Problem& pb, SoluteState& s) {
+  HistMove h;
+  std::memset(&h, 0, sizeof h);
+  const int n = (int)s.order.size();
+  for (int i = 0; i < n; ++i) {
+    const int q = s.order[i];
+    h.src[i] = slots8(pb, s) + (size_t)q * pb.mP;
+    h.dst[i] = reinterpret_cast<uint16_t*>(s.R.p) + (size_t)q * pb.mP;
+    h.inv[i] = 1.0f / s.rsc[q];
+  }
+  const int ch = (int)std::min<int64_t>(1024, (pb.mP / 4 + NT - 1) / NT);
+  hipLaunchKernelGGL(hist_to_bf16, dim3(ch, n), dim3(NT), 0, pb.s, h, pb.mP);
+  s.r8 = 0;
+}
+
 void rebase_start(Problem& pb, const Config& cf, int b, double r2, bool seed) {
   auto& s = pb.st[b];
   s.ready_at = -1;
@@ -999,8 +1026,9 @@ void rebase_start(Problem& pb, const Config& cf, int b, double r2, bool seed) {
   const int64_t mP = pb.mP;
   const int D = pb.D;
   const int ch = (int)std::min<int64_t>(2048, (mP + NT - 1) / NT);
+  if (seed) s.r8 = pb.r8 == 2 || (pb.r8 == 1 && s.low > PULAY_BELOW);
   float* U0 = reinterpret_cast<float*>(s.U.p);
-  void* R0 = s.R.p;  // slot 0, BF16 or FP32
+  void* R0 = s.r8 ? (void*)slots8(pb, s) : (void*)s.R.p;  // slot 0, FP8, BF16 or FP32
   if (seed) {
     s.dcur = s.t32.p;
     s.dshift = s.t32b.p;
@@ -1013,7 +1041,7 @@ void rebase_start(Problem& pb, const Config& cf, int b, double r2, bool seed) {
     if (pb.u16) U0 = s.ucur;
   }
   float r8s = 0.f;  // FP8 history: r_0 = F(t_b) scaled by 240 / max|F(t_b)|
-  if (seed && pb.r8) {
+  if (seed && s.r8) {
     s.rsc.assign(D, 1.f);
     r8s = fp8_scale(s.resid);
     s.rsc[0] = r8s;
@@ -1073,7 +1101,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
   std::vector<double> out((size_t)B * NOUT);
   std::vector<int> act(B, 0);
   pb.period = D >= PULAY_DEPTH && pb.g.special == 0 && cf.mode == 0 ? pb.pulay : 1;
-  pb.r8 = !pb.r16 ? 0 : pb.r8_fixed >= 0 ? pb.r8_fixed : pb.period == 1;
+  pb.r8 = !pb.r16 || pb.r8_fixed == 0 ? 0 : pb.r8_fixed > 0 || pb.period == 1 ? 2 : 1;
   for (int b = 0; b < B; ++b) {
     auto& s = pb.st[b];
     s.low = INFINITY;
@@ -1177,7 +1205,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
     std::memset(&m, 0, sizeof m);
     m.ucur = s.ucur;
     m.U = static_cast<uint16_t*>(static_cast<void*>(s.U.p));
-    m.R = static_cast<uint8_t*>(static_cast<void*>(s.R.p));
+    m.R = s.r8 ? slots8(pb, s) : static_cast<uint8_t*>(static_cast<void*>(s.R.p));
     m.mP = mP;
     m.rb_rinf = s.rb_rinf;
     m.tol_half = 0.5 * s.tol_mixed;
@@ -1193,7 +1221,8 @@ void iterate_batch(Problem& pb, const Config& cf) {
     m.iters = s.iters;
     m.iters32 = s.iters32;
     m.hold = pb.rebase_wait > 0;
-    m.rbytes = pb.r8 ? 1 : 2;
+    m.rbytes = s.r8 ? 1 : 2;
+    m.to16 = s.r8 && pb.r8 == 1;
     m.period = pb.period;
     m.skipped = s.skipped;
     m.pend = s.pend;
@@ -1207,7 +1236,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
     for (int i = 0; i < m.ndot; ++i) m.dotted[i] = s.dotted[i];
     for (int q = 0; q < D; ++q) {
       m.sbase[q] = s.sbase[q];
-      m.rsc[q] = pb.r8 ? s.rsc[q] : 1.f;
+      m.rsc[q] = s.r8 ? s.rsc[q] : 1.f;
       for (int j = 0; j < D; ++j) m.gram[q * MAX_DIIS + j] = s.gram[q * D + j];
     }
     m.resid = s.resid;
@@ -1227,7 +1256,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
     s.slot_new = m.slot_new;
     for (int q = 0; q < D; ++q) {
       s.sbase[q] = m.sbase[q];
-      if (pb.r8) s.rsc[q] = m.rsc[q];
+      if (s.r8) s.rsc[q] = m.rsc[q];
       for (int j = 0; j < D; ++j) s.gram[q * D + j] = m.gram[q * MAX_DIIS + j];
     }
     s.since_best = m.since_best;
@@ -1330,8 +1359,11 @@ void iterate_batch(Problem& pb, const Config& cf) {
       d.active = s.active && !s.parked && (s.phase32 != 0) == fp32;
       if (!d.active) return;
       auto slotU = [&](int q) { return (void*)((char*)s.U.p + (size_t)q * mP * sz); };
-      const size_t szr = fp32 && pb.r8 ? 1 : (fp32 && pb.r16 ? 2 : sz);  // FP8 / BF16 history
-      auto slotR = [&](int q) { return (void*)((char*)s.R.p + (size_t)q * mP * szr); };
+      if (fp32 && s.r8 && pb.r8 == 1 && s.low <= PULAY_BELOW) history_to_bf16(pb, s);
+      const bool r8 = fp32 && s.r8;
+      const size_t szr = r8 ? 1 : (fp32 && pb.r16 ? 2 : sz);  // FP8 / BF16 history
+      char* const R0 = r8 ? (char*)slots8(pb, s) : (char*)s.R.p;
+      auto slotR = [&](int q) { return (void*)(R0 + (size_t)q * mP * szr); };
       d.t = fp32 ? (void*)s.dcur : (void*)s.t64.p;
       d.ncomb = (int)s.coef.size();
       const bool u16 = fp32 && pb.u16;
@@ -1399,7 +1431,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
       d.ngram = s.rows == 2 ? nh + 1 : 0;
       d.nrow = s.pend + 1;
       d.gpart = s.gpart.p;
-      if (fp32 && pb.r8) {
+      if (r8) {
         d.r8 = 1;
         d.rsc = fp8_scale(s.resid);
         s.rsc[s.slot_new] = d.rsc;
@@ -1459,7 +1491,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
       evaluate(pb, true, sd, 1, hist);
       wait_status();
       ++npass32;
-      std::vector<int> rebase_mask(B, 0), back;
+      std::vector<int> rebase_mask(B, 0), back, to16;
       bool any_rebase = false;
       for (int b = 0; b < B; ++b) {
         auto& s = pb.st[b];
@@ -1480,7 +1512,11 @@ void iterate_batch(Problem& pb, const Config& cf) {
           rebase_mask[b] = 1;
           any_rebase = true;
           back.push_back(b);
-        } else if (q.flag == 4 || q.flag == 5) {
+        } else if (q.flag == 6 || q.flag == 7) {  // its history goes to BF16 first
+          to16.push_back(b);
+          back.push_back(b);
+        }
+        if (q.flag == 4 || q.flag == 5 || q.flag == 7) {
           if (s.ready_at < 0) s.ready_at = npass32;
           s.parked = q.flag == 5;
         }
@@ -1502,6 +1538,8 @@ void iterate_batch(Problem& pb, const Config& cf) {
         for (int b = 0; b < B; ++b)
           if (rebase_mask[b]) dev_dirty.push_back(b);
       }
+      for (int b : to16)
+        if (!rebase_mask[b]) dev_dirty.push_back(b);
       continue;
     }
     for (int b = 0; b < B; ++b) make_desc(b);
