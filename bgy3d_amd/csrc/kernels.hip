@@ -264,6 +264,7 @@ mdiis_step(const double* __restrict__ out, MdiisDev* __restrict__ mst,
         s.best = r2;
         s.since_best = 0;
         s.pend = s.skipped = 0;
+        if (s.low <= PULAY_BELOW) s.period = 1;
       }
       s.picard = !extrap || s.n == 1;
     }

@@ -76,17 +76,24 @@ constexpr int NOUT = 2 + MAX_ROWS * MAX_DIIS;
 // a reading of it (Banerjee, Suryanarayana and Pask, Chem. Phys. Lett. 647,
 // 31 (2016)); their Gram rows are formed together at the next extrapolation.
 // It begins once max|F| fell to PULAY_BELOW, where the closure is close to
-// linear (above, a plain step can overshoot: with period 3 from the start
-// Cl- with PSE-3 took 78 passes instead of 45, and Na+ with HNC could
-// overflow), and with at least PULAY_DEPTH entries.  Passes to 1e-10, MDIIS each pass and period 3: 227 and 215, 322
-// and 263, 425 and 233 (14-site solutes, KH, 64^3), 393 and 315 (PSE-3), 375
-// and 268 (saline), 45 and 55 (Cl-, PSE-3, the worst seen).  Not for the 3D
-// solvent: 82 and 122.  Not for the adjoint either, whose stopping test leaves
+// linear, and with at least PULAY_DEPTH entries.  Above, a plain step can
+// overshoot, and ions with HNC and PSE-3 or 4 overflow and begin again along the
+// closures: below 1.0 one in 90 of 2400 random solves (ions, 2 to 11 sites, 32^3
+// to 64^3, depths 5 to 16, steps 0.3 to 0.8) took more than 1.5 times the
+// passes, some three times, and 3 were lost that converge with MDIIS each pass;
+// below 0.3 one in 600 did, 1.9 times at most, and none was lost; below 0.1 as
+// below 0.3.  A restart, which a plain step caused or did not prevent, ends it for
+// the rest of the iteration (with a step of 3 plain steps diverge by
+// themselves: of 20 solves one survived without that), and the closures of an
+// iteration that overflowed are walked with MDIIS each pass.  Passes of those
+// random solves against MDIIS each pass: 0.84 times (FP64) and 0.98 times
+// (mixed) at depth 5, 0.95 and 0.99 at 8, 1.03 at 16; two of three passes read
+// no history.  Not for the 3D solvent: 82 passes and 122.
 // its gradients open by up to 2e-9: 604 and 190 passes, but other gradients
 // within that, while with an extrapolation at every pass they repeat to 1e-10.
 constexpr int PULAY_PERIOD = 3;
 constexpr int PULAY_DEPTH = 5;
-constexpr double PULAY_BELOW = 1.0;
+constexpr double PULAY_BELOW = 0.3;
 // Restart limits on ||F||^2 over its best: at an extrapolation, after a plain
 // step.
 constexpr double RESTART_EXTRAP = 100.0, RESTART_PLAIN = 1e4;

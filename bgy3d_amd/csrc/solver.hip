@@ -396,6 +396,7 @@ struct SoluteState {
   int skipped = 0;            // plain steps since the last extrapolation
   int pend = 0;               // newest entries without Gram rows
   int rows = 0;               // of the pending pass: 0 none, 1 its dots, 2 gram_rows
+  int period = 1;             // PULAY_PERIOD, or 1: every pass extrapolates
   int picard = 0;             // the next pass takes t = the newest u
   int talias = -1;            // FP64: the u slot the last pass read as its t
   int r8 = 0;                 // the FP32 phase's residual history is in FP8 now
@@ -406,7 +407,7 @@ struct Problem {
   int N[3];
   double L[3], h[3];
   int D;          // DIIS depth (1 = Picard)
-  int period = 1; // of the running iteration: PULAY_PERIOD or 1 (kernels.hpp)
+  int period = 1; // the running iteration begins with: PULAY_PERIOD or 1 (kernels.hpp)
   int mixed;
   int r16 = env_int("RISM3D_R_BF16", 1);  // FP32 phase: residual history in BF16
   int D32 = env_int("RISM3D_DEPTH32", 0);   // FP32 phase: MDIIS depth (0: D)
@@ -917,6 +918,7 @@ struct Config {
   double lam, tol, mixed_tol;
   int mode = 0;          // 0: F(t) = 0; 1: adjoint lambda = D K lambda + g
   double rel_tol = 0.0;  // mode 1: stop at max|r| <= rel_tol max|g|
+  int every = 0;         // 1: an extrapolation at every pass
 };
 
 // Copy the iterate between its FP32 and FP64 buffers for the solutes whose
@@ -1100,11 +1102,12 @@ void iterate_batch(Problem& pb, const Config& cf) {
   std::vector<SoluteDesc> sd(B);
   std::vector<double> out((size_t)B * NOUT);
   std::vector<int> act(B, 0);
-  pb.period = D >= PULAY_DEPTH && pb.g.special == 0 && cf.mode == 0 ? pb.pulay : 1;
+  pb.period = D >= PULAY_DEPTH && pb.g.special == 0 && cf.mode == 0 && !cf.every ? pb.pulay : 1;
   pb.r8 = !pb.r16 || pb.r8_fixed == 0 ? 0 : pb.r8_fixed > 0 || pb.period == 1 ? 2 : 1;
   for (int b = 0; b < B; ++b) {
     auto& s = pb.st[b];
     s.low = INFINITY;
+    s.period = pb.period;
     s.skipped = s.pend = s.rows = s.picard = 0;
     s.talias = -1;
     if (s.active && pb.period > 1 && !s.gpart.p)
@@ -1223,7 +1226,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
     m.hold = pb.rebase_wait > 0;
     m.rbytes = s.r8 ? 1 : 2;
     m.to16 = s.r8 && pb.r8 == 1;
-    m.period = pb.period;
+    m.period = s.period;
     m.skipped = s.skipped;
     m.pend = s.pend;
     m.rows = s.rows;
@@ -1247,6 +1250,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
     auto& s = pb.st[b];
     s.order.assign(m.order, m.order + m.n);
     s.coef.assign(m.coef, m.coef + m.n);
+    s.period = m.period;
     s.skipped = m.skipped;
     s.pend = m.pend;
     s.rows = m.rows;
@@ -1424,7 +1428,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
       // history; or, after plain steps, theirs and its own by gram_rows.  The
       // polish after an FP32 phase extrapolates at every pass (few passes).
       const bool polish = !fp32 && cf.precision != RISM3D_FP64;
-      const int period = s.low <= PULAY_BELOW && !polish ? pb.period : 1;
+      const int period = s.low <= PULAY_BELOW && !polish ? s.period : 1;
       s.rows = s.skipped + 1 >= period ? (s.pend ? 2 : 1) : 0;
       const int nh = (int)s.dotted.size();
       d.ndot = s.rows == 1 ? nh : 0;
@@ -1579,7 +1583,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
         // The new entry still enters the history (the rebase moves it).
         // ready (with a rebase wait): the 1e3 drop, or mixed_tol / 2 reached
         const bool drop = !only32 && rinf <= 1e-3 * s.rb_rinf, conv = rinf <= 0.5 * s.tol_mixed;
-        if (s.stall32 >= stall_passes(pb.period, s.low) || s.iters32 >= cf.max_iter || (pb.rebase_wait <= 0 && (drop || conv)) ||
+        if (s.stall32 >= stall_passes(s.period, s.low) || s.iters32 >= cf.max_iter || (pb.rebase_wait <= 0 && (drop || conv)) ||
             (only32 && conv)) {
           rebase_mask[b] = 1;
           any_rebase = true;
@@ -1635,6 +1639,7 @@ void iterate_batch(Problem& pb, const Config& cf) {
         s.best = r2;
         s.since_best = 0;
         s.pend = s.skipped = 0;
+        if (s.low <= PULAY_BELOW) s.period = 1;  // no more plain steps (kernels.hpp)
       }
       const int nh = (int)s.order.size();
       s.picard = !extrap || nh == 1;
@@ -1952,6 +1957,7 @@ void continuation(Problem& pb, const Config& cf, int target) {
       s.since_best = 0;
     }
     Config c = cf;
+    c.every = 1;  // its first iteration may have overflowed by a plain step
     if (!last) {
       c.tol = std::max(cf.tol, 1e-2);
       c.mixed_tol = std::max(cf.mixed_tol, 1e-2);
