@@ -88,9 +88,10 @@ constexpr int NOUT = 2 + MAX_ROWS * MAX_DIIS;
 // iteration that overflowed are walked with MDIIS each pass.  Passes of those
 // random solves against MDIIS each pass: 0.84 times (FP64) and 0.98 times
 // (mixed) at depth 5, 0.95 and 0.99 at 8, 1.03 at 16; two of three passes read
-// no history.  Not for the 3D solvent: 82 passes and 122.
-// its gradients open by up to 2e-9: 604 and 190 passes, but other gradients
-// within that, while with an extrapolation at every pass they repeat to 1e-10.
+// no history.  Not for the 3D solvent: 82 passes and 122.  Not for the adjoint
+// either, whose stopping test leaves its gradients open by up to 2e-9: 604 passes
+// and 190, but other gradients within that, while with an extrapolation at every
+// pass they repeat to 1e-10.
 constexpr int PULAY_PERIOD = 3;
 constexpr int PULAY_DEPTH = 5;
 constexpr double PULAY_BELOW = 0.3;
