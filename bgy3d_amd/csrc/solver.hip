@@ -509,6 +509,7 @@ struct Problem {
   } knob[2] = {{env_int("RISM3D_PLANES", 1), env_int("RISM3D_ZSTAR_ORDER", 3), 0, 0},
                {env_int("RISM3D_PLANES", 1), env_int("RISM3D_ZSTAR_ORDER", 3),
                 env_int("RISM3D_ZSTAR_WIDE", 0), env_int("RISM3D_NYQ", 1)}};
+  int trial = 0;    // passes one after the other whose results nobody takes (tune)
   int noalloc = 0;  // buffers from the fixed scratch: no pinned staging, no graphs
 };
 
@@ -622,7 +623,9 @@ void evaluate(Problem& pb, bool fp32, std::vector<SoluteDesc>& sd, int step = 0,
   g.zwide = kn.zwide;
   g.nyq = kn.nyq;
   SoluteDesc* dsd = step ? pb.d_sd32.p : pb.d_sd.p;
-  const bool pinned = !step && !pb.noalloc;  // this pass's host traffic through pb.io
+  // this pass's host traffic through pb.io, which waits for a pass whose results
+  // were not taken; the tuner's trials go without it, back to back
+  const bool pinned = !step && !pb.noalloc && !pb.trial;
   Profile& pf = g_prof;
   std::vector<SoluteDesc> sdp;  // profiling, step 2: the descriptors on the device
   if (pinned) {
@@ -872,10 +875,12 @@ void tune(Problem& pb, bool fp32, int verbose) {
     bool prof;
     explicit Pause(Problem& p) : pb(p), graphs(p.use_graphs), prof(g_prof.on) {
       pb.use_graphs = 0;
+      pb.trial = 1;
       g_prof.on = false;
     }
     ~Pause() {
       pb.use_graphs = graphs;
+      pb.trial = 0;
       g_prof.on = prof;
     }
   } pause(pb);
@@ -886,7 +891,9 @@ void tune(Problem& pb, bool fp32, int verbose) {
   double best_ms = INFINITY;
   for (const auto& c : cand) {
     pb.knob[fp32 ? 1 : 0] = c;
-    evaluate(pb, fp32, sd);  // untimed: first launch of these kernels
+    // untimed: first launch of these kernels, and of the first candidate as
+    // many as the descriptors' ring has slots (first use of each)
+    for (int r = 0; r < (&c == &cand[0] ? PinnedRing::SLOTS : 1); ++r) evaluate(pb, fp32, sd);
     HIPCHK(hipEventRecord(e0, pb.s));
     for (int r = 0; r < 5; ++r) evaluate(pb, fp32, sd);
     HIPCHK(hipEventRecord(e1, pb.s));
