@@ -831,7 +831,10 @@ void tune(Problem& pb, bool fp32, int verbose) {
     T.loaded = true;
     auto it = T.best.find(key);
     if (it != T.best.end()) {
-      pb.knob[fp32 ? 1 : 0] = it->second.first;
+      Problem::Knobs c = it->second.first;
+      // FP64 has no choice of planes (below); files from before it had any hold 0
+      if (!fp32) c.planes = pb.knob[0].planes;
+      pb.knob[fp32 ? 1 : 0] = c;
       return;
     }
   }

@@ -42,3 +42,38 @@ def test_trials_run_back_to_back(chi_w, tmp_path, monkeypatch):
         print(f"  32x32x{n2}: trial {1e3 * trial:.1f} us, pass {1e6 * per_pass:.1f} us", flush=True)
         ratio.append(1e-3 * trial / per_pass)
     assert sorted(ratio)[1] <= 1.1
+
+
+CHILD = """
+import json, os
+import numpy as np
+from bgy3d_amd import rism3d as R
+from bgy3d_amd import synthetic as S
+s = json.loads(os.environ["CASE"])
+chi = np.load(os.environ["CHI"])
+R.profile_start()
+out = R.hnc3d_run_solute(S.solute(2, n=4, net=0), "%s", s, chi=chi)
+print(json.dumps({"kernels": sorted(R.profile_read()), "mu": out["free-energy"]}))
+""" % W
+
+
+def test_file_without_fp64_planes(chi_w, tmp_path):
+    """A file written when FP64 had no xy planes has 0 for them: the solve stays
+    on planes.  In a process of its own, as a file is read at the first tuning."""
+    print("case tuner file", flush=True)
+    import json
+    import os
+    import subprocess
+    import sys
+    np.save(tmp_path / "chi.npy", chi_w)
+    f = tmp_path / "tune.txt"
+    f.write_text("32x32x32,m3,B1,fp64 0 2 0 0 0.0350\n")
+    s = _settings(32, tune=1, **{"max-iter": 3})
+    env = dict(os.environ, CASE=json.dumps(s), CHI=str(tmp_path / "chi.npy"),
+               RISM3D_TUNE_FILE=str(f))
+    p = subprocess.run([sys.executable, "-c", CHILD], env=env, capture_output=True, text=True,
+                       timeout=100)
+    assert p.returncode == 0, p.stderr
+    got = json.loads(p.stdout.strip().split("\n")[-1])
+    assert "closure_r2c_xy<double>" in got["kernels"], got
+    assert f.read_text().count("fp64") == 1  # the entry was used, nothing timed
