@@ -544,9 +544,10 @@ void download_out(Problem& pb, std::vector<double>& out) {
     return true;
   };
   long spin = 0;
-  bool ended = false;
+  bool ended = false, any = false;
   for (int b = 0; b < pb.B; ++b)
-    for (int q : io.q[b])
+    for (int q : io.q[b]) {
+      any = true;
       while (!taken((size_t)b * NOUT + q)) {
         // the stream is asked only now and then (a failed pass ends the wait
         // within milliseconds): its lock is shared with the launches of other
@@ -563,7 +564,10 @@ void download_out(Problem& pb, std::vector<double>& out) {
         HIPCHK(hipStreamSynchronize(pb.s));
         ended = true;  // everything it wrote arrives by the next look
       }
-  io.open = false;
+    }
+  // a result tells that load_sd has read io.sd; a pass of inactive solutes
+  // leaves none, and the next one waits for it
+  if (any) io.open = false;
 }
 
 // Per-kernel HIP-event timing of the residual chain (rism3d_profile_*).
