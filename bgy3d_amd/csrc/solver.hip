@@ -2950,8 +2950,16 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
       }
     }
     // their pointers up in one copy, the sums of the chunks down in another
+    const int cp = (int)std::min<int64_t>(2048, (g.P + NT - 1) / NT);
     Pinned up(3 * B * sizeof(void*));
     DevBuf<void*> d_up(3 * B);
+    DevBuf<double> d_mu((size_t)B * cp * 5);
+    Pinned mu_host(d_mu.n * 8);
+    const double* mu = mu_host.as<double>();
+    struct Idle {  // before these buffers go back, also after a failed call
+      hipStream_t s;
+      ~Idle() { (void)hipStreamSynchronize(s); }
+    } idle{pb.s};
     for (int b = 0; b < B; ++b) {
       up.as<const void*>()[b] = tt[b];
       up.as<const void*>()[B + b] = gg[b];
@@ -2959,14 +2967,10 @@ int run_impl(const Inputs& in, rism3d_result* res, std::vector<double>* t_init,
     }
     HIPCHK(hipMemcpyAsync(d_up.p, up.as<void>(), 3 * B * sizeof(void*), hipMemcpyHostToDevice, pb.s));
     double* const* d_up64 = reinterpret_cast<double* const*>(d_up.p);
-    const int cp = (int)std::min<int64_t>(2048, (g.P + NT - 1) / NT);
-    DevBuf<double> d_mu((size_t)B * cp * 5);
     hipLaunchKernelGGL(mu_density, dim3(cp, B), dim3(NT), 0, pb.s, pb.d_sites, g,
                        (const double* const*)d_up64, (const double* const*)(d_up64 + 2 * B),
                        pd.L[0], pd.L[1], pd.L[2], pb.h[0], pb.h[1], pb.h[2],
                        want_g ? d_up64 + B : (double* const*)nullptr, d_mu.p);
-    Pinned mu_host(d_mu.n * 8);
-    const double* mu = mu_host.as<double>();
     HIPCHK(hipMemcpyAsync(mu_host.as<void>(), d_mu.p, d_mu.n * 8, hipMemcpyDeviceToHost, pb.s));
     HIPCHK(hipStreamSynchronize(pb.s));
     HIPCHK(hipGetLastError());
