@@ -27,8 +27,8 @@ __host__ __device__ constexpr int rows_for(int M) {
   return M <= 16 ? 64 : M <= 32 ? 32 : M <= 64 ? 16 : M <= 128 ? 8 : 4;
 }
 
-// Twiddles: every chain kernel copies its tables to LDS (stw) beside its first
-// loads.  Read from global memory inside the stages they shared the vector
+// Twiddles: every chain kernel but zstar (which reads them from memory) copies
+// its tables to LDS (stw) beside its first loads.  Read from global memory inside the stages they shared the vector
 // cache and its wait counter with the streams, and each stage waited on both (us per
 // launch, from global memory and from LDS: closure and residual of 24 x 128^3
 // in FP32 719 and 667, 597 and 547, its z pass 281 and 241; 192^3 with 5 sites
@@ -749,7 +749,7 @@ __device__ __forceinline__ void oz_point(cpx<double> (&c)[MS * (MS + 1) / 2],
 // points of all MS sites in registers for the contraction.  LDS per
 // workgroup is 1/MS of zstar's, so a 128-byte row of kx columns (16 FP32
 // or 8 FP64) fits at high occupancy.  Same arithmetic as zstar, point by
-// point.  Grid as zstar.
+// point.  1D grid: the Nyquist blocks of every solute, then the tiles (below).
 // OZ > 0 (FP64, special 1): the solvent-solvent step of OZ sites instead,
 // MS = OZ (OZ + 1) / 2 pairs (oz_point).  zstar's oz_pairs keeps its matrices
 // in scratch (their loops run to a run-time site count) and took 60% of a

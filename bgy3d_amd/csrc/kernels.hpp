@@ -194,7 +194,7 @@ struct GridArgs {
   int zB, ztiles;      // z pass: solutes and kx tiles of the launch
   int nyq;             // FP32 z pass: the Nyquist column in blocks of its own
   int zwide;           // FP32 z pass at N2 <= 128: 32 kx columns, 512 threads
-  // ylay (the FP32 xy-plane chain): W is y-major, point (site, ky, z, kx <
+  // ylay (the xy-plane chain): W is y-major, point (site, ky, z, kx <
   // N0/2) at site K + ky N2 NH + z NH + kx, so that the z pass reads whole
   // regions of the spectrum, and the Nyquist column kx = N0/2 is compact
   // behind the sites, (site, z, ky) at m K + site N1 N2 + z N1 + ky (cpx<T>

@@ -84,9 +84,10 @@ enum rism3d_status {
    bgy3d-snes.c:16-35) plus MDIIS.  Every solver stops at max|F| <=
    norm_tol.  NEWTON, JAGER and TRIAL run in FP64 only. */
 enum rism3d_solver {
-  RISM3D_SOLVER_MDIIS = 0,  /* default: MDIIS / Anderson mixing, near the
-                               root at every third step, plain steps
-                               between (periodic Pulay)                  */
+  RISM3D_SOLVER_MDIIS = 0,  /* default: MDIIS / Anderson mixing, once max|F|
+                               is below 0.3 at every third step, plain
+                               steps between (periodic Pulay), until a
+                               restart                                   */
   RISM3D_SOLVER_PICARD = 1, /* x += lambda F(x) (bgy3d-snes.c:348-384)  */
   RISM3D_SOLVER_NEWTON = 2, /* Newton, GMRES(30) on the matrix-free
                                Jacobian, backtracking line search
@@ -104,8 +105,8 @@ enum rism3d_precision {
                                every rebase, then polish_iters FP64 steps;
                                no FP32 floor.  The FP32 MDIIS history is
                                kept as the newest u in FP32, BF16
-                               differences of u and BF16 residuals (FP8
-                               where every pass extrapolates: depth < 5);
+                               differences of u and FP8 residuals, which
+                               go to BF16 when periodic mixing begins;
                                solutes ready for a rebase wait for one
                                another (grouped FP64 passes)             */
   RISM3D_FP32 = 2           /* FP32 passes only, around the starting
